@@ -282,7 +282,7 @@ def main():
         "config": {"workload": "config 2 scene (1,040,384 tris) at 1920x1080, R_inc incoherent bounce rays, "
                                "closest hit", "rays_per_step": n, "bvh": bvh_name,
                    "block": args.block or 128,
-                   "lds_stack": args.stack or 16},
+                   "lds_stack": args.stack or 8},
         "roofline": {"bound": "hbm", "achieved": round(achieved_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved_gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "achieved_kind": "algorithmic bytes (B_ray x rays) / mean launch time: an effective bandwidth",

@@ -351,6 +351,7 @@ void finalize_bvh(Ctx& ctx, int32_t ninner)
     bvh.max_depth = maxd;
     bvh.max_leaf_size = maxleaf;
     bvh.sah_cost = root_area > 0 ? sah / root_area : 0.0;
+    build_wide(ctx);
     bvh.valid = true;
 }
 

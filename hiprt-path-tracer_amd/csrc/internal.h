@@ -55,7 +55,7 @@ struct DeviceBuffer {
 
 struct TraceConfig {
     int block_size = 128;
-    int lds_stack = 16;
+    int lds_stack = 8; // entries of 8 bytes a lane; 6 waves per SIMD fit (16: 5, 587 us for 549 us at 8)
     int queue_tile = 1; // rays a wave takes per work-counter atomic, in units of 64
 };
 
@@ -94,6 +94,11 @@ struct Bvh {
     double sah_cost = 0.0;
     DeviceBuffer nodes;           // BvhNode[node_count]
     DeviceBuffer tris;            // TriRecord[triangle_count] in leaf order
+    // the 6-wide tree the traversal walks, made from the binary one
+    int32_t wide_count = 0;       // nodes, root = node 0
+    int32_t wide_stack = 0;       // entries a traversal's stack can hold at most
+    DeviceBuffer wide;            // WideNode[wide_count]
+    DeviceBuffer wide_tris;       // TriRecord[triangle_count] in the wide leaves' order
 };
 
 // Per-resolution render buffers and settings of the path-tracing passes.
@@ -283,6 +288,9 @@ void restir_spatiotemporal_pass(Ctx& ctx, uint32_t sample_number, uint32_t rando
 // bvh_build.hip
 void build_lbvh(Ctx& ctx);
 void build_sah_binned(Ctx& ctx);
+
+// bvh_wide.hip: the 6-wide tree from the finished binary one.
+void build_wide(Ctx& ctx);
 
 // trace.hip
 void trace_closest(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint32_t* counts, uint32_t n,

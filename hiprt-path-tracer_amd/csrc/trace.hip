@@ -4,25 +4,30 @@
 // trace_main_path_ray, evaluate_shadow_ray_occluded and
 // evaluate_bsdf_light_sample_ray (src/Device/includes/Intersect.h:200-324,
 // :544-643). CDNA4 has no ray-tracing units, so this is a plain stackful
-// traversal:
-//   * one 64-byte BvhNode fetch per step tests both child boxes;
-//   * leaf children are intersected immediately (Moller-Trumbore, exact
-//     reference arithmetic), interior children are visited near-first and the
-//     far one pushed;
-//   * the per-lane stack lives in LDS, laid out [depth][lane] so the 64 lanes
-//     of a wave touch 64 consecutive dwords (no bank conflicts); entries
+// traversal of a 6-wide tree (layout.h: WideNode), one ray per lane:
+//   * one 64-byte node fetch tests the quantised boxes of up to six children;
+//     those hit are sorted by entry distance, the nearest is taken and the
+//     others are pushed with their distances, so that an entry behind the
+//     closest hit found since is dropped without a fetch;
+//   * a leaf is a reference to its first triangle (Moller-Trumbore, exact
+//     reference arithmetic), taken from the stack like a node. Lanes at leaves
+//     wait until LEAF_LANES of them are there (or no lane is at a node): the
+//     wave then pays for the triangle test once for many;
+//   * the per-lane stack lives in LDS, laid out [depth][lane]; entries
 //     deeper than the LDS stack spill to a per-thread global array;
-//   * a persistent grid sized from occupancy; each wave pulls batches of 64
-//     rays from a global counter so that long rays do not stall a whole block;
-//   * optionally the rays to trace come from a segmented queue of slot
-//     indices (seglist.h) whose length is read on the device (the path passes
-//     enqueue only live rays); results go to the rays' own slots.
+//   * a persistent grid sized from occupancy; each wave takes batches of rays
+//     from a global counter and hands them to lanes whose ray is done, once
+//     REFILL_LANES of them are;
+//   * optionally the rays to trace come from segmented queues of slot
+//     indices (seglist.h) whose lengths are read on the device (the path
+//     passes enqueue only live rays); results go to the rays' own slots.
 //
-// Results are exact: the box test is widened (boxes padded at build time and
-// the slab interval relatively widened by 2^-16) so it never rejects a node
-// holding the closest Moller-Trumbore hit, and ties in t go to the smaller
-// primitive index. Hit IDs and t are therefore bit-identical to a brute-force
-// loop over all triangles with the same arithmetic.
+// Results are exact: the box test is conservative (boxes padded at build time,
+// quantised outwards, and the slab interval relatively widened by 2^-16), so
+// it never rejects a node holding the closest Moller-Trumbore hit, and ties in
+// t go to the smaller primitive index. Hit IDs and t are therefore
+// bit-identical to a brute-force loop over all triangles with the same
+// arithmetic.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -38,7 +43,7 @@
 namespace mipt {
 namespace {
 
-enum Mode { CLOSEST = 0, ANY = 1, CLOSEST_COUNTED = 2 };
+enum Mode { CLOSEST = 0, ANY = 1, CLOSEST_COUNTED = 2, QUEUED = 3 };
 
 constexpr float WIDEN_LO = 1.0f - 1.52587890625e-05f; // 1 - 2^-16
 constexpr float WIDEN_HI = 1.0f + 1.52587890625e-05f;
@@ -49,230 +54,26 @@ __device__ __forceinline__ float safe_inv(float d)
     return 1.0f / (fabsf(d) > tiny ? d : copysignf(tiny, d));
 }
 
-// Slab test of one box; returns the widened entry distance or +inf on a miss.
-__device__ __forceinline__ float box_enter(float lox, float loy, float loz, float hix, float hiy, float hiz,
-                                           pt::f3 inv, pt::f3 oinv, float tfar_limit)
-{
-    float tx0 = __builtin_fmaf(lox, inv.x, -oinv.x), tx1 = __builtin_fmaf(hix, inv.x, -oinv.x);
-    float ty0 = __builtin_fmaf(loy, inv.y, -oinv.y), ty1 = __builtin_fmaf(hiy, inv.y, -oinv.y);
-    float tz0 = __builtin_fmaf(loz, inv.z, -oinv.z), tz1 = __builtin_fmaf(hiz, inv.z, -oinv.z);
-    float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.0f));
-    float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), tfar_limit));
-    return (tn * WIDEN_LO <= tf * WIDEN_HI) ? tn : INFINITY;
-}
-
 __global__ void k_reset_counter(uint32_t* c) { c[0] = 0u; }
 
-// Result of one ray's traversal.
-struct RayHit {
-    int32_t prim;
-    float t, u, v;
-    uint32_t nodes, tris;
-};
+// Lanes at a leaf that make the wave test triangles (1 to 24 measured within
+// 2 % of each other, 32 lost 20 %: lanes that wait test no boxes), and lanes
+// without a ray that make it take more (8 to 24: the same).
+constexpr int LEAF_LANES = 8;
+constexpr int REFILL_LANES = 16;
+// Fewer rays than the grid has lanes are dealt to 2 waves per SIMD, at least
+// MIN_BATCH to a wave: a wave of few rays takes fewer different branches and
+// ends sooner, but more waves than that wait for each other's instructions
+// (120,000 bounce rays of the 1M-triangle scene: 195 us at 64 rays a wave,
+// 160 us at 24, 140 to 146 us dealt so).
+constexpr uint32_t MIN_BATCH = 8;
+constexpr uint32_t FEW_WAVES_PER_CU = 8;
 
-// Traverses one ray (the 32-byte record ra, rb) from the root. `any` stops at
-// the first accepted hit (any-hit rays are shadow rays: maxT is the light
-// distance). The LDS stack is [depth][thread] over the block; entries past
-// STACK go to the thread's spill column.
-template <int BLOCK, int STACK, bool COUNT>
-__device__ __forceinline__ RayHit traverse(const BvhNode* __restrict__ nodes, const TriRecord* __restrict__ tris,
-                                           int32_t root, float4 ra, float4 rb, bool any, int32_t* stack,
-                                           int32_t* __restrict__ spill, uint32_t spill_stride, uint32_t gtid,
-                                           uint32_t max_steps)
-{
-    const pt::f3 o = pt::mk(ra.x, ra.y, ra.z);
-    const pt::f3 d = pt::mk(rb.x, rb.y, rb.z);
-    const int32_t last_prim = __float_as_int(ra.w);
-    const pt::f3 inv = pt::mk(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z));
-    const pt::f3 oinv = pt::mk(o.x * inv.x, o.y * inv.y, o.z * inv.z);
+constexpr int32_t IDLE = 0x7fffffff; // no node or leaf to visit (node indices stay below)
 
-    float best_t = rb.w;
-    int32_t best_prim = -1;
-    float best_u = 0.0f, best_v = 0.0f;
-    uint32_t n_nodes = 0, n_tris = 0;
-    bool done = false;
-
-    int32_t node = root;
-    int sp = 0;
-    // A tree traversal visits each interior node at most once; the cap
-    // only guards against a malformed node array.
-    for (uint32_t step = 0; !done && step < max_steps; step++)
-    {
-        const BvhNode* np = nodes + node;
-        const float4 a = np->a, b = np->b, c = np->c;
-        const int4 refs = np->d;
-        if (COUNT)
-            n_nodes++;
-        const float t0 = box_enter(a.x, a.y, a.z, a.w, b.x, b.y, inv, oinv, best_t);
-        const float t1 = box_enter(b.z, b.w, c.x, c.y, c.z, c.w, inv, oinv, best_t);
-        const int32_t ch[2] = {refs.x, refs.y};
-        const float tc[2] = {t0, t1};
-
-        // Leaf children first.
-        for (int s = 0; s < 2 && !done; s++)
-        {
-            if (ch[s] >= 0 || tc[s] == INFINITY)
-                continue;
-            const int32_t first = leaf_first(ch[s]);
-            const int32_t cnt = leaf_count(ch[s]);
-            for (int32_t k = 0; k < cnt; k++)
-            {
-                const TriRecord* tr = tris + first + k;
-                const float4 v0 = tr->v0, e1 = tr->e1, e2 = tr->e2;
-                const int32_t prim = __float_as_int(v0.w);
-                if (COUNT)
-                    n_tris++;
-                float t, u, v;
-                if (!pt::mt_intersect(pt::mk(v0.x, v0.y, v0.z), pt::mk(e1.x, e1.y, e1.z), pt::mk(e2.x, e2.y, e2.z),
-                                      o, d, t, u, v))
-                    continue;
-                if (prim == last_prim)
-                    continue;
-                if (t < best_t || (t == best_t && prim < best_prim))
-                {
-                    best_t = t;
-                    best_prim = prim;
-                    best_u = u;
-                    best_v = v;
-                    if (any)
-                    {
-                        done = true;
-                        break;
-                    }
-                }
-            }
-        }
-        if (done)
-            break;
-
-        // Interior children: near first, far pushed.
-        const bool h0 = ch[0] >= 0 && t0 != INFINITY;
-        const bool h1 = ch[1] >= 0 && t1 != INFINITY;
-        int32_t next = -1;
-        if (h0 && h1)
-        {
-            const bool first0 = t0 <= t1;
-            next = first0 ? ch[0] : ch[1];
-            const int32_t far = first0 ? ch[1] : ch[0];
-            if (sp < STACK)
-                stack[sp * BLOCK + threadIdx.x] = far;
-            else
-                spill[(size_t)(sp - STACK) * spill_stride + gtid] = far;
-            sp++;
-        }
-        else if (h0)
-            next = ch[0];
-        else if (h1)
-            next = ch[1];
-
-        if (next < 0)
-        {
-            if (sp == 0)
-                break;
-            sp--;
-            next = sp < STACK ? stack[sp * BLOCK + threadIdx.x] : spill[(size_t)(sp - STACK) * spill_stride + gtid];
-        }
-        node = next;
-    }
-    return RayHit{best_prim, best_t, best_u, best_v, n_nodes, n_tris};
-}
-
-__device__ __forceinline__ int4 hit_record(const RayHit& h)
-{
-    return h.prim >= 0 ? make_int4(h.prim, __float_as_int(h.t), __float_as_int(h.u), __float_as_int(h.v))
-                       : make_int4(-1, __float_as_int(-1.0f), 0, 0);
-}
-
-// Next tile of a wave: `tile` consecutive batches of 64 rays (the queue
-// tile). Each wave's first tile is its own by index; later tiles come from
-// the work counter, past the statically assigned ones. A launch on fewer
-// rays than the grid's lanes then touches the counter only from the waves
-// that had work: a same-address atomic from every wave costs tens of
-// microseconds per launch. Larger tiles take fewer atomics and balance
-// the waves' uneven ray lengths less finely.
-struct BatchCursor {
-    uint32_t next;
-    bool first;
-
-    __device__ __forceinline__ void init(int block, uint32_t tile)
-    {
-        next = (blockIdx.x * ((uint32_t)block / 64u) + threadIdx.x / 64u) * 64u * tile;
-        first = true;
-    }
-
-    __device__ __forceinline__ uint32_t take(uint32_t* work_counter, int block, uint32_t tile)
-    {
-        uint32_t base = next;
-        if (!first)
-        {
-            const uint32_t waves = gridDim.x * ((uint32_t)block / 64u);
-            if ((threadIdx.x & 63u) == 0)
-                base = atomicAdd(work_counter, 64u * tile) + waves * 64u * tile;
-            base = __shfl(base, 0, 64);
-        }
-        first = false;
-        return base;
-    }
-};
-
-template <int BLOCK, int STACK, int MODE>
-__global__ __launch_bounds__(BLOCK) void k_trace(const BvhNode* __restrict__ nodes, const TriRecord* __restrict__ tris,
-                                                 int32_t root, const float4* __restrict__ rays, int4* __restrict__ hits,
-                                                 uint8_t* __restrict__ occluded, uint2* __restrict__ counts, uint32_t n,
-                                                 int32_t* __restrict__ spill, uint32_t spill_stride,
-                                                 uint32_t* __restrict__ work_counter, uint32_t max_steps,
-                                                 const uint32_t* __restrict__ queue,
-                                                 const uint32_t* __restrict__ queue_counts, uint32_t queue_seg_cap,
-                                                 uint32_t tile)
-{
-    __shared__ int32_t stack[STACK * BLOCK];
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t gtid = blockIdx.x * BLOCK + threadIdx.x;
-    SegMap map{};
-    if (queue)
-    {
-        map.init(queue_counts, queue_seg_cap);
-        n = min(n, map.total);
-    }
-    BatchCursor cur;
-    cur.init(BLOCK, tile);
-    for (;;)
-    {
-        const uint32_t first = cur.take(work_counter, BLOCK, tile);
-        if (first >= n)
-            break;
-        for (uint32_t k = 0; k < tile; k++)
-        {
-            const uint32_t base = first + 64u * k;
-            if (base >= n)
-                break;
-            const uint32_t w = base + lane;
-            uint32_t r = w;
-            if (queue)
-                r = queue[map.slot(w < n ? w : n - 1u)]; // every lane takes part in the search
-            if (w >= n)
-                continue;
-            const RayHit h = traverse<BLOCK, STACK, MODE == CLOSEST_COUNTED>(
-                nodes, tris, root, rays[2 * (size_t)r], rays[2 * (size_t)r + 1], MODE == ANY, stack, spill,
-                spill_stride, gtid, max_steps);
-            if (MODE == ANY)
-                occluded[r] = h.prim >= 0 ? 1 : 0;
-            else
-            {
-                hits[r] = hit_record(h);
-                if (MODE == CLOSEST_COUNTED)
-                    counts[r] = make_uint2(h.nodes, h.tris);
-            }
-        }
-    }
-}
-
-// The rays of up to three segmented queues in one launch: dense index w runs
-// over queue 0, then 1, then 2, each range rounded up to whole waves so that
-// a wave traces one queue; a queue with `occluded` set is traced any-hit, the
-// others closest-hit. One launch instead of three keeps the grid busy when
-// the queues are short (a launch costs about the traversal latency of its
-// longest ray, whatever its length).
+// A ray set: `rays` indexed by slot; with `occluded` it is traced any-hit
+// (shadow rays: tmax is the light distance), else closest-hit into `hits`.
+// Slots come from a segmented queue, or are 0 .. n-1 without one.
 struct QueueJob {
     const float4* rays;
     int4* hits;
@@ -282,96 +83,359 @@ struct QueueJob {
     uint32_t seg_cap;
 };
 
-struct QueueJobs {
+struct TraceArgs {
+    const WideNode* nodes;
+    const TriRecord* tris;
     QueueJob job[3];
+    uint2* counts;      // nodes and triangles per ray (instrumented variant)
+    uint32_t n;         // rays without a queue
+    uint2* spill;       // stack entries past the LDS ones, a column per thread
+    uint32_t spill_stride;
+    uint32_t* work_counter;
+    uint32_t tile;
+    uint32_t few_waves; // waves that fewer rays than the grid's lanes are dealt to
 };
 
-template <int BLOCK, int STACK>
-__global__ __launch_bounds__(BLOCK) void k_trace_queues(const BvhNode* __restrict__ nodes,
-                                                        const TriRecord* __restrict__ tris, int32_t root, QueueJobs q,
-                                                        int32_t* __restrict__ spill, uint32_t spill_stride,
-                                                        uint32_t* __restrict__ work_counter, uint32_t max_steps,
-                                                        uint32_t tile)
+__device__ __forceinline__ uint32_t med3(uint32_t a, uint32_t b, uint32_t c) { return max(min(a, b), min(max(a, b), c)); }
+
+// Sorts six keys: two triples by three-operand minimum, median and maximum
+// (one instruction each), then a merge: 18 instructions against 24 of a
+// network of two-operand comparators.
+__device__ __forceinline__ void sort6(uint32_t k[6])
 {
-    __shared__ int32_t stack[STACK * BLOCK];
+    const uint32_t a0 = min(min(k[0], k[1]), k[2]), a1 = med3(k[0], k[1], k[2]), a2 = max(max(k[0], k[1]), k[2]);
+    const uint32_t b0 = min(min(k[3], k[4]), k[5]), b1 = med3(k[3], k[4], k[5]), b2 = max(max(k[3], k[4]), k[5]);
+    const uint32_t x = max(a0, b0), y = min(a2, b2), p = min(a1, b1), q = max(a1, b1);
+    const uint32_t m = max(x, p), n = min(q, y);
+    k[0] = min(a0, b0);
+    k[1] = min(x, p);
+    k[2] = min(m, n);
+    k[3] = max(m, n);
+    k[4] = max(q, y);
+    k[5] = max(a2, b2);
+}
+
+template <int I> __device__ __forceinline__ float byte_of(uint32_t w) { return (float)((w >> (8 * I)) & 0xffu); }
+
+// One ray set, or (QUEUED) the rays of up to three segmented queues: dense
+// index w runs over queue 0, then 1, then 2. One launch instead of three keeps
+// the grid busy when the queues are short (a launch costs about the traversal
+// latency of its longest ray, whatever its length).
+//
+// Bound by instruction issue: the vector units are busy 83 % of the time over
+// 2,073,600 incoherent rays on 1,040,384 triangles (17 nodes and 4.6 triangles
+// a ray, 45 of 64 lanes at a node in a mean node step, about 210 instructions;
+// the 64-byte record costs 4 loads, the L2 serves 2.4 GB). A binary tree of
+// 64-byte nodes with float boxes took 43.8 nodes a ray, and the same 4
+// loads for each: 910 us, now 514 us; 700,001 shadow rays 564 us, now 300 us.
+// Reading the nodes by groups of four lanes through LDS (a quarter of the cache
+// accesses) cost more in instructions and LDS than it saved (680 us), a second
+// put-aside leaf per lane let culling lag (552 us).
+template <int BLOCK, int STACK, int MODE>
+__global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
+{
+    constexpr bool QUEUES = MODE == QUEUED;
+    __shared__ uint2 stack[STACK * BLOCK];
     // Segment starts of the three queues (the same for every wave): read
     // from LDS by a per-lane binary search, so no registers hold them while
     // the rays are traversed.
-    __shared__ uint32_t seg_start[3][SEG_COUNT];
+    __shared__ uint32_t seg_start[QUEUES ? 3 : 1][SEG_COUNT];
     __shared__ uint32_t queue_end[3];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t gtid = blockIdx.x * BLOCK + threadIdx.x;
-    if (threadIdx.x < 64u)
+    uint32_t total = a.n, end0 = 0u, end1 = 0u;
+    if (QUEUES)
     {
-        uint32_t total = 0;
-#pragma unroll
-        for (int k = 0; k < 3; k++)
+        if (threadIdx.x < 64u)
         {
-            SegMap m{};
-            m.excl = 0u;
-            m.total = 0u;
-            if (q.job[k].slots)
-                m.init(q.job[k].counts, q.job[k].seg_cap);
-            seg_start[k][lane] = m.excl;
-            total += m.total;
-            if (lane == 0)
-                queue_end[k] = total;
+            uint32_t sum = 0;
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+            {
+                SegMap m{};
+                m.excl = 0u;
+                m.total = 0u;
+                if (a.job[k].slots)
+                    m.init(a.job[k].counts, a.job[k].seg_cap);
+                seg_start[QUEUES ? k : 0][lane] = m.excl;
+                sum += m.total;
+                if (lane == 0)
+                    queue_end[k] = sum;
+            }
         }
+        __syncthreads();
+        end0 = __builtin_amdgcn_readfirstlane(queue_end[0]);
+        end1 = __builtin_amdgcn_readfirstlane(queue_end[1]);
+        total = __builtin_amdgcn_readfirstlane(queue_end[2]);
     }
-    __syncthreads();
-    // each queue's range starts on a whole wave
-    const uint32_t n0 = queue_end[0], n1 = queue_end[1] - n0, n2 = queue_end[2] - queue_end[1];
-    const uint32_t start1 = (n0 + 63u) & ~63u;
-    const uint32_t start2 = start1 + ((n1 + 63u) & ~63u);
-    const uint32_t total = start2 + n2;
-    BatchCursor cur;
-    cur.init(BLOCK, tile);
+
+    // The wave's rays: its first batch by index, later ones from the work
+    // counter, past the statically assigned ones (a same-address atomic from
+    // every wave costs tens of microseconds per launch). With fewer rays than
+    // lanes the batches shrink, down to MIN_BATCH rays: more waves, each with
+    // fewer different paths through the tree, end sooner.
+    const uint32_t waves = gridDim.x * (BLOCK / 64u);
+    uint32_t batch = 64u * a.tile;
+    if (total < waves * 64u)
+        batch = min(64u, max(MIN_BATCH, (total + a.few_waves - 1u) / a.few_waves));
+    uint32_t next = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64u) + threadIdx.x / 64u) * batch;
+    uint32_t batch_end = min(next + batch, total);
+    bool more = next < total;
+
+    // the lane's ray
+    pt::f3 o{}, d{};
+    float inv_nx = 0.0f, inv_ny = 0.0f, inv_nz = 0.0f, inv_fx = 0.0f, inv_fy = 0.0f, inv_fz = 0.0f;
+    float best_t = 0.0f, best_u = 0.0f, best_v = 0.0f;
+    int32_t best_prim = -1, last_prim = -1;
+    uint32_t slot = 0u, job = 0u;
+    uint32_t n_nodes = 0, n_tris = 0;
+    bool any = MODE == ANY, has_ray = false;
+    int32_t cur = IDLE;  // node or leaf to visit next
+    int32_t leaf = 0;    // leaf whose triangles wait to be tested, 0 for none
+    int sp = 0;
+
     for (;;)
     {
-        const uint32_t first = cur.take(work_counter, BLOCK, tile);
-        if (first >= total)
-            break;
-        for (uint32_t kt = 0; kt < tile; kt++)
+        const uint64_t idle = __ballot(cur == IDLE && leaf == 0 && sp == 0);
+        if (idle == ~0ull || (more && __popcll(idle) >= REFILL_LANES))
         {
-            const uint32_t base = first + 64u * kt;
-            if (base >= total)
-                break;
-            // the wave's queue (uniform over the wave)
-            const int k = base < start1 ? 0 : (base < start2 ? 1 : 2);
-            const uint32_t local = base + lane - (k == 0 ? 0u : (k == 1 ? start1 : start2));
-            const uint32_t count = k == 0 ? n0 : (k == 1 ? n1 : n2);
-            if (local >= count)
-                continue;
-            // fields picked by selects: indexing the argument struct by a
-            // run-time value would copy it to scratch memory
-            const float4* rays = k == 0 ? q.job[0].rays : (k == 1 ? q.job[1].rays : q.job[2].rays);
-            const uint32_t* slots = k == 0 ? q.job[0].slots : (k == 1 ? q.job[1].slots : q.job[2].slots);
-            const uint32_t seg_cap = k == 0 ? q.job[0].seg_cap : (k == 1 ? q.job[1].seg_cap : q.job[2].seg_cap);
-            // last segment whose start is <= local
-            int lo = 0, hi = (int)SEG_COUNT - 1;
-            for (int step = 0; step < 6; step++)
+            const bool free = cur == IDLE && leaf == 0 && sp == 0;
+            if (free && has_ray)
             {
-                const int mid = (lo + hi + 1) >> 1;
-                if (seg_start[k][mid] <= local)
-                    lo = mid;
+                has_ray = false;
+                if (any)
+                {
+                    uint8_t* occ = a.job[0].occluded;
+                    if (QUEUES)
+                        occ = job == 0u ? a.job[0].occluded : (job == 1u ? a.job[1].occluded : a.job[2].occluded);
+                    occ[slot] = best_prim >= 0 ? 1 : 0;
+                }
                 else
-                    hi = mid - 1;
+                {
+                    int4* hits = a.job[0].hits;
+                    if (QUEUES)
+                        hits = job == 0u ? a.job[0].hits : (job == 1u ? a.job[1].hits : a.job[2].hits);
+                    hits[slot] = best_prim >= 0 ? make_int4(best_prim, __float_as_int(best_t), __float_as_int(best_u),
+                                                            __float_as_int(best_v))
+                                                : make_int4(-1, __float_as_int(-1.0f), 0, 0);
+                    if (MODE == CLOSEST_COUNTED)
+                        a.counts[slot] = make_uint2(n_nodes, n_tris);
+                }
             }
-            const uint32_t r = slots[(size_t)lo * seg_cap + (local - seg_start[k][lo])];
-            const float4 ra = rays[2 * (size_t)r], rb = rays[2 * (size_t)r + 1];
-            uint8_t* occluded = k == 0 ? q.job[0].occluded : (k == 1 ? q.job[1].occluded : q.job[2].occluded);
-            if (occluded)
+            if (more && next >= batch_end)
             {
-                const RayHit h = traverse<BLOCK, STACK, false>(nodes, tris, root, ra, rb, true, stack, spill,
-                                                              spill_stride, gtid, max_steps);
-                occluded[r] = h.prim >= 0 ? 1 : 0;
+                // with every ray assigned by index there is nothing to ask for
+                if (waves * batch >= total)
+                    more = false;
+                else
+                {
+                    uint32_t base = 0u;
+                    if (lane == 0u)
+                        base = atomicAdd(a.work_counter, batch);
+                    next = __builtin_amdgcn_readfirstlane(base) + waves * batch;
+                    batch_end = min(next + batch, total);
+                    more = next < total;
+                }
+            }
+            if (more)
+            {
+                const uint32_t left = batch_end - next;
+                const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                if (free && rank < left)
+                {
+                    const uint32_t w = next + rank;
+                    const float4* rays = a.job[0].rays;
+                    slot = w;
+                    if (QUEUES)
+                    {
+                        // fields picked by selects: indexing the argument
+                        // struct by a run-time value would copy it to scratch
+                        job = w < end0 ? 0u : (w < end1 ? 1u : 2u);
+                        const uint32_t local = w - (job == 0u ? 0u : (job == 1u ? end0 : end1));
+                        rays = job == 0u ? a.job[0].rays : (job == 1u ? a.job[1].rays : a.job[2].rays);
+                        const uint32_t* slots =
+                            job == 0u ? a.job[0].slots : (job == 1u ? a.job[1].slots : a.job[2].slots);
+                        const uint32_t seg_cap =
+                            job == 0u ? a.job[0].seg_cap : (job == 1u ? a.job[1].seg_cap : a.job[2].seg_cap);
+                        any = job == 0u ? a.job[0].occluded != nullptr
+                                        : (job == 1u ? a.job[1].occluded != nullptr : a.job[2].occluded != nullptr);
+                        // last segment whose start is <= local
+                        int lo = 0, hi = (int)SEG_COUNT - 1;
+                        for (int step = 0; step < 6; step++)
+                        {
+                            const int mid = (lo + hi + 1) >> 1;
+                            if (seg_start[QUEUES ? job : 0][mid] <= local)
+                                lo = mid;
+                            else
+                                hi = mid - 1;
+                        }
+                        slot = slots[(size_t)lo * seg_cap + (local - seg_start[QUEUES ? job : 0][lo])];
+                    }
+                    const float4 ra = rays[2 * (size_t)slot], rb = rays[2 * (size_t)slot + 1];
+                    o = pt::mk(ra.x, ra.y, ra.z);
+                    d = pt::mk(rb.x, rb.y, rb.z);
+                    last_prim = __float_as_int(ra.w);
+                    best_t = rb.w;
+                    best_prim = -1;
+                    best_u = best_v = 0.0f;
+                    const float ix = safe_inv(d.x), iy = safe_inv(d.y), iz = safe_inv(d.z);
+                    inv_nx = ix * WIDEN_LO;
+                    inv_ny = iy * WIDEN_LO;
+                    inv_nz = iz * WIDEN_LO;
+                    inv_fx = ix * WIDEN_HI;
+                    inv_fy = iy * WIDEN_HI;
+                    inv_fz = iz * WIDEN_HI;
+                    if (MODE == CLOSEST_COUNTED)
+                        n_nodes = n_tris = 0u;
+                    has_ray = true;
+                    sp = 0;
+                    // Nothing is hit at or past tmax, nor by a ray with an
+                    // infinite or NaN component (every triangle test then
+                    // compares a NaN, an infinity or 0).
+                    const bool finite = __builtin_isfinite(o.x) && __builtin_isfinite(o.y) && __builtin_isfinite(o.z) &&
+                                        __builtin_isfinite(d.x) && __builtin_isfinite(d.y) && __builtin_isfinite(d.z);
+                    cur = best_t > 0.0f && finite ? 0 : IDLE;
+                }
+                next += min((uint32_t)__popcll(idle), left);
+            }
+            else if (idle == ~0ull)
+                break;
+        }
+
+        const bool at_node = (uint32_t)cur < (uint32_t)IDLE;
+        if (at_node)
+        {
+            const WideNode* np = a.nodes + cur;
+            const float4 org = np->origin;
+            const uint4 refs = np->refs, qxy = np->qxy, qz = np->qz;
+            if (MODE == CLOSEST_COUNTED)
+                n_nodes++;
+            const uint32_t ex = (uint32_t)__float_as_int(org.w);
+            const float sx = __uint_as_float(ex << 23), sy = __uint_as_float((ex << 14) & 0x7f800000u),
+                        sz = __uint_as_float(ex & 0x7f800000u);
+            const uint32_t count = (ex >> 17) & 7u;
+            const float px = org.x - o.x, py = org.y - o.y, pz = org.z - o.z;
+            const float nbx = px * inv_nx, nby = py * inv_ny, nbz = pz * inv_nz;
+            const float fbx = px * inv_fx, fby = py * inv_fy, fbz = pz * inv_fz;
+            const float nsx = sx * inv_nx, nsy = sy * inv_ny, nsz = sz * inv_nz;
+            const float fsx = sx * inv_fx, fsy = sy * inv_fy, fsz = sz * inv_fz;
+            // entry and exit planes by the sign of the direction
+            const bool bx = inv_nx < 0.0f, by = inv_ny < 0.0f, bz = inv_nz < 0.0f;
+            const uint32_t tx = bx ? __builtin_rotateright32(refs.w, 16) : refs.w;
+            const uint32_t ty = by ? __builtin_rotateright32(qz.z, 16) : qz.z;
+            const uint32_t tz = bz ? __builtin_rotateright32(qz.w, 16) : qz.w;
+            const uint32_t nx = bx ? qxy.y : qxy.x, fx = bx ? qxy.x : qxy.y;
+            const uint32_t ny = by ? qxy.w : qxy.z, fy = by ? qxy.z : qxy.w;
+            const uint32_t nz = bz ? qz.y : qz.x, fz = bz ? qz.x : qz.y;
+            const float far_limit = best_t * WIDEN_HI;
+            uint32_t key[WIDE_CHILDREN], hits = 0u;
+#define MIPT_CHILD(K, NX, FX, NY, FY, NZ, FZ)                                                                          \
+    {                                                                                                                  \
+        const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(NX, nsx, nbx), __builtin_fmaf(NY, nsy, nby)),                \
+                                     __builtin_fmaf(NZ, nsz, nbz)),                                                    \
+                               0.0f);                                                                                  \
+        const float tf = fminf(fminf(fminf(__builtin_fmaf(FX, fsx, fbx), __builtin_fmaf(FY, fsy, fby)),                \
+                                     __builtin_fmaf(FZ, fsz, fbz)),                                                    \
+                               far_limit);                                                                             \
+        const bool hit = tn <= tf && K < count;                                                                        \
+        key[K] = hit ? ((__float_as_uint(tn) & ~31u) | (5u * K + 1u)) : ~0u;                                           \
+        hits += hit ? 1u : 0u;                                                                                         \
+    }
+            MIPT_CHILD(0, byte_of<0>(nx), byte_of<0>(fx), byte_of<0>(ny), byte_of<0>(fy), byte_of<0>(nz), byte_of<0>(fz))
+            MIPT_CHILD(1, byte_of<1>(nx), byte_of<1>(fx), byte_of<1>(ny), byte_of<1>(fy), byte_of<1>(nz), byte_of<1>(fz))
+            MIPT_CHILD(2, byte_of<2>(nx), byte_of<2>(fx), byte_of<2>(ny), byte_of<2>(fy), byte_of<2>(nz), byte_of<2>(fz))
+            MIPT_CHILD(3, byte_of<3>(nx), byte_of<3>(fx), byte_of<3>(ny), byte_of<3>(fy), byte_of<3>(nz), byte_of<3>(fz))
+            MIPT_CHILD(4, byte_of<0>(tx), byte_of<2>(tx), byte_of<0>(ty), byte_of<2>(ty), byte_of<0>(tz), byte_of<2>(tz))
+            MIPT_CHILD(5, byte_of<1>(tx), byte_of<3>(tx), byte_of<1>(ty), byte_of<3>(ty), byte_of<1>(tz), byte_of<3>(tz))
+#undef MIPT_CHILD
+            sort6(key); // nearest first, misses last
+            auto ref_of = [&](uint32_t k) {
+                const uint32_t m = __builtin_amdgcn_ubfe(refs.z, k, 5u);
+                return (m < 16u ? refs.y : refs.x) + m;
+            };
+            // the nearest is next, the others go on the stack, farthest first:
+            // the k-th nearest to entry sp + hits - 1 - k
+            const int top = sp + (int)hits - 1;
+            if (!__any(top > STACK))
+            {
+#pragma unroll
+                for (int k = 1; k < WIDE_CHILDREN; k++)
+                    if (key[k] != ~0u)
+                        stack[(top - k) * BLOCK + threadIdx.x] = make_uint2(key[k], ref_of(key[k]));
             }
             else
             {
-                const RayHit h = traverse<BLOCK, STACK, false>(nodes, tris, root, ra, rb, false, stack, spill,
-                                                              spill_stride, gtid, max_steps);
-                int4* hits = k == 0 ? q.job[0].hits : (k == 1 ? q.job[1].hits : q.job[2].hits);
-                hits[r] = hit_record(h);
+#pragma unroll
+                for (int k = 1; k < WIDE_CHILDREN; k++)
+                    if (key[k] != ~0u)
+                    {
+                        const uint2 e = make_uint2(key[k], ref_of(key[k]));
+                        if (top - k < STACK)
+                            stack[(top - k) * BLOCK + threadIdx.x] = e;
+                        else
+                            a.spill[(size_t)(top - k - STACK) * a.spill_stride + gtid] = e;
+                    }
+            }
+            cur = IDLE;
+            if (hits > 0u)
+            {
+                sp = top;
+                cur = (int32_t)ref_of(key[0]);
+            }
+        }
+        // A leaf is put aside and the lane goes on; with one put aside already
+        // it waits for its turn. A lane without a node takes one entry: one
+        // behind the closest hit costs it this round, which is cheaper than a
+        // loop that runs as long as any lane drops entries.
+        auto put_aside = [&]() {
+            if (cur < 0 && leaf == 0)
+            {
+                leaf = cur;
+                cur = IDLE;
+            }
+        };
+        put_aside();
+        if (cur == IDLE && sp > 0)
+        {
+            sp--;
+            uint2 e;
+            if (sp < STACK)
+                e = stack[sp * BLOCK + threadIdx.x];
+            else
+                e = a.spill[(size_t)(sp - STACK) * a.spill_stride + gtid];
+            // the entry's distance is already widened downwards
+            if (__uint_as_float(e.x) <= best_t * WIDEN_HI)
+                cur = (int32_t)e.y;
+            put_aside();
+        }
+
+        const uint64_t leaves = __ballot(leaf != 0);
+        if (leaves && (!more || __popcll(leaves) >= LEAF_LANES || !__ballot((uint32_t)cur < (uint32_t)IDLE)))
+        {
+            if (leaf != 0)
+            {
+                const TriRecord* tr = a.tris + ((uint32_t)leaf & ~WIDE_LEAF);
+                const float4 v0 = tr->v0, e1 = tr->e1, e2 = tr->e2;
+                const int32_t prim = __float_as_int(v0.w);
+                if (MODE == CLOSEST_COUNTED)
+                    n_tris++;
+                float t, u, v;
+                leaf = __float_as_int(e1.w) != 0 ? 0 : leaf + 1;
+                if (pt::mt_intersect(pt::mk(v0.x, v0.y, v0.z), pt::mk(e1.x, e1.y, e1.z), pt::mk(e2.x, e2.y, e2.z), o, d,
+                                     t, u, v) &&
+                    prim != last_prim && (t < best_t || (t == best_t && prim < best_prim)))
+                {
+                    best_t = t;
+                    best_prim = prim;
+                    best_u = u;
+                    best_v = v;
+                    if (any)
+                    {
+                        cur = IDLE;
+                        leaf = 0;
+                        sp = 0;
+                    }
+                }
             }
         }
     }
@@ -388,9 +452,7 @@ __global__ void k_all_miss(int4* __restrict__ hits, uint8_t* __restrict__ occlud
         occluded[i] = 0;
 }
 
-using TraceFn = void (*)(const BvhNode*, const TriRecord*, int32_t, const float4*, int4*, uint8_t*, uint2*,
-                         uint32_t, int32_t*, uint32_t, uint32_t*, uint32_t, const uint32_t*, const uint32_t*, uint32_t,
-                         uint32_t);
+using TraceFn = void (*)(TraceArgs);
 
 template <int BLOCK, int STACK>
 TraceFn pick_mode(int mode)
@@ -399,6 +461,7 @@ TraceFn pick_mode(int mode)
     {
     case CLOSEST: return k_trace<BLOCK, STACK, CLOSEST>;
     case ANY: return k_trace<BLOCK, STACK, ANY>;
+    case QUEUED: return k_trace<BLOCK, STACK, QUEUED>;
     default: return k_trace<BLOCK, STACK, CLOSEST_COUNTED>;
     }
 }
@@ -430,31 +493,6 @@ struct Launch {
     unsigned grid;
 };
 
-using QueuesFn = void (*)(const BvhNode*, const TriRecord*, int32_t, QueueJobs, int32_t*, uint32_t, uint32_t*, uint32_t,
-                          uint32_t);
-
-template <int BLOCK>
-QueuesFn pick_queues_stack(int stack)
-{
-    switch (stack)
-    {
-    case 8: return k_trace_queues<BLOCK, 8>;
-    case 16: return k_trace_queues<BLOCK, 16>;
-    case 24: return k_trace_queues<BLOCK, 24>;
-    default: return k_trace_queues<BLOCK, 32>;
-    }
-}
-
-QueuesFn pick_queues(int block, int stack)
-{
-    switch (block)
-    {
-    case 64: return pick_queues_stack<64>(stack);
-    case 128: return pick_queues_stack<128>(stack);
-    default: return pick_queues_stack<256>(stack);
-    }
-}
-
 // Persistent grid: the blocks that fit on the device at once, at most enough
 // for n rays.
 unsigned persistent_grid(Ctx& ctx, const void* fn, uint32_t n)
@@ -481,7 +519,8 @@ unsigned persistent_grid(Ctx& ctx, const void* fn, uint32_t n)
         occupancy[key] = per_cu;
     }
     const uint64_t max_grid = (uint64_t)per_cu * (uint64_t)ctx.cu_count;
-    const uint64_t need = ((uint64_t)n + block - 1) / block;
+    // a wave may take as few as MIN_BATCH rays
+    const uint64_t need = ((uint64_t)n + (uint64_t)(MIN_BATCH * (block / 64)) - 1) / (uint64_t)(MIN_BATCH * (block / 64));
     const uint64_t g = need < max_grid ? need : max_grid;
     return (unsigned)(g ? g : 1);
 }
@@ -494,28 +533,39 @@ Launch plan(Ctx& ctx, int mode, uint32_t n)
     return l;
 }
 
-// n: rays (or, with a queue, the queue's capacity: slots [0, n) of rays).
 // Work counter and spill columns of a persistent grid of `threads` threads.
 struct Scratch {
     uint32_t* counter;
-    int32_t* spill;
+    uint2* spill;
 };
 
 Scratch trace_scratch(Ctx& ctx, uint32_t threads)
 {
-    // Spill entries: the stack never holds more than max_depth entries. The
-    // columns are sized for every thread the device can hold (32 waves per
-    // CU), not for this launch's grid, so that launches of different grids
+    // The columns are sized for every thread the device can hold (32 waves
+    // per CU), not for this launch's grid, so that launches of different grids
     // on one stream never reallocate the buffer under queued kernels.
-    const int spill_depth = ctx.bvh.max_depth - ctx.trace_cfg.lds_stack;
+    const int spill_depth = ctx.bvh.wide_stack - ctx.trace_cfg.lds_stack;
     const size_t spill_off = 256; // work counter lives at the front
     const size_t columns = std::max<size_t>(threads, (size_t)ctx.cu_count * 32u * 64u);
     size_t spill_bytes = spill_off;
     if (spill_depth > 0)
-        spill_bytes = spill_off + sizeof(int32_t) * (size_t)spill_depth * columns;
+        spill_bytes = spill_off + sizeof(uint2) * (size_t)spill_depth * columns;
     ctx.spill.reserve(spill_bytes);
     return Scratch{ctx.spill.as<uint32_t>(),
-                   reinterpret_cast<int32_t*>(reinterpret_cast<char*>(ctx.spill.ptr) + spill_off)};
+                   reinterpret_cast<uint2*>(reinterpret_cast<char*>(ctx.spill.ptr) + spill_off)};
+}
+
+TraceArgs trace_args(Ctx& ctx, uint32_t threads, const Scratch& sc)
+{
+    TraceArgs a{};
+    a.nodes = ctx.bvh.wide.as<WideNode>();
+    a.tris = ctx.bvh.wide_tris.as<TriRecord>();
+    a.spill = sc.spill;
+    a.spill_stride = threads;
+    a.work_counter = sc.counter;
+    a.tile = (uint32_t)ctx.trace_cfg.queue_tile;
+    a.few_waves = (uint32_t)ctx.cu_count * FEW_WAVES_PER_CU;
+    return a;
 }
 
 bool trace_ready(Ctx& ctx)
@@ -526,7 +576,7 @@ bool trace_ready(Ctx& ctx)
 }
 
 void launch(Ctx& ctx, int mode, const mipt_ray* rays, mipt_hit* hits, uint8_t* occluded, uint32_t* counts, uint32_t n,
-            const SegList* queue, hipStream_t stream)
+            hipStream_t stream)
 {
     if (n == 0)
         return;
@@ -541,13 +591,14 @@ void launch(Ctx& ctx, int mode, const mipt_ray* rays, mipt_hit* hits, uint8_t* o
     const int block = ctx.trace_cfg.block_size;
     const uint32_t threads = l.grid * (uint32_t)block;
     const Scratch sc = trace_scratch(ctx, threads);
+    TraceArgs a = trace_args(ctx, threads, sc);
+    a.job[0].rays = reinterpret_cast<const float4*>(rays);
+    a.job[0].hits = reinterpret_cast<int4*>(hits);
+    a.job[0].occluded = occluded;
+    a.counts = reinterpret_cast<uint2*>(counts);
+    a.n = n;
     hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
-    hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(block), 0, stream, ctx.bvh.nodes.as<BvhNode>(),
-                       ctx.bvh.tris.as<TriRecord>(), ctx.bvh.root, reinterpret_cast<const float4*>(rays),
-                       reinterpret_cast<int4*>(hits), occluded, reinterpret_cast<uint2*>(counts), n, sc.spill, threads,
-                       sc.counter, (uint32_t)ctx.bvh.node_count + 1u, queue ? queue->slots : nullptr,
-                       queue ? queue->counts : nullptr, queue ? queue->seg_cap : 0u,
-                       (uint32_t)ctx.trace_cfg.queue_tile);
+    hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(block), 0, stream, a);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -610,28 +661,29 @@ void trace_closest_noalloc(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint3
     // that the whole grid's columns do not fit, the grid shrinks to the
     // blocks whose columns do (every wave takes rays from the work counter,
     // so fewer blocks trace the same rays).
-    const int spill_depth = std::max(0, ctx.bvh.max_depth - ctx.trace_cfg.lds_stack);
+    const int spill_depth = std::max(0, ctx.bvh.wide_stack - ctx.trace_cfg.lds_stack);
     const size_t room = MIPT_TRACE_NOALLOC_SCRATCH_BYTES - NOALLOC_COUNTER_BYTES;
     unsigned grid = l.grid;
     if (spill_depth > 0)
     {
-        const size_t per_block = sizeof(int32_t) * (size_t)spill_depth * (size_t)block;
+        const size_t per_block = sizeof(uint2) * (size_t)spill_depth * (size_t)block;
         const size_t fit = room / per_block;
         if (fit == 0)
             fail(MIPT_ERR_INVALID_ARGUMENT,
-                 "mipt_trace_closest_noalloc: a BVH of depth " + std::to_string(ctx.bvh.max_depth) +
-                     " needs more than the " + std::to_string(MIPT_TRACE_NOALLOC_SCRATCH_BYTES) +
+                 "mipt_trace_closest_noalloc: a BVH of " + std::to_string(ctx.bvh.wide_stack) +
+                     " stack entries needs more than the " + std::to_string(MIPT_TRACE_NOALLOC_SCRATCH_BYTES) +
                      "-byte scratch for one block's spill stack");
         grid = (unsigned)std::min<size_t>(grid, fit);
     }
     const uint32_t threads = grid * (uint32_t)block;
-    uint32_t* counter = reinterpret_cast<uint32_t*>(base);
-    int32_t* spill = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(base) + NOALLOC_COUNTER_BYTES);
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, counter);
-    hipLaunchKernelGGL(l.fn, dim3(grid), dim3(block), 0, stream, ctx.bvh.nodes.as<BvhNode>(),
-                       ctx.bvh.tris.as<TriRecord>(), ctx.bvh.root, reinterpret_cast<const float4*>(rays),
-                       reinterpret_cast<int4*>(hits), nullptr, nullptr, n, spill, threads, counter,
-                       (uint32_t)ctx.bvh.node_count + 1u, nullptr, nullptr, 0u, (uint32_t)ctx.trace_cfg.queue_tile);
+    const Scratch sc{reinterpret_cast<uint32_t*>(base),
+                     reinterpret_cast<uint2*>(reinterpret_cast<char*>(base) + NOALLOC_COUNTER_BYTES)};
+    TraceArgs a = trace_args(ctx, threads, sc);
+    a.job[0].rays = reinterpret_cast<const float4*>(rays);
+    a.job[0].hits = reinterpret_cast<int4*>(hits);
+    a.n = n;
+    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
+    hipLaunchKernelGGL(l.fn, dim3(grid), dim3(block), 0, stream, a);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -668,10 +720,10 @@ void autotune_trace(Ctx& ctx, const mipt_ray* rays, uint32_t n, int32_t repeats,
                     ctx.trace_cfg.lds_stack = stacks[si];
                     ctx.trace_cfg.queue_tile = tiles[ti];
                     // one untimed launch: occupancy query, spill columns
-                    launch(ctx, CLOSEST, rays, hits, nullptr, nullptr, n, nullptr, stream);
+                    launch(ctx, CLOSEST, rays, hits, nullptr, nullptr, n, stream);
                     HIP_CHECK(hipEventRecord(e0, stream));
                     for (int r = 0; r < repeats; r++)
-                        launch(ctx, CLOSEST, rays, hits, nullptr, nullptr, n, nullptr, stream);
+                        launch(ctx, CLOSEST, rays, hits, nullptr, nullptr, n, stream);
                     HIP_CHECK(hipEventRecord(e1, stream));
                     HIP_CHECK(hipEventSynchronize(e1));
                     float ms = 0.0f;
@@ -679,7 +731,8 @@ void autotune_trace(Ctx& ctx, const mipt_ray* rays, uint32_t n, int32_t repeats,
                     const double mean = (double)ms / repeats;
                     if (table)
                         table[(bi * 4 + si) * 3 + ti] = mean;
-                    if (blocks[bi] == 128 && stacks[si] == 16 && tiles[ti] == 1)
+                    if (blocks[bi] == TraceConfig{}.block_size && stacks[si] == TraceConfig{}.lds_stack &&
+                        tiles[ti] == TraceConfig{}.queue_tile)
                         at_default = mean;
                     if (tried == 0 || mean < best)
                     {
@@ -712,24 +765,26 @@ void autotune_trace(Ctx& ctx, const mipt_ray* rays, uint32_t n, int32_t repeats,
 
 void trace_closest(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint32_t* counts, uint32_t n, hipStream_t stream)
 {
-    launch(ctx, counts ? CLOSEST_COUNTED : CLOSEST, rays, hits, nullptr, counts, n, nullptr, stream);
+    launch(ctx, counts ? CLOSEST_COUNTED : CLOSEST, rays, hits, nullptr, counts, n, stream);
 }
 
 void trace_any(Ctx& ctx, const mipt_ray* rays, uint8_t* occluded, uint32_t n, hipStream_t stream)
 {
-    launch(ctx, ANY, rays, nullptr, occluded, nullptr, n, nullptr, stream);
+    launch(ctx, ANY, rays, nullptr, occluded, nullptr, n, stream);
 }
 
 void trace_closest_queue(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, const SegList& queue, uint32_t capacity,
                          hipStream_t stream)
 {
-    launch(ctx, CLOSEST, rays, hits, nullptr, nullptr, capacity, &queue, stream);
+    const TraceQueue q{rays, hits, nullptr, &queue};
+    trace_queues(ctx, &q, 1, capacity, stream);
 }
 
 void trace_any_queue(Ctx& ctx, const mipt_ray* rays, uint8_t* occluded, const SegList& queue, uint32_t capacity,
                      hipStream_t stream)
 {
-    launch(ctx, ANY, rays, nullptr, occluded, nullptr, capacity, &queue, stream);
+    const TraceQueue q{rays, nullptr, occluded, &queue};
+    trace_queues(ctx, &q, 1, capacity, stream);
 }
 
 void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t capacity, hipStream_t stream)
@@ -746,10 +801,14 @@ void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t capacity, h
         HIP_CHECK(hipGetLastError());
         return;
     }
-    QueueJobs jobs{};
+    const Launch l = plan(ctx, QUEUED, (uint32_t)std::min<uint64_t>((uint64_t)capacity * count, 0xffffffffull));
+    const int block = ctx.trace_cfg.block_size;
+    const uint32_t threads = l.grid * (uint32_t)block;
+    const Scratch sc = trace_scratch(ctx, threads);
+    TraceArgs a = trace_args(ctx, threads, sc);
     for (int k = 0; k < count; k++)
     {
-        QueueJob& j = jobs.job[k];
+        QueueJob& j = a.job[k];
         j.rays = reinterpret_cast<const float4*>(q[k].rays);
         j.hits = reinterpret_cast<int4*>(q[k].hits);
         j.occluded = q[k].occluded;
@@ -757,17 +816,8 @@ void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t capacity, h
         j.counts = q[k].queue->counts;
         j.seg_cap = q[k].queue->seg_cap;
     }
-    const int block = ctx.trace_cfg.block_size;
-    const QueuesFn fn = pick_queues(block, ctx.trace_cfg.lds_stack);
-    const unsigned grid = persistent_grid(ctx, reinterpret_cast<const void*>(fn), (uint32_t)std::min<uint64_t>(
-                                                                                     (uint64_t)capacity * count,
-                                                                                     0xffffffffull));
-    const uint32_t threads = grid * (uint32_t)block;
-    const Scratch sc = trace_scratch(ctx, threads);
     hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, stream, ctx.bvh.nodes.as<BvhNode>(),
-                       ctx.bvh.tris.as<TriRecord>(), ctx.bvh.root, jobs, sc.spill, threads, sc.counter,
-                       (uint32_t)ctx.bvh.node_count + 1u, (uint32_t)ctx.trace_cfg.queue_tile);
+    hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(block), 0, stream, a);
     HIP_CHECK(hipGetLastError());
 }
 
