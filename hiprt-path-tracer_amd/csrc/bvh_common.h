@@ -124,17 +124,24 @@ __global__ __launch_bounds__(BOUNDS_BLOCK) void k_tri_boxes(const float* __restr
 
 // Folds the partials of `blocks` blocks into bounds (as ordered uint32,
 // [0..2] scene lo, [3..5] scene hi, [6..8] centroid lo, [9..11] centroid hi)
-// and the absolute pad (2^-22 of the largest scene extent).
-__global__ void k_bounds_final(const float* __restrict__ partial, int32_t blocks, uint32_t* __restrict__ bounds,
-                               float* __restrict__ pad)
+// and the absolute pad (2^-22 of the largest scene extent). One block of 12
+// waves, one for each bound (12 threads of one wave, each over all 1024 partials,
+// took 130 us).
+constexpr int BOUNDS_FINAL_BLOCK = 12 * 64;
+
+__global__ __launch_bounds__(BOUNDS_FINAL_BLOCK) void k_bounds_final(const float* __restrict__ partial, int32_t blocks,
+                                                                     uint32_t* __restrict__ bounds,
+                                                                     float* __restrict__ pad)
 {
     __shared__ float res[12];
-    if (threadIdx.x < 12)
+    const int k = threadIdx.x / 64;
+    const bool lower = (k % 6) < 3;
+    float r = lower ? INFINITY : -INFINITY;
+    for (int32_t b = threadIdx.x % 64; b < blocks; b += 64)
+        r = lower ? fminf(r, partial[12 * b + k]) : fmaxf(r, partial[12 * b + k]);
+    r = lower ? wave_min(r) : wave_max(r);
+    if (threadIdx.x % 64 == 0)
     {
-        const int k = threadIdx.x;
-        float r = (k % 6) < 3 ? INFINITY : -INFINITY;
-        for (int32_t b = 0; b < blocks; b++)
-            r = (k % 6) < 3 ? fminf(r, partial[12 * b + k]) : fmaxf(r, partial[12 * b + k]);
         res[k] = r;
         bounds[k] = f2o(r);
     }
@@ -142,7 +149,7 @@ __global__ void k_bounds_final(const float* __restrict__ partial, int32_t blocks
     if (threadIdx.x == 0)
     {
         float ext = 0.0f;
-        for (int k = 0; k < 3; k++) ext = fmaxf(ext, res[3 + k] - res[k]);
+        for (int a = 0; a < 3; a++) ext = fmaxf(ext, res[3 + a] - res[a]);
         pad[0] = ext * PAD_ABS;
     }
 }
@@ -181,15 +188,35 @@ inline unsigned bounds_grid(int32_t n)
 } // namespace
 } // namespace bvhc
 
-// Host side, after a builder wrote `node_capacity` BvhNodes (root = node 0)
-// and the TriRecords: validates the reachable tree (each interior node
-// reached once, each triangle in exactly one leaf), computes its statistics
-// and SAH cost, and lays the reachable nodes out depth first. Defined in
-// bvh_build.hip.
-void finalize_bvh(Ctx& ctx, int32_t node_capacity);
+// One allocation for all the temporaries of a build: sizes are added first,
+// then get() gives their addresses.
+struct BuildScratch {
+    DeviceBuffer buf;
+    size_t total = 0;
+    size_t add(size_t bytes)
+    {
+        const size_t at = total;
+        total += (bytes + 255) & ~(size_t)255;
+        return at;
+    }
+    void allocate() { buf.reserve(total); }
+    template <class T> T* get(size_t at) const { return reinterpret_cast<T*>(reinterpret_cast<char*>(buf.ptr) + at); }
+};
+
+// Nodes as a builder writes them carry the first triangle of their range in
+// d.z and their depth in d.w, or NODE_UNUSED there when the tree does not hold
+// them.
+constexpr int32_t NODE_UNUSED = -1;
+
+// After a builder wrote `count` such nodes (root = node 0) and the
+// TriRecords: validates the tree (each interior node referenced once, by a
+// parent one level up, each triangle in exactly one leaf), computes its
+// statistics and SAH cost, and lays it out depth first into ctx.bvh.nodes, then
+// makes the wide tree. Defined in bvh_build.hip.
+void finalize_bvh(Ctx& ctx, const BvhNode* d_nodes, int32_t count);
 
 // The one-triangle tree: a root whose first child is the leaf and whose
 // second child has an empty box. Defined in bvh_build.hip.
-void write_single_triangle_root(Ctx& ctx, const float4* d_lo, const float4* d_hi);
+void write_single_triangle_root(BvhNode* d_node, const float4* d_lo, const float4* d_hi);
 
 } // namespace mipt

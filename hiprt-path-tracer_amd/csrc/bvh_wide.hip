@@ -1,9 +1,10 @@
 // bvh_wide.hip -- collapses the built binary tree into the 6-wide quantised
 // tree the traversal walks (layout.h: WideNode).
 //
-// One level of wide nodes per launch, a thread per wide node: it opens the
-// binary node's children, largest box first, until six are held, writes the
-// quantised record and lists its interior children for the next level. The
+// A thread per wide node, level by level: it opens the binary node's children,
+// largest box first, until six are held, writes the quantised record and
+// lists its interior children for the next level. One block does the levels
+// of up to SMALL_LEVEL nodes without the host; each larger level is a launch. The
 // children of a node, and the triangles of its leaf children, are contiguous;
 // the triangles are copied into the order this gives.
 #include <hip/hip_runtime.h>
@@ -15,11 +16,14 @@ namespace mipt {
 namespace {
 
 constexpr int WIDE_BLOCK = 64;
+constexpr int SMALL_BLOCK = 256;
+constexpr uint32_t SMALL_LEVEL = 1024;
 
 struct Counters {
     uint32_t nodes;
     uint32_t tris;
     uint32_t max_stack;
+    uint32_t begin; // first node of the level that k_wide_small left to do
 };
 
 // Exclusive prefix sum over the wave; total gets the wave's sum.
@@ -116,16 +120,12 @@ __device__ __forceinline__ uint32_t pack_tail(const uint8_t* qlo, const uint8_t*
     return (uint32_t)qlo[4] | ((uint32_t)qlo[5] << 8) | ((uint32_t)qhi[4] << 16) | ((uint32_t)qhi[5] << 24);
 }
 
-__global__ __launch_bounds__(WIDE_BLOCK) void k_wide_level(const BvhNode* __restrict__ nodes,
-                                                           const TriRecord* __restrict__ tris, int32_t single,
-                                                           uint32_t begin, uint32_t end,
-                                                           int32_t* __restrict__ item_ref,
-                                                           uint32_t* __restrict__ item_stack,
-                                                           WideNode* __restrict__ out, TriRecord* __restrict__ tri_out,
-                                                           Counters* __restrict__ counters)
+// Makes wide node j (every lane of the wave must call it).
+__device__ __forceinline__ void collapse(const BvhNode* __restrict__ nodes, const TriRecord* __restrict__ tris,
+                                         int32_t single, uint32_t j, bool active, int32_t* item_ref,
+                                         uint32_t* item_stack, WideNode* __restrict__ out,
+                                         TriRecord* __restrict__ tri_out, Counters* counters)
 {
-    const uint32_t j = begin + blockIdx.x * WIDE_BLOCK + threadIdx.x;
-    const bool active = j < end;
     Child c[WIDE_CHILDREN];
     int count = 0;
     if (active)
@@ -262,11 +262,54 @@ __global__ __launch_bounds__(WIDE_BLOCK) void k_wide_level(const BvhNode* __rest
         atomicMax(&counters->max_stack, need);
 }
 
-__global__ void k_wide_init(int32_t* item_ref, uint32_t* item_stack, Counters* counters)
+// The root and the levels after it, up to one of more than SMALL_LEVEL nodes;
+// counters->begin is then that level's first node (all nodes: the tree is done).
+__global__ __launch_bounds__(SMALL_BLOCK) void k_wide_small(const BvhNode* __restrict__ nodes,
+                                                            const TriRecord* __restrict__ tris, int32_t single,
+                                                            int32_t* item_ref, uint32_t* item_stack,
+                                                            WideNode* __restrict__ out, TriRecord* __restrict__ tri_out,
+                                                            Counters* counters)
 {
-    item_ref[0] = 0;
-    item_stack[0] = 0u;
-    *counters = Counters{1u, 0u, 0u};
+    __shared__ uint32_t level_end;
+    if (threadIdx.x == 0)
+    {
+        item_ref[0] = 0;
+        item_stack[0] = 0u;
+        *counters = Counters{1u, 0u, 0u, 0u};
+        level_end = 1u;
+    }
+    __threadfence_block();
+    __syncthreads();
+    uint32_t begin = 0;
+    for (;;)
+    {
+        const uint32_t end = level_end;
+        if (begin == end || end - begin > SMALL_LEVEL)
+            break;
+        for (uint32_t base = begin; base < end; base += SMALL_BLOCK)
+        {
+            const uint32_t j = base + threadIdx.x;
+            collapse(nodes, tris, single, j, j < end, item_ref, item_stack, out, tri_out, counters);
+        }
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0)
+            level_end = atomicAdd(&counters->nodes, 0u);
+        __syncthreads();
+        begin = end;
+    }
+    if (threadIdx.x == 0)
+        counters->begin = begin;
+}
+
+__global__ __launch_bounds__(WIDE_BLOCK) void k_wide_level(const BvhNode* __restrict__ nodes,
+                                                           const TriRecord* __restrict__ tris, int32_t single,
+                                                           uint32_t begin, uint32_t end, int32_t* item_ref,
+                                                           uint32_t* item_stack, WideNode* __restrict__ out,
+                                                           TriRecord* __restrict__ tri_out, Counters* counters)
+{
+    const uint32_t j = begin + blockIdx.x * WIDE_BLOCK + threadIdx.x;
+    collapse(nodes, tris, single, j, j < end, item_ref, item_stack, out, tri_out, counters);
 }
 
 } // namespace
@@ -280,24 +323,33 @@ void build_wide(Ctx& ctx)
     const size_t capacity = (size_t)bvh.node_count;
     bvh.wide.reserve(sizeof(WideNode) * capacity);
     bvh.wide_tris.reserve(sizeof(TriRecord) * (size_t)n);
-    DeviceBuffer item_ref, item_stack, counters;
-    item_ref.reserve(sizeof(int32_t) * capacity);
-    item_stack.reserve(sizeof(uint32_t) * capacity);
-    counters.reserve(sizeof(Counters));
-    hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(1), 0, s, item_ref.as<int32_t>(), item_stack.as<uint32_t>(),
-                       counters.as<Counters>());
-    Counters h{1u, 0u, 0u};
-    for (uint32_t begin = 0; begin < h.nodes;)
-    {
-        const uint32_t end = h.nodes;
-        hipLaunchKernelGGL(k_wide_level, dim3(bvhc::blocks(end - begin, WIDE_BLOCK)), dim3(WIDE_BLOCK), 0, s,
-                           bvh.nodes.as<BvhNode>(), bvh.tris.as<TriRecord>(), (int32_t)(n == 1), begin, end,
-                           item_ref.as<int32_t>(), item_stack.as<uint32_t>(), bvh.wide.as<WideNode>(),
-                           bvh.wide_tris.as<TriRecord>(), counters.as<Counters>());
+    BuildScratch sc;
+    const size_t o_ref = sc.add(sizeof(int32_t) * capacity), o_stack = sc.add(sizeof(uint32_t) * capacity),
+                 o_counters = sc.add(sizeof(Counters));
+    sc.allocate();
+    int32_t* item_ref = sc.get<int32_t>(o_ref);
+    uint32_t* item_stack = sc.get<uint32_t>(o_stack);
+    Counters* counters = sc.get<Counters>(o_counters);
+    const BvhNode* nodes = bvh.nodes.as<BvhNode>();
+    const TriRecord* tris = bvh.tris.as<TriRecord>();
+    WideNode* out = bvh.wide.as<WideNode>();
+    TriRecord* tri_out = bvh.wide_tris.as<TriRecord>();
+    Counters h{};
+    auto read_counters = [&] {
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipMemcpy(&h, counters.ptr, sizeof(h), hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(&h, counters, sizeof(h), hipMemcpyDeviceToHost));
         if (h.nodes > capacity || h.tris > (uint32_t)n)
             fail(MIPT_ERR_HIP, "wide BVH: more nodes or triangles than the binary tree holds");
+    };
+    hipLaunchKernelGGL(k_wide_small, dim3(1), dim3(SMALL_BLOCK), 0, s, nodes, tris, (int32_t)(n == 1), item_ref,
+                       item_stack, out, tri_out, counters);
+    read_counters();
+    for (uint32_t begin = h.begin; begin < h.nodes;)
+    {
+        const uint32_t end = h.nodes;
+        hipLaunchKernelGGL(k_wide_level, dim3(bvhc::blocks(end - begin, WIDE_BLOCK)), dim3(WIDE_BLOCK), 0, s, nodes,
+                           tris, (int32_t)(n == 1), begin, end, item_ref, item_stack, out, tri_out, counters);
+        read_counters();
         begin = end;
     }
     if (h.tris != (uint32_t)n)
