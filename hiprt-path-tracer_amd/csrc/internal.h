@@ -185,7 +185,7 @@ struct Nrc {
     uint32_t last_sel_stride = 1, last_sel_offset = 0, last_sel_limit = 0;
     DeviceBuffer grid_f16, grid_master, grid_m, grid_v, grid_grad;
     DeviceBuffer w_master, w_m, w_v, w_grad, wt, wk;
-    DeviceBuffer x0, xcm, dycm, dx0, loss, count;
+    DeviceBuffer enc, xcm, dycm, dx0, loss, count, grad_bins;
     // records of the path pass
     DeviceBuffer queries, query_pix, query_out, counters, train_queries, train_targets, train_pix, train_rad;
     DeviceBuffer query_list, train_list, list_counts; // segmented pixel lists of the query kernel

@@ -49,17 +49,29 @@ struct NrcDev {
     const _Float16* grid_f16;
 };
 
+// Encoded rows: one plane per grid level with the level's two features of every
+// row (bf16 pair), the NRC_MISC other inputs of each row together (the last
+// 4 are zero), and planes of the row's position in the grid's cube. `stride` rows.
+constexpr int NRC_MISC = 32;
+
+struct EncDev {
+    uint32_t* feat; // [levels][stride]
+    uint16_t* misc; // [stride][NRC_MISC]
+    float* pos;     // [3][stride]
+    uint32_t stride;
+};
+
 struct NrcTrainDev {
     const uint16_t* wt;   // W^T per layer, [N][64] bf16
     const uint16_t* wk;   // W per layer, [64][N] bf16
-    const uint16_t* x0;   // encoded rows, [rows][64] bf16
+    EncDev enc;           // the batch's encoded rows
     const float* targets; // [records][4]
     RowSel sel;           // the batch's rows among the records
     uint32_t batch_stride;
     int32_t levels;
     uint16_t* xcm;        // layer inputs, column-major [layer][64][stride]
     uint16_t* dycm;       // layer output gradients, column-major [layer][64][stride]
-    float* dx0;           // grid-feature gradients [stride][32]
+    float* dx0;           // grid-feature gradients, column-major [2 * levels][batch_stride]
     float* loss_sum;
     float* wgrad;         // FP32 [K][N] per layer
     float* ggrad;         // FP32 grid gradient

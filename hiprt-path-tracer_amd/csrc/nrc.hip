@@ -27,6 +27,13 @@ namespace {
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
+// Rows from which the grid gradient is binned instead of added by global
+// atomics. A whole training step, atomics against bins: 2048 rows 214 / 234 us
+// at 2^19 entries a level, 99 / 101 us at 2^14; 4096 rows 247 / 238 and 128 / 113;
+// 65,536 rows 1146 / 489 and 1006 / 309.
+constexpr uint32_t GRAD_BIN_MIN_ROWS = 4096;
+constexpr uint32_t GRAD_MAX_RANGES = 1u << (24 - 13); // per level (log2_table is at most 24)
+constexpr uint32_t GRAD_BIN_ROWS = 1u << 16;          // rows binned at a time: 100 MB of updates at most
 constexpr int TILE_LD = NRC_WIDTH + 8; // LDS row stride (bf16) of an activation tile
 
 // binary32 -> bfloat16, round to nearest even (finite inputs).
@@ -108,89 +115,155 @@ __device__ __forceinline__ void normalized_position(const NrcDev& P, const float
 }
 
 // Query record (16 floats): position, direction, normal, roughness, albedo.
-// Encodes the selected rows into x0 rows [0, rows) and zero-fills the rows up
-// to the next multiple of pad (at most n rows in all).
+// Encodes the selected rows into E rows [0, rows) and zero-fills the rows up
+// to the next multiple of pad (at most n rows in all), in two kernels.
 //
-// Launch: NRC_XCDS x chunks blocks of 128 threads (encode_launch). Workgroups
-// go to the 8 XCDs round-robin, so block b runs on XCD b % 8 and interpolates
-// the levels l with l % 8 == b % 8 for rows [128 (b / 8), +128): each XCD's
-// L2 (4 MB) then holds the tables of two levels (2 MB of FP16 pairs each at
-// 2^19 entries) instead of missing on all sixteen. The block whose chunk
-// index matches its XCD (chunk % 8 == b % 8) also writes the other inputs
-// and the zero padding of its rows.
-constexpr uint32_t NRC_XCDS = 8;
-
-__global__ __launch_bounds__(128) void k_nrc_encode(NrcDev P, const float4* __restrict__ queries, RowSel sel,
-                                                    uint32_t n, uint32_t pad, uint16_t* __restrict__ x0)
+// k_nrc_inputs reads each record once: the inputs that are not grid features,
+// and the position in the grid's cube.
+__global__ __launch_bounds__(256) void k_nrc_inputs(NrcDev P, const float4* __restrict__ queries, RowSel sel,
+                                                    uint32_t n, uint32_t pad, EncDev E)
 {
-    const uint32_t xcd = blockIdx.x % NRC_XCDS;
-    const uint32_t chunk = blockIdx.x / NRC_XCDS;
-    const uint32_t row = chunk * blockDim.x + threadIdx.x;
+    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t rows = sel.rows();
     const uint32_t padded = (rows + pad - 1) / pad * pad;
     if (row >= n || row >= padded)
         return;
-    uint16_t* out = x0 + (size_t)row * NRC_WIDTH;
-    const bool misc = chunk % NRC_XCDS == xcd;
+    uint4* out = reinterpret_cast<uint4*>(E.misc + (size_t)row * NRC_MISC);
     if (row >= rows)
     {
-        if (misc)
-            for (int k = 0; k < NRC_WIDTH; k += 8)
-                *reinterpret_cast<uint4*>(out + k) = make_uint4(0u, 0u, 0u, 0u);
+        for (int k = 0; k < NRC_MISC / 8; k++)
+            out[k] = make_uint4(0u, 0u, 0u, 0u);
         return;
     }
     const size_t rec = sel.record(row);
-    const float4 a = queries[4 * rec];
-    const float q3[3] = {a.x, a.y, a.z};
-    float pos[3];
-    normalized_position(P, q3, pos);
-    const uint32_t tmask = (1u << P.log2_table) - 1u;
-    for (int l = (int)xcd; l < P.levels; l += (int)NRC_XCDS)
-    {
-        const NrcGridLevel& L = P.level[l];
-        float f0 = 0.0f, f1 = 0.0f;
-        for (int cc = 0; cc < 8; cc++)
-        {
-            uint32_t idx;
-            float w;
-            corner(L, pos, cc, tmask, idx, w);
-            const size_t e = ((size_t)l << P.log2_table) + idx;
-            const uint32_t pair = reinterpret_cast<const uint32_t*>(P.grid_f16)[e];
-            f0 += w * (float)__builtin_bit_cast(_Float16, (uint16_t)(pair & 0xffffu));
-            f1 += w * (float)__builtin_bit_cast(_Float16, (uint16_t)(pair >> 16));
-        }
-        *reinterpret_cast<uint32_t*>(out + 2 * l) = (uint32_t)to_bf16(f0) | ((uint32_t)to_bf16(f1) << 16);
-    }
-    if (!misc)
-        return;
-    const float4 b = queries[4 * rec + 1], c = queries[4 * rec + 2], d = queries[4 * rec + 3];
+    const float4 a = queries[4 * rec], b = queries[4 * rec + 1], c = queries[4 * rec + 2], d = queries[4 * rec + 3];
     const float q[16] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
-    int k = 2 * P.levels;
+    float pos[3];
+    normalized_position(P, q, pos);
+    for (int i = 0; i < 3; i++)
+        E.pos[(size_t)i * E.stride + row] = pos[i];
+    uint16_t m[NRC_MISC];
     float u, v;
     oct_uv(q[3], q[4], q[5], u, v);
-    one_blob(u, out + k);
-    one_blob(v, out + k + NRC_BLOB);
-    k += 2 * NRC_BLOB;
+    one_blob(u, m);
+    one_blob(v, m + NRC_BLOB);
     oct_uv(q[6], q[7], q[8], u, v);
-    one_blob(u, out + k);
-    one_blob(v, out + k + NRC_BLOB);
-    k += 2 * NRC_BLOB;
-    one_blob(q[9], out + k);
-    k += NRC_BLOB;
-    out[k++] = to_bf16(q[10]);
-    out[k++] = to_bf16(q[11]);
-    out[k++] = to_bf16(q[12]);
-    out[k++] = to_bf16(1.0f);
-    for (; k < NRC_WIDTH; k++)
-        out[k] = 0;
+    one_blob(u, m + 2 * NRC_BLOB);
+    one_blob(v, m + 3 * NRC_BLOB);
+    one_blob(q[9], m + 4 * NRC_BLOB);
+    m[5 * NRC_BLOB] = to_bf16(q[10]);
+    m[5 * NRC_BLOB + 1] = to_bf16(q[11]);
+    m[5 * NRC_BLOB + 2] = to_bf16(q[12]);
+    m[5 * NRC_BLOB + 3] = to_bf16(1.0f);
+    for (int k = 5 * NRC_BLOB + 4; k < NRC_MISC; k++)
+        m[k] = 0;
+    for (int k = 0; k < NRC_MISC / 8; k++)
+    {
+        uint32_t w[4];
+        for (int i = 0; i < 4; i++)
+            w[i] = (uint32_t)m[8 * k + 2 * i] | ((uint32_t)m[8 * k + 2 * i + 1] << 16);
+        out[k] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
+// k_nrc_grid interpolates one level for one row per thread. Workgroups go to
+// the 8 XCDs round-robin, so block b runs on XCD b % 8: it takes level
+// b % 8 for every row first and level b % 8 + 8 after that, so that an XCD's L2
+// (4 MB) holds one level's table (2 MB of FP16 pairs at 2^19 entries) and the
+// position planes stream past it. The two corners along x are next to
+// each other in the table when the lower one's x is even (hashed: the
+// index is x XOR terms of y and z) or the level is dense and its index
+// even: one 8-byte load then brings both.
+//
+// Bound by the gathers (a lane's 4 or 8 bytes are a cache access of their own).
+// Reading the 64-byte records on every XCD and writing 4 bytes of each
+// 128-byte input row from each of them cost more than the gathers:
+// 1,000,003 rows x 16 levels took 800 us that way.
+constexpr uint32_t NRC_XCDS = 8;
+
+__global__ __launch_bounds__(256) void k_nrc_grid(NrcDev P, RowSel sel, uint32_t n, uint32_t pad, uint32_t chunks,
+                                                  EncDev E)
+{
+    const uint32_t turn = blockIdx.x / NRC_XCDS;
+    const int l = (int)(blockIdx.x % NRC_XCDS + NRC_XCDS * (turn / chunks));
+    const uint32_t row = (turn % chunks) * blockDim.x + threadIdx.x;
+    const uint32_t rows = sel.rows();
+    const uint32_t padded = (rows + pad - 1) / pad * pad;
+    if (l >= P.levels || row >= n || row >= padded)
+        return;
+    uint32_t* out = E.feat + (size_t)l * E.stride + row;
+    if (row >= rows)
+    {
+        *out = 0u;
+        return;
+    }
+    float pos[3];
+    for (int i = 0; i < 3; i++)
+        pos[i] = E.pos[(size_t)i * E.stride + row];
+    const uint32_t tmask = (1u << P.log2_table) - 1u;
+    const NrcGridLevel& L = P.level[l];
+    const uint32_t* table = reinterpret_cast<const uint32_t*>(P.grid_f16) + ((size_t)l << P.log2_table);
+    uint32_t pair[8];
+    float w[8];
+    for (int cc = 0; cc < 8; cc += 2)
+    {
+        uint32_t i0, i1;
+        corner(L, pos, cc, tmask, i0, w[cc]);
+        corner(L, pos, cc + 1, tmask, i1, w[cc + 1]);
+        const uint2 both = *reinterpret_cast<const uint2*>(table + (i0 & ~1u));
+        pair[cc] = (i0 & 1u) ? both.y : both.x;
+        pair[cc + 1] = (i0 & 1u) ? both.x : both.y;
+        if (i1 != (i0 ^ 1u))
+            pair[cc + 1] = table[i1];
+    }
+    float f0 = 0.0f, f1 = 0.0f;
+    for (int cc = 0; cc < 8; cc++)
+    {
+        f0 += w[cc] * (float)__builtin_bit_cast(_Float16, (uint16_t)(pair[cc] & 0xffffu));
+        f1 += w[cc] * (float)__builtin_bit_cast(_Float16, (uint16_t)(pair[cc] >> 16));
+    }
+    *out = (uint32_t)to_bf16(f0) | ((uint32_t)to_bf16(f1) << 16);
+}
+
+// Rows of NRC_WIDTH inputs as the network counts them: the grid features,
+// the other inputs, zeros (a thread per pair of inputs).
+__global__ void k_nrc_rows(EncDev E, int levels, uint32_t n, uint32_t* __restrict__ out)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t row = (uint32_t)(i / (NRC_WIDTH / 2));
+    const int k = (int)(i % (NRC_WIDTH / 2));
+    if (row >= n)
+        return;
+    uint32_t v = 0u;
+    if (k < levels)
+        v = E.feat[(size_t)k * E.stride + row];
+    else if (k - levels < NRC_MISC / 2)
+        v = reinterpret_cast<const uint32_t*>(E.misc + (size_t)row * NRC_MISC)[k - levels];
+    out[i] = v;
+}
+
+// The cache's encode workspace for n rows.
+EncDev enc_buffer(Nrc& C, uint32_t n)
+{
+    EncDev E{};
+    E.stride = (n + 63u) & ~63u;
+    const size_t S = E.stride;
+    const int levels = C.settings.grid_levels;
+    C.enc.reserve(S * (4 * (size_t)levels + 2 * NRC_MISC + 4 * 3));
+    E.feat = C.enc.as<uint32_t>();
+    E.misc = reinterpret_cast<uint16_t*>(E.feat + S * levels);
+    E.pos = reinterpret_cast<float*>(E.misc + S * NRC_MISC);
+    return E;
 }
 
 void encode_launch(const NrcDev& P, const float* d_queries, const RowSel& sel, uint32_t n, uint32_t pad,
-                   uint16_t* x0, hipStream_t s)
+                   const EncDev& E, hipStream_t s)
 {
-    const unsigned chunks = (unsigned)((n + 127u) / 128u);
-    hipLaunchKernelGGL(k_nrc_encode, dim3(NRC_XCDS * chunks), dim3(128), 0, s, P,
-                       reinterpret_cast<const float4*>(d_queries), sel, n, pad, x0);
+    const unsigned chunks = (n + 255u) / 256u;
+    const unsigned turns = ((unsigned)P.levels + NRC_XCDS - 1) / NRC_XCDS;
+    hipLaunchKernelGGL(k_nrc_inputs, dim3(chunks), dim3(256), 0, s, P, reinterpret_cast<const float4*>(d_queries), sel,
+                       n, pad, E);
+    hipLaunchKernelGGL(k_nrc_grid, dim3(NRC_XCDS * turns * chunks), dim3(256), 0, s, P, sel, n, pad, chunks, E);
 }
 
 // ---------------------------------------------------------------------------
@@ -213,54 +286,114 @@ __device__ __forceinline__ v4f layer_block(const v8bf a[2], const uint16_t* wt, 
     return acc;
 }
 
-// Inference: out[row] = MLP(x0[row]) (RGB + 0), rows < count.
-__global__ __launch_bounds__(256) void k_nrc_forward(const uint16_t* __restrict__ wt_global,
-                                                     const uint16_t* __restrict__ x0, const uint32_t* count,
-                                                     uint32_t n, float4* __restrict__ out)
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+// Two binary32 -> bfloat16 (round to nearest even), in one instruction.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b)
 {
-    __shared__ uint16_t wt[NRC_WEIGHTS];
-    __shared__ uint16_t tiles[4][16 * TILE_LD];
-    load_weights_lds(wt_global, wt, NRC_WEIGHTS);
-    __syncthreads();
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));
+}
+
+constexpr int FWD_FRAGS = (NRC_LAYERS - 1) * 8 + 2; // 64-lane weight fragments: 4 feature blocks x 2 k-steps a layer
+
+// Inference: out[row] = MLP(encoded row) (RGB + 0), rows < count.
+//
+// Each layer is the transposed product W^T X^T: the rows are the columns of
+// the MFMA's result, and a lane that holds features 16 mb + 4 g + i (g = lane / 16,
+// i < 4) of a row feeds them to the next layer as they are, with the next
+// weights' k order permuted to match (fragment (mb, s), slot 8 g + j of k-step s:
+// feature 16 (2 s + j / 4) + 4 g + j % 4). The activations never leave the
+// registers, and a weight fragment read from LDS serves the 64 rows (4
+// columns blocks) of a wave: through LDS tiles of 16 rows, with the fragments
+// read for each, 1,000,003 rows took 132 us.
+__global__ __launch_bounds__(256, 3) void k_nrc_forward(const uint16_t* __restrict__ wt_global, EncDev E, int levels,
+                                                     const uint32_t* count, uint32_t n, float4* __restrict__ out)
+{
+    __shared__ uint4 frag[FWD_FRAGS * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t rows = *count < n ? *count : n;
-    uint16_t* tile = tiles[wave];
-    const uint32_t tiles_total = (rows + 15) / 16;
-    for (uint32_t t = blockIdx.x * 4 + wave; t < tiles_total; t += gridDim.x * 4)
+    if (blockIdx.x * 4u * 64u >= rows)
+        return;
+    for (int f = wave; f < FWD_FRAGS; f += 4)
     {
-        const uint32_t r0 = t * 16;
-        v8bf a[2];
-        for (int s = 0; s < 2; s++)
-            a[s] = load_v8(x0 + (size_t)(r0 + (lane & 15)) * NRC_WIDTH + 32 * s + 8 * (lane >> 4));
-        for (int layer = 0; layer < NRC_LAYERS; layer++)
+        const int layer = f < 40 ? f / 8 : 5, mb = f < 40 ? (f % 8) / 2 : 0, s = f % 2;
+        const int g = lane >> 4;
+        const uint16_t* w = wt_global + NRC_WOFF(layer) + (size_t)(16 * mb + (lane & 15)) * NRC_WIDTH;
+        uint16_t v[8];
+        for (int j = 0; j < 8; j++)
         {
-            const uint16_t* w = wt + NRC_WOFF(layer);
-            if (layer < NRC_LAYERS - 1)
+            // layer 0 takes the grid features in k-step 0 and the other inputs in step 1
+            const int slot = 8 * g + j;
+            const int k = layer > 0 ? 16 * (2 * s + (j >> 2)) + 4 * g + (j & 3) : (s == 0 ? slot : 2 * levels + slot);
+            v[j] = k < NRC_WIDTH && (layer > 0 || s == 1 || slot < 2 * levels) ? w[k] : (uint16_t)0;
+        }
+        frag[f * 64 + lane] = make_uint4((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16),
+                                         (uint32_t)v[4] | ((uint32_t)v[5] << 16), (uint32_t)v[6] | ((uint32_t)v[7] << 16));
+    }
+    __syncthreads();
+    const uint32_t tiles = (rows + 63) / 64;
+    const int col = lane & 15, g = lane >> 4;
+    for (uint32_t t = blockIdx.x * 4 + wave; t < tiles; t += gridDim.x * 4)
+    {
+        // rows 4 col + q of the 64 (q < 4: the column block)
+        const uint32_t r = t * 64 + 4 * col;
+        uint32_t x[4][2][4]; // [column block][k-step][8 bf16]
+        for (int p = 0; p < 4; p++)
+        {
+            const int l = 4 * g + p;
+            uint4 f = make_uint4(0u, 0u, 0u, 0u);
+            if (l < levels)
+                f = *reinterpret_cast<const uint4*>(E.feat + (size_t)l * E.stride + r);
+            x[0][0][p] = f.x;
+            x[1][0][p] = f.y;
+            x[2][0][p] = f.z;
+            x[3][0][p] = f.w;
+        }
+        for (int q = 0; q < 4; q++)
+        {
+            const uint4 m = *reinterpret_cast<const uint4*>(E.misc + (size_t)(r + q) * NRC_MISC + 8 * g);
+            x[q][1][0] = m.x;
+            x[q][1][1] = m.y;
+            x[q][1][2] = m.z;
+            x[q][1][3] = m.w;
+        }
+        auto operand = [](const uint32_t* v) { return __builtin_bit_cast(v8bf, make_uint4(v[0], v[1], v[2], v[3])); };
+#pragma unroll 1
+        for (int layer = 0; layer < NRC_LAYERS - 1; layer++)
+        {
+            uint32_t y[4][2][4];
+#pragma unroll
+            for (int mb = 0; mb < 4; mb++)
             {
-                for (int nb = 0; nb < 4; nb++)
+                const v8bf a0 = __builtin_bit_cast(v8bf, frag[(layer * 8 + 2 * mb) * 64 + lane]);
+                const v8bf a1 = __builtin_bit_cast(v8bf, frag[(layer * 8 + 2 * mb + 1) * 64 + lane]);
+#pragma unroll
+                for (int q = 0; q < 4; q++)
                 {
-                    const v4f acc = layer_block(a, w, nb, lane);
-                    for (int i = 0; i < 4; i++)
-                        tile[(4 * (lane >> 4) + i) * TILE_LD + 16 * nb + (lane & 15)] = to_bf16(fmaxf(acc[i], 0.0f));
+                    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                    acc = mfma(a0, operand(x[q][0]), acc);
+                    acc = mfma(a1, operand(x[q][1]), acc);
+                    y[q][mb >> 1][2 * (mb & 1)] = pack_bf16(fmaxf(acc[0], 0.0f), fmaxf(acc[1], 0.0f));
+                    y[q][mb >> 1][2 * (mb & 1) + 1] = pack_bf16(fmaxf(acc[2], 0.0f), fmaxf(acc[3], 0.0f));
                 }
-                __builtin_amdgcn_s_waitcnt(0xc07f);
-                __builtin_amdgcn_wave_barrier();
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
                 for (int s = 0; s < 2; s++)
-                    a[s] = load_v8(tile + (lane & 15) * TILE_LD + 32 * s + 8 * (lane >> 4));
-                __builtin_amdgcn_wave_barrier();
-            }
-            else
-            {
-                const v4f acc = layer_block(a, w, 0, lane);
-                const int col = lane & 15;
-                if (col < 4)
                     for (int i = 0; i < 4; i++)
-                    {
-                        const uint32_t row = r0 + 4 * (lane >> 4) + i;
-                        if (row < rows)
-                            reinterpret_cast<float*>(out)[4 * (size_t)row + col] = col < 3 ? acc[i] : 0.0f;
-                    }
-            }
+                        x[q][s][i] = y[q][s][i];
+        }
+        const v8bf a0 = __builtin_bit_cast(v8bf, frag[40 * 64 + lane]);
+        const v8bf a1 = __builtin_bit_cast(v8bf, frag[41 * 64 + lane]);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            acc = mfma(a0, operand(x[q][0]), acc);
+            acc = mfma(a1, operand(x[q][1]), acc);
+            if (g == 0 && r + q < rows)
+                out[r + q] = make_float4(acc[0], acc[1], acc[2], 0.0f);
         }
     }
 }
@@ -268,7 +401,7 @@ __global__ __launch_bounds__(256) void k_nrc_forward(const uint16_t* __restrict_
 // Training: forward, loss gradient and backward of one 16-row tile per wave.
 // Writes the layer inputs X_l and output gradients dY_l column-major
 // ([64][batch_stride], bf16) for the weight-gradient GEMMs, dX0 (float,
-// [batch][2 * levels]) for the grid, and adds the loss to *loss_sum. Tiles
+// column-major) for the grid, and adds the loss to *loss_sum. Tiles
 // cover the rows rounded up to 32 (the k-step of the dW GEMM); the encoded
 // rows past the count are zero, so their activations and gradients are zero.
 __global__ __launch_bounds__(256) void k_nrc_train_fwd_bwd(NrcTrainDev T)
@@ -286,13 +419,27 @@ __global__ __launch_bounds__(256) void k_nrc_train_fwd_bwd(NrcTrainDev T)
     for (uint32_t t = blockIdx.x * 4 + wave; t < tiles_total; t += gridDim.x * 4)
     {
         const uint32_t r0 = t * 16;
-        // layer-0 input tile (row-major in LDS) from the encoded rows
+        // layer-0 input tile (row-major in LDS) from the encoded rows: 4 rows
+        // of a level's plane, and a quarter of a row's other inputs, per lane
         uint16_t* x_in = acts[wave][0];
-        for (int s = 0; s < 2; s++)
         {
-            const int r = lane & 15, k0 = 32 * s + 8 * (lane >> 4);
-            *reinterpret_cast<uint4*>(x_in + r * TILE_LD + k0) =
-                *reinterpret_cast<const uint4*>(T.x0 + (size_t)(r0 + r) * NRC_WIDTH + k0);
+            const int l = lane >> 2, r = 4 * (lane & 3);
+            if (l < T.levels)
+            {
+                const uint4 f = *reinterpret_cast<const uint4*>(T.enc.feat + (size_t)l * T.enc.stride + r0 + r);
+                const uint32_t v[4] = {f.x, f.y, f.z, f.w};
+                for (int i = 0; i < 4; i++)
+                    *reinterpret_cast<uint32_t*>(x_in + (r + i) * TILE_LD + 2 * l) = v[i];
+            }
+            const int row = lane >> 2, k0 = 8 * (lane & 3);
+            const uint4 m = *reinterpret_cast<const uint4*>(T.enc.misc + (size_t)(r0 + row) * NRC_MISC + k0);
+            const uint32_t v[4] = {m.x, m.y, m.z, m.w};
+            uint16_t* dst = x_in + row * TILE_LD + 2 * T.levels + k0;
+            for (int i = 0; i < 4; i++)
+                *reinterpret_cast<uint32_t*>(dst + 2 * i) = v[i];
+            // zeros after them (with fewer than 16 levels)
+            for (int k = 2 * T.levels + NRC_MISC + 2 * (lane & 3); k < NRC_WIDTH; k += 8)
+                *reinterpret_cast<uint32_t*>(x_in + row * TILE_LD + k) = 0u;
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);
         __builtin_amdgcn_wave_barrier();
@@ -401,12 +548,11 @@ __global__ __launch_bounds__(256) void k_nrc_train_fwd_bwd(NrcTrainDev T)
                 else
                 {
                     // gradient of the grid features (columns < 2 * levels)
+                    const uint32_t row = r0 + 4 * (lane >> 4);
                     if (k < 2 * T.levels)
-                        for (int i = 0; i < 4; i++)
-                        {
-                            const uint32_t row = r0 + 4 * (lane >> 4) + i;
-                            T.dx0[(size_t)row * NRC_GRID_MAX + k] = row < rows ? acc[i] : 0.0f;
-                        }
+                        *reinterpret_cast<float4*>(T.dx0 + (size_t)k * S + row) =
+                            make_float4(row < rows ? acc[0] : 0.0f, row + 1 < rows ? acc[1] : 0.0f,
+                                        row + 2 < rows ? acc[2] : 0.0f, row + 3 < rows ? acc[3] : 0.0f);
                 }
             }
             __builtin_amdgcn_s_waitcnt(0xc07f);
@@ -458,38 +604,243 @@ __global__ __launch_bounds__(256) void k_nrc_weight_grad(NrcTrainDev T, uint32_t
         }
 }
 
-// Grid gradient: scatters the feature gradients to the 8 corners of a level.
-__global__ __launch_bounds__(128) void k_nrc_grid_grad(NrcDev P, NrcTrainDev T, const float4* __restrict__ queries)
+// Grid gradient by global atomics: a thread per (row, level) adds the feature
+// gradients to the level's 8 corners.
+__global__ __launch_bounds__(128) void k_nrc_grid_grad(NrcDev P, NrcTrainDev T)
 {
-    // One thread per (row, level): a batch has few rows, and a row's 16 levels
-    // x 8 corners x 2 atomics in one thread left the GPU latency-bound. Blocks
-    // map to XCDs as in k_nrc_encode (levels l % 8 == block % 8), so each
-    // XCD's atomics stay within the tables of two levels.
-    const uint32_t xcd = blockIdx.x % NRC_XCDS;
-    const uint32_t row = (blockIdx.x / NRC_XCDS) * blockDim.x + threadIdx.x;
+    const int l = (int)blockIdx.y;
+    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t rows = T.sel.rows();
     if (row >= rows)
         return;
-    const float4 a = queries[4 * T.sel.record(row)];
-    const float q[3] = {a.x, a.y, a.z};
     float pos[3];
-    normalized_position(P, q, pos);
+    for (int i = 0; i < 3; i++)
+        pos[i] = T.enc.pos[(size_t)i * T.enc.stride + row];
     const uint32_t tmask = (1u << P.log2_table) - 1u;
     const float scale = 1.0f / (3.0f * (float)rows);
-    for (int l = (int)xcd; l < P.levels; l += (int)NRC_XCDS)
+    const NrcGridLevel& L = P.level[l];
+    const float g0 = T.dx0[(size_t)(2 * l) * T.batch_stride + row] * scale;
+    const float g1 = T.dx0[(size_t)(2 * l + 1) * T.batch_stride + row] * scale;
+    for (int cc = 0; cc < 8; cc++)
     {
-        const NrcGridLevel& L = P.level[l];
-        const float g0 = T.dx0[(size_t)row * NRC_GRID_MAX + 2 * l] * scale;
-        const float g1 = T.dx0[(size_t)row * NRC_GRID_MAX + 2 * l + 1] * scale;
+        uint32_t idx;
+        float w;
+        corner(L, pos, cc, tmask, idx, w);
+        const size_t e = ((size_t)l << P.log2_table) + idx;
+        atomicAdd(T.ggrad + 2 * e, w * g0);
+        atomicAdd(T.ggrad + 2 * e + 1, w * g1);
+    }
+}
+
+// The same without global atomics on the gradient, which the memory side serves at
+// 18 G/s however they are ordered: the corner updates are binned by ranges
+// of 2^log2_e table entries of a level (count, prefix sums, scatter), then a
+// block adds the updates of one range in LDS and writes the range once.
+struct GradBins {
+    uint32_t* counts;  // [levels][ranges]
+    uint32_t* cursors; // [levels][ranges]: first free place of each bin
+    uint32_t* entry;   // [levels][rows * 8]: entry within its range
+    float2* value;     // the same places: the two features' addends
+    uint2* items;      // (bin, first update of it) a block adds; item_count of them
+    uint32_t* item_count;
+    uint32_t places;   // rows * 8: places of a level
+    uint32_t first_row, rows; // this pass's rows
+    int log2_e;
+};
+
+// The 8 corners of a row at a level.
+__device__ __forceinline__ void row_corners(const NrcDev& P, const EncDev& E, int l, uint32_t row, uint32_t idx[8],
+                                            float w[8])
+{
+    float pos[3];
+    for (int i = 0; i < 3; i++)
+        pos[i] = E.pos[(size_t)i * E.stride + row];
+    const uint32_t tmask = (1u << P.log2_table) - 1u;
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++)
+        corner(P.level[l], pos, cc, tmask, idx[cc], w[cc]);
+}
+
+constexpr int GRAD_BIN_BLOCK = 512;
+constexpr int GRAD_ADD_BLOCK = 512;
+constexpr uint32_t GRAD_SHARE = 8192; // updates a block adds (4096 and 16384: within 10 %)
+
+__global__ void k_nrc_bins_reset(GradBins B, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        B.counts[i] = 0u;
+    if (i == 0u)
+        *B.item_count = 0u;
+}
+
+template <bool SCATTER>
+__global__ __launch_bounds__(GRAD_BIN_BLOCK) void k_nrc_bin(NrcDev P, NrcTrainDev T, GradBins B)
+{
+    __shared__ uint32_t hist[GRAD_MAX_RANGES], base[GRAD_MAX_RANGES];
+    const int l = (int)blockIdx.y;
+    const uint32_t ranges = 1u << (P.log2_table - B.log2_e);
+    const uint32_t rows = T.sel.rows();
+    const uint32_t end = min(B.first_row + B.rows, rows);
+    const uint32_t row = B.first_row + blockIdx.x * GRAD_BIN_BLOCK + threadIdx.x;
+    if (row - threadIdx.x >= end)
+        return;
+    for (uint32_t i = threadIdx.x; i < ranges; i += GRAD_BIN_BLOCK)
+        hist[i] = 0u;
+    __syncthreads();
+    uint32_t idx[8], rank[8];
+    float w[8];
+    if (row < end)
+    {
+        row_corners(P, T.enc, l, row, idx, w);
+#pragma unroll
         for (int cc = 0; cc < 8; cc++)
+            rank[cc] = atomicAdd(&hist[idx[cc] >> B.log2_e], 1u);
+    }
+    __syncthreads();
+    uint32_t* global = (SCATTER ? B.cursors : B.counts) + (size_t)l * ranges;
+    for (uint32_t i = threadIdx.x; i < ranges; i += GRAD_BIN_BLOCK)
+        if (hist[i] > 0u)
+            base[i] = atomicAdd(&global[i], hist[i]);
+    if (!SCATTER)
+        return;
+    __syncthreads();
+    if (row >= end)
+        return;
+    const float scale = 1.0f / (3.0f * (float)rows);
+    const float g0 = T.dx0[(size_t)(2 * l) * T.batch_stride + row] * scale;
+    const float g1 = T.dx0[(size_t)(2 * l + 1) * T.batch_stride + row] * scale;
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++)
+    {
+        const size_t at = (size_t)l * B.places + base[idx[cc] >> B.log2_e] + rank[cc];
+        B.entry[at] = idx[cc] & ((1u << B.log2_e) - 1u);
+        B.value[at] = make_float2(w[cc] * g0, w[cc] * g1);
+    }
+}
+
+// Start of each bin within its level (one block per level), and the list of the
+// blocks' shares: GRAD_SHARE updates of a bin at most.
+__global__ __launch_bounds__(256) void k_nrc_bin_starts(GradBins B, uint32_t ranges)
+{
+    __shared__ uint32_t part[256];
+    const uint32_t* counts = B.counts + (size_t)blockIdx.x * ranges;
+    uint32_t* cursors = B.cursors + (size_t)blockIdx.x * ranges;
+    const uint32_t per = (ranges + 255u) / 256u, first = threadIdx.x * per;
+    uint32_t sum = 0u;
+    for (uint32_t i = first; i < min(first + per, ranges); i++)
+        sum += counts[i];
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    for (uint32_t off = 1; off < 256u; off <<= 1)
+    {
+        const uint32_t v = threadIdx.x >= off ? part[threadIdx.x - off] : 0u;
+        __syncthreads();
+        part[threadIdx.x] += v;
+        __syncthreads();
+    }
+    uint32_t start = part[threadIdx.x] - sum;
+    for (uint32_t i = first; i < min(first + per, ranges); i++)
+    {
+        cursors[i] = start;
+        start += counts[i];
+        const uint32_t shares = (counts[i] + GRAD_SHARE - 1u) / GRAD_SHARE;
+        if (shares > 0u)
         {
-            uint32_t idx;
-            float w;
-            corner(L, pos, cc, tmask, idx, w);
-            const size_t e = ((size_t)l << P.log2_table) + idx;
-            atomicAdd(T.ggrad + 2 * e, w * g0);
-            atomicAdd(T.ggrad + 2 * e + 1, w * g1);
+            const uint32_t at = atomicAdd(B.item_count, shares);
+            for (uint32_t k = 0; k < shares; k++)
+                B.items[at + k] = make_uint2(blockIdx.x * ranges + i, k * GRAD_SHARE);
         }
+    }
+}
+
+// A share of a bin: a whole bin's sums are added to the gradient by plain stores,
+// those of a bin in several shares by atomics. The LDS serves float atomics at
+// 3.6 cycles a lane: one block for the 300,000 updates that a coarse
+// level's only bin gets from a frame took 730 us.
+template <int LOG2_E>
+__global__ __launch_bounds__(GRAD_ADD_BLOCK) void k_nrc_bin_add(NrcDev P, NrcTrainDev T, GradBins B)
+{
+    constexpr uint32_t ENTRIES = 1u << LOG2_E;
+    __shared__ float4 sums4[ENTRIES / 2];
+    float* sums = reinterpret_cast<float*>(sums4);
+    if (blockIdx.x >= *B.item_count)
+        return;
+    const uint2 item = B.items[blockIdx.x];
+    const uint32_t bin = item.x; // level * ranges + range
+    const uint32_t ranges = 1u << (P.log2_table - LOG2_E);
+    const int l = (int)(bin / ranges);
+    const uint32_t count = B.counts[bin], end = min(item.y + GRAD_SHARE, count);
+    for (uint32_t i = threadIdx.x; i < ENTRIES / 2; i += GRAD_ADD_BLOCK)
+        sums4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    __syncthreads();
+    // after the scatter the cursor is the bin's end
+    const size_t first = (size_t)l * B.places + B.cursors[bin] - count;
+#pragma unroll 4
+    for (uint32_t i = item.y + threadIdx.x; i < end; i += GRAD_ADD_BLOCK)
+    {
+        const uint32_t e = B.entry[first + i];
+        const float2 v = B.value[first + i];
+        atomicAdd(&sums[2 * e], v.x);
+        atomicAdd(&sums[2 * e + 1], v.y);
+    }
+    __syncthreads();
+    float* out = T.ggrad + 2 * (((size_t)l << P.log2_table) + (size_t)(bin % ranges) * ENTRIES);
+    if (count > GRAD_SHARE)
+    {
+        for (uint32_t i = threadIdx.x; i < 2 * ENTRIES; i += GRAD_ADD_BLOCK)
+            if (sums[i] != 0.0f)
+                atomicAdd(out + i, sums[i]);
+        return;
+    }
+    float4* out4 = reinterpret_cast<float4*>(out);
+    for (uint32_t i = threadIdx.x; i < ENTRIES / 2; i += GRAD_ADD_BLOCK)
+    {
+        const float4 v = sums4[i];
+        if (v.x != 0.0f || v.y != 0.0f || v.z != 0.0f || v.w != 0.0f)
+        {
+            const float4 o = out4[i];
+            out4[i] = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
+        }
+    }
+}
+
+void grid_grad_launch(Nrc& C, const NrcDev& P, const NrcTrainDev& T, uint32_t batch, hipStream_t s)
+{
+    const int lt = P.log2_table;
+    const unsigned levels = (unsigned)P.levels;
+    if (batch < GRAD_BIN_MIN_ROWS || lt < 10)
+    {
+        hipLaunchKernelGGL(k_nrc_grid_grad, dim3((batch + 127u) / 128u, levels), dim3(128), 0, s, P, T);
+        return;
+    }
+    GradBins B{};
+    B.log2_e = lt <= 14 ? 10 : 13;
+    const uint32_t ranges = 1u << (lt - B.log2_e);
+    const uint32_t pass = std::min<uint32_t>(batch, GRAD_BIN_ROWS);
+    const size_t bins = (size_t)levels * ranges, places = (size_t)8 * pass;
+    const size_t max_items = bins + places * levels / GRAD_SHARE;
+    C.grad_bins.reserve(8 * bins + 12 * places * levels + 8 * max_items + 8);
+    B.value = C.grad_bins.as<float2>();
+    B.items = reinterpret_cast<uint2*>(B.value + places * levels);
+    B.entry = reinterpret_cast<uint32_t*>(B.items + max_items);
+    B.counts = B.entry + places * levels;
+    B.cursors = B.counts + bins;
+    B.item_count = B.cursors + bins;
+    B.places = (uint32_t)places;
+    for (uint32_t r = 0; r < batch; r += pass)
+    {
+        B.first_row = r;
+        B.rows = std::min(pass, batch - r);
+        const dim3 grid((B.rows + GRAD_BIN_BLOCK - 1) / GRAD_BIN_BLOCK, levels);
+        hipLaunchKernelGGL(k_nrc_bins_reset, dim3((unsigned)((bins + 255) / 256)), dim3(256), 0, s, B, (uint32_t)bins);
+        hipLaunchKernelGGL(k_nrc_bin<false>, grid, dim3(GRAD_BIN_BLOCK), 0, s, P, T, B);
+        hipLaunchKernelGGL(k_nrc_bin_starts, dim3(levels), dim3(256), 0, s, B, ranges);
+        hipLaunchKernelGGL(k_nrc_bin<true>, grid, dim3(GRAD_BIN_BLOCK), 0, s, P, T, B);
+        if (B.log2_e == 10)
+            hipLaunchKernelGGL(k_nrc_bin_add<10>, dim3((unsigned)max_items), dim3(GRAD_ADD_BLOCK), 0, s, P, T, B);
+        else
+            hipLaunchKernelGGL(k_nrc_bin_add<13>, dim3((unsigned)max_items), dim3(GRAD_ADD_BLOCK), 0, s, P, T, B);
     }
 }
 
@@ -765,9 +1116,7 @@ void nrc_infer(Ctx& ctx, const float* d_queries, const uint32_t* d_count, uint32
         fail(MIPT_ERR_INVALID_ARGUMENT, "radiance cache not configured: call mipt_set_radiance_cache first");
     if (n == 0)
         return;
-    // rows are padded to whole 16-row tiles (zero rows past the count)
-    const uint32_t n16 = (n + 15) & ~15u;
-    C.x0.reserve(2 * (size_t)n16 * NRC_WIDTH);
+    const EncDev E = enc_buffer(C, n);
     C.count.reserve(4);
     if (!d_count)
     {
@@ -775,10 +1124,10 @@ void nrc_infer(Ctx& ctx, const float* d_queries, const uint32_t* d_count, uint32
         d_count = C.count.as<uint32_t>();
     }
     const NrcDev P = nrc_dev(ctx);
-    encode_launch(P, d_queries, RowSel{d_count, 1u, 0u, n}, n16, 16u, C.x0.as<uint16_t>(), s);
-    const unsigned grid = (unsigned)std::min<size_t>(blocks_for((n + 15) / 16, 4), (size_t)ctx.cu_count * 4);
-    hipLaunchKernelGGL(k_nrc_forward, dim3(grid), dim3(256), 0, s, C.wt.as<uint16_t>(), C.x0.as<uint16_t>(),
-                       d_count, n, reinterpret_cast<float4*>(d_out));
+    encode_launch(P, d_queries, RowSel{d_count, 1u, 0u, n}, n, 1u, E, s);
+    const unsigned grid = (unsigned)std::min<size_t>(blocks_for((n + 63) / 64, 4), (size_t)ctx.cu_count * 3);
+    hipLaunchKernelGGL(k_nrc_forward, dim3(grid), dim3(256), 0, s, C.wt.as<uint16_t>(), E, P.levels, d_count, n,
+                       reinterpret_cast<float4*>(d_out));
     HIP_CHECK(hipGetLastError());
 }
 
@@ -791,7 +1140,10 @@ void nrc_encode(Ctx& ctx, const float* d_queries, uint32_t n, uint16_t* d_out, h
         return;
     C.count.reserve(4);
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, C.count.as<uint32_t>(), n);
-    encode_launch(nrc_dev(ctx), d_queries, RowSel{C.count.as<uint32_t>(), 1u, 0u, n}, n, 1u, d_out, s);
+    const EncDev E = enc_buffer(C, n);
+    encode_launch(nrc_dev(ctx), d_queries, RowSel{C.count.as<uint32_t>(), 1u, 0u, n}, n, 1u, E, s);
+    hipLaunchKernelGGL(k_nrc_rows, dim3(blocks_for((size_t)n * (NRC_WIDTH / 2), 256)), dim3(256), 0, s, E,
+                       (int)C.settings.grid_levels, n, reinterpret_cast<uint32_t*>(d_out));
     HIP_CHECK(hipGetLastError());
 }
 
@@ -808,7 +1160,7 @@ void nrc_gradients(Ctx& ctx, const float* d_queries, const float* d_targets, con
     if (batch == 0)
         return;
     const uint32_t stride = (batch + 31) & ~31u;
-    C.x0.reserve(2 * (size_t)stride * NRC_WIDTH);
+    const EncDev E = enc_buffer(C, stride);
     C.xcm.reserve(2 * (size_t)NRC_LAYERS * NRC_WIDTH * stride);
     C.dycm.reserve(2 * (size_t)NRC_LAYERS * NRC_WIDTH * stride);
     C.dx0.reserve(4 * (size_t)stride * NRC_GRID_MAX);
@@ -826,13 +1178,13 @@ void nrc_gradients(Ctx& ctx, const float* d_queries, const float* d_targets, con
     C.last_sel_limit = batch;
     const NrcDev P = nrc_dev(ctx);
     // encode the batch; rows past its count up to a multiple of 32 are zero
-    encode_launch(P, d_queries, sel, stride, 32u, C.x0.as<uint16_t>(), s);
+    encode_launch(P, d_queries, sel, stride, 32u, E, s);
     if (clear_loss)
         hipLaunchKernelGGL(k_nrc_zero, dim3(1), dim3(64), 0, s, C.loss.as<float>(), (size_t)1);
     NrcTrainDev T{};
     T.wt = C.wt.as<uint16_t>();
     T.wk = C.wk.as<uint16_t>();
-    T.x0 = C.x0.as<uint16_t>();
+    T.enc = E;
     T.targets = d_targets;
     T.sel = sel;
     T.batch_stride = stride;
@@ -847,8 +1199,7 @@ void nrc_gradients(Ctx& ctx, const float* d_queries, const float* d_targets, con
     hipLaunchKernelGGL(k_nrc_train_fwd_bwd, dim3(grid), dim3(256), 0, s, T);
     const uint32_t chunk = 1024;
     hipLaunchKernelGGL(k_nrc_weight_grad, dim3(blocks_for(stride, chunk), NRC_LAYERS), dim3(256), 0, s, T, chunk);
-    hipLaunchKernelGGL(k_nrc_grid_grad, dim3(NRC_XCDS * blocks_for(stride, 128)), dim3(128), 0, s, P, T,
-                       reinterpret_cast<const float4*>(d_queries));
+    grid_grad_launch(C, P, T, batch, s);
     HIP_CHECK(hipGetLastError());
 }
 
