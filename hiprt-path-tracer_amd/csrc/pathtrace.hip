@@ -251,8 +251,8 @@ __device__ __forceinline__ LiveIndex live_index(const SegList& l)
 // evaluate_ReSTIR_DI_reservoir (ReSTIR/DI/FinalShading.h:16-101) without the
 // shadow ray: returns the contribution and whether a shadow ray must decide it.
 __device__ __forceinline__ Color restir_final_shading(const PtData& d, uint32_t pix, const pt::Material& m, f3 p, f3 sn,
-                                                      f3 gn, f3 view, pt::VolumeState& vs, bool& need_shadow,
-                                                      f3& dir_out, float& dist_out)
+                                                      f3 gn, f3 view, pt::VolumeState& vs, const pt::ViewTerms& t,
+                                                      bool& need_shadow, f3& dir_out, float& dist_out)
 {
     need_shadow = false;
     const float4 ra = d.restir_out[2 * (size_t)pix], rb = d.restir_out[2 * (size_t)pix + 1];
@@ -284,7 +284,7 @@ __device__ __forceinline__ Color restir_final_shading(const PtData& d, uint32_t 
         need_shadow = true;
     pt::BsdfCtx c{view, sn, gn, dir, flags & pt::RESTIR_FLAG_LOBE_MASK, pt::REGULARIZATION_MIS, 0.0f, &vs, 0};
     float bpdf;
-    const Color f = pt::principled_eval(frame_globals(d), m, c, bpdf);
+    const Color f = pt::principled_eval(frame_globals(d), m, c, t, bpdf);
     float cosine = pt::dot(sn, dir);
     if (flags & pt::FROM_GLASS_REFRACT)
         cosine = fabsf(cosine);
@@ -328,6 +328,11 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
         vol_load(d, pix, vs);
     else
         vol_canonical_at(vs, mat_index, m.dielectric_priority);
+    // every direction of this vertex is evaluated with these; the continuation
+    // replaces the lobes by the unregularised ones
+    const pt::BsdfCtx vertex{view, sn, gn, pt::mk(0.0f, 0.0f, 0.0f), pt::NO_INFO, pt::REGULARIZATION_MIS,
+                             path_roughness, &vs, 0};
+    pt::ViewTerms t = pt::view_terms(frame_globals(d), m, vertex);
 
     if (bounce > 0 || d.enable_direct)
     {
@@ -342,7 +347,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
         bool need_shadow;
         f3 dir;
         float dist;
-        const Color contrib = restir_final_shading(d, pix, m, p, sn, gn, view, vs, need_shadow, dir, dist);
+        const Color contrib = restir_final_shading(d, pix, m, p, sn, gn, view, vs, t, need_shadow, dir, dist);
         d.nee_light[pix] = stc(contrib, 0.0f);
         flags |= FLAG_NEE_LIGHT;
         if (need_shadow)
@@ -381,7 +386,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
                 {
                     pt::BsdfCtx c{view, sn, gn, dirn, pt::NO_INFO, pt::REGULARIZATION_MIS, path_roughness, &vs, 0};
                     float bsdf_pdf = 0.0f;
-                    f = pt::principled_eval(frame_globals(d), m, c, bsdf_pdf);
+                    f = pt::principled_eval(frame_globals(d), m, c, t, bsdf_pdf);
                     target = pt::luminance(f * ls.emission * cos_p);
                     const float spdf =
                         cos_at_light < 1.0e-8f ? 0.0f : ls.area_pdf * (dist * dist) / cos_at_light;
@@ -407,7 +412,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
                           &vs, 0};
             f3 dir;
             float bpdf;
-            const Color f = pt::principled_sample(frame_globals(d), m, c, dir, bpdf, rng);
+            const Color f = pt::principled_sample(frame_globals(d), m, c, t, dir, bpdf, rng);
             if (bpdf > 0.0f)
             {
                 d.nee_bsdf[pix] = stc(f, bpdf);
@@ -443,7 +448,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
                 pt::VolumeState vs_light = vs;
                 pt::BsdfCtx c{view, sn, gn, dirn, pt::NO_INFO, pt::REGULARIZATION_MIS, path_roughness, &vs_light, 0};
                 float bsdf_pdf;
-                const Color f = pt::principled_eval(frame_globals(d), m, c, bsdf_pdf);
+                const Color f = pt::principled_eval(frame_globals(d), m, c, t, bsdf_pdf);
                 if (vs_light.distance != vs.distance)
                 {
                     light_floor = true;
@@ -472,7 +477,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
                       0};
         f3 dir;
         float bpdf;
-        const Color f = pt::principled_sample(frame_globals(d), m, c, dir, bpdf, rng);
+        const Color f = pt::principled_sample(frame_globals(d), m, c, t, dir, bpdf, rng);
         if (bpdf > 0.0f)
         {
             const float cosine = fabsf(pt::dot(sn, dir));
@@ -501,7 +506,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
             pt::VolumeState vs_env = vs;
             pt::BsdfCtx c{view, sn, gn, edir, pt::NO_INFO, pt::REGULARIZATION_MIS, path_roughness, &vs_env, 0};
             float bsdf_pdf;
-            const Color f = pt::principled_eval(frame_globals(d), m, c, bsdf_pdf);
+            const Color f = pt::principled_eval(frame_globals(d), m, c, t, bsdf_pdf);
             const float w = balance_heuristic(epdf, 1.0f, bsdf_pdf, 1.0f);
             env_light = f * ecos * w * ecol / epdf / 1.0f;
             env_floor = vs_env.distance != vs.distance;
@@ -514,7 +519,7 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
                       0};
         f3 bdir;
         float bpdf;
-        const Color f = pt::principled_sample(frame_globals(d), m, c, bdir, bpdf, rng);
+        const Color f = pt::principled_sample(frame_globals(d), m, c, t, bdir, bpdf, rng);
         const float bcos = fabsf(pt::dot(sn, bdir));
         if (bpdf > 0.0f)
         {
@@ -538,9 +543,11 @@ __device__ __forceinline__ void shade_vertex(const PtData& d, int32_t bounce, ui
     {
         pt::BsdfCtx c{view, sn, gn, pt::mk(0.0f, 0.0f, 0.0f), pt::NO_INFO, pt::NO_REGULARIZATION, path_roughness, &vs,
                       1};
+        if (frame_globals(d).regularize)
+            pt::view_lobes(frame_globals(d), m, c, t);
         f3 dir;
         float bpdf;
-        const Color f = pt::principled_sample(frame_globals(d), m, c, dir, bpdf, rng);
+        const Color f = pt::principled_sample(frame_globals(d), m, c, t, dir, bpdf, rng);
         // RayPayload::accumulate_roughness (RayPayload.h:52-89)
         if (c.info == pt::FROM_DIFFUSE || c.info == pt::FROM_DIFFUSE_TRANSMISSION)
             path_roughness = 1.0f;

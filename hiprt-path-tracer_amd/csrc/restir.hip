@@ -264,13 +264,24 @@ __device__ __forceinline__ f3 sample_direction(const PtData& d, f3 p, f3 point, 
     return pt::vdiv(to, dist);
 }
 
+// The view terms of a surface's evaluations. A surface without a material
+// (a miss of the previous frame) has none and is not evaluated either.
+__device__ __forceinline__ pt::ViewTerms surface_terms(const PtData& d, const Surface& s)
+{
+    pt::VolumeState vs = surface_volume(d, s);
+    const pt::BsdfCtx c{s.view, s.sn, s.gn, pt::mk(0.0f, 0.0f, 0.0f), pt::NO_INFO, pt::NO_REGULARIZATION, 0.0f, &vs, 0};
+    return pt::view_terms(d.g, d.mats[s.mat], c);
+}
+
 // ReSTIR_DI_evaluate_target_function<false> (DI/TargetFunction.h:49-98): the
 // luminance of f * Le * cos * G (G = 1 for an envmap sample, whose Le is the
 // envmap's radiance in that direction). The visibility factor, when wanted,
 // is applied by the caller from a shadow ray (origin s.p, direction dir_out,
 // tmax dist_out - 1e-4), traced only when the value is non-zero.
-__device__ __forceinline__ float target_function(const PtData& d, const Surface& s, f3 point, int32_t tri, uint32_t flags,
-                                                 f3& dir_out, float& dist_out)
+// `terms()` gives the surface's view terms, once the evaluation needs them.
+template <typename Terms>
+__device__ __forceinline__ float target_function(const PtData& d, const Surface& s, const Terms& terms, f3 point,
+                                                 int32_t tri, uint32_t flags, f3& dir_out, float& dist_out)
 {
     dist_out = 0.0f;
     const bool env = (flags & pt::RESTIR_FLAG_ENVMAP) != 0u;
@@ -287,7 +298,7 @@ __device__ __forceinline__ float target_function(const PtData& d, const Surface&
     pt::VolumeState vs = surface_volume(d, s);
     pt::BsdfCtx c{s.view, s.sn, s.gn, dir, flags & pt::RESTIR_FLAG_LOBE_MASK, pt::NO_REGULARIZATION, 0.0f, &vs, 0};
     float bpdf;
-    const Color f = pt::principled_eval(d.g, m, c, bpdf);
+    const Color f = pt::principled_eval(d.g, m, c, terms(), bpdf);
     Color emission;
     float geometry = 1.0f;
     if (env)
@@ -302,6 +313,13 @@ __device__ __forceinline__ float target_function(const PtData& d, const Surface&
         geometry /= dist * dist;
     }
     return luminance(((f * emission) * cosine) * geometry);
+}
+
+// For one evaluation of a surface.
+__device__ __forceinline__ float target_function(const PtData& d, const Surface& s, f3 point, int32_t tri, uint32_t flags,
+                                                 f3& dir_out, float& dist_out)
+{
+    return target_function(d, s, [&] { return surface_terms(d, s); }, point, tri, flags, dir_out, dist_out);
 }
 
 // The probability that a light candidate samples the envmap rather than an
@@ -393,8 +411,8 @@ __global__ void k_presample_lights(PtData d, float env_prob, float4* __restrict_
 // Samples BSDF candidates from index `cand` on until one needs a ray
 // (returns true, ray written to slot 0) or none is left (false).
 __device__ __forceinline__ bool next_bsdf_candidate(const PtData& d, const RsData& r, uint32_t pix, const Surface& s,
-                                                    const pt::Material& m, int32_t& cand, pt::Xorshift32& rng,
-                                                    float& bpdf_out, uint32_t& info_out)
+                                                    const pt::Material& m, const pt::ViewTerms& t, int32_t& cand,
+                                                    pt::Xorshift32& rng, float& bpdf_out, uint32_t& info_out)
 {
     const int32_t nb = r.s.number_of_initial_bsdf_candidates;
     while (cand < nb)
@@ -403,7 +421,7 @@ __device__ __forceinline__ bool next_bsdf_candidate(const PtData& d, const RsDat
         pt::BsdfCtx c{s.view, s.sn, s.gn, pt::mk(0.0f, 0.0f, 0.0f), pt::NO_INFO, pt::NO_REGULARIZATION, 0.0f, &vs, 0};
         f3 dir;
         float bpdf;
-        pt::principled_sample(d.g, m, c, dir, bpdf, rng);
+        pt::principled_sample(d.g, m, c, t, dir, bpdf, rng);
         if (bpdf > 0.0f)
         {
             write_ray(r.rays, pix, s.p, s.prim, dir, 1.0e35f - 1.0e-4f);
@@ -435,6 +453,9 @@ __device__ __forceinline__ void finish_initial(const PtData& d, const RsData& r,
     need_vis = 1u;
 }
 
+// Bound by instruction issue (81 % busy): about 1500 instructions of a wave a
+// light candidate when every evaluation builds its view terms, 3.28 ms for 32
+// candidates at 1080p; with the terms built once, 2.45 ms.
 __global__ __launch_bounds__(256, 2) void k_ic_start(PtData d, RsData r)
 {
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
@@ -450,6 +471,7 @@ __global__ __launch_bounds__(256, 2) void k_ic_start(PtData d, RsData r)
     }
     const Surface s = surface_current(d, pix);
     const pt::Material& m = d.mats[s.mat];
+    const pt::ViewTerms t = surface_terms(d, s);
     Res res = res_empty();
     const int32_t nl = r.s.number_of_initial_light_candidates;
     const int32_t nb = r.s.number_of_initial_bsdf_candidates;
@@ -525,7 +547,7 @@ __global__ __launch_bounds__(256, 2) void k_ic_start(PtData d, RsData r)
             pt::VolumeState vs = surface_volume(d, s);
             pt::BsdfCtx c{s.view, s.sn, s.gn, dir, pt::NO_INFO, pt::NO_REGULARIZATION, 0.0f, &vs, 0};
             float bsdf_pdf;
-            const Color f = pt::principled_eval(d.g, m, c, bsdf_pdf);
+            const Color f = pt::principled_eval(d.g, m, c, t, bsdf_pdf);
             // ReSTIR_DI_evaluate_target_function<false> of this light sample:
             // its BSDF evaluation has the same arguments as the one above (the
             // direction is recomputed from the same point by the same
@@ -564,7 +586,7 @@ __global__ __launch_bounds__(256, 2) void k_ic_start(PtData d, RsData r)
     int32_t cand = 0;
     float bpdf = 0.0f;
     uint32_t info = 0u;
-    if (next_bsdf_candidate(d, r, pix, s, m, cand, rng, bpdf, info))
+    if (next_bsdf_candidate(d, r, pix, s, m, t, cand, rng, bpdf, info))
     {
         write_inactive(r.rays, (size_t)r.n + pix);
         state_store(r, pix, res, rng.state, PHASE_PENDING, bpdf, __int_as_float(cand), info);
@@ -576,7 +598,10 @@ __global__ __launch_bounds__(256, 2) void k_ic_start(PtData d, RsData r)
 }
 
 // sample_bsdf_candidates (InitialCandidates.h:300-440) after the closest hit.
-__global__ __launch_bounds__(256, 2) void k_ic_bsdf(PtData d, RsData r)
+// Most pixels leave early, the rest wait on gathers: three waves a SIMD take
+// 159 us for 185 with two (1/3 of 1080p, envmap), four 152 but 285 for 218 where
+// every candidate hits geometry.
+__global__ __launch_bounds__(256, 3) void k_ic_bsdf(PtData d, RsData r)
 {
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
     if (pix >= r.n)
@@ -652,7 +677,7 @@ __global__ __launch_bounds__(256, 2) void k_ic_bsdf(PtData d, RsData r)
         }
     }
     cand++;
-    if (next_bsdf_candidate(d, r, pix, s, m, cand, rng, bpdf, info))
+    if (cand < nb && next_bsdf_candidate(d, r, pix, s, m, surface_terms(d, s), cand, rng, bpdf, info))
     {
         state_store(r, pix, res, rng.state, PHASE_PENDING, bpdf, __int_as_float(cand), info);
         return;
@@ -718,7 +743,7 @@ __device__ __forceinline__ int32_t pixel_coord(float v) { return (v > -1.0e9f &&
 // random pixels within neighbor_search_radius (x offset drawn first), the
 // first that passes the similarity heuristics against the previous G-buffer;
 // index -1 without one. (x, y) is the rounded reprojected pixel.
-__device__ int3 temporal_neighbor(const PtData& d, const RsData& r, uint32_t pix, f3 cnormal, pt::Xorshift32& rng)
+__device__ __forceinline__ int3 temporal_neighbor(const PtData& d, const RsData& r, uint32_t pix, f3 cnormal, pt::Xorshift32& rng)
 {
     const int32_t W = d.width, H = d.height;
     if (r.accumulate)
@@ -783,7 +808,7 @@ __device__ __forceinline__ void state_store_neighbor(const RsData& r, uint32_t p
     r.state[4 * (size_t)pix + 3].z = __int_as_float(neighbor);
 }
 
-__global__ void k_tp_start(PtData d, RsData r)
+__global__ __launch_bounds__(256, 2) void k_tp_start(PtData d, RsData r)
 {
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
     if (pix >= r.n)
@@ -937,7 +962,10 @@ __device__ __forceinline__ bool similar(const PtData& d, const RsData& r, int32_
     return plane && normal;
 }
 
-__global__ __launch_bounds__(256, 2) void k_sp_start(PtData d, RsData r)
+// Neighbour surfaces and reservoirs are gathers at random pixels and instruction
+// issue is only 60 % busy: three waves a SIMD instead of two take 1.23 ms for
+// 1.38 (1080p, five neighbours), four, which spill, 1.58.
+__global__ __launch_bounds__(256, 3) void k_sp_start(PtData d, RsData r)
 {
     const uint32_t pix = blockIdx.x * blockDim.x + threadIdx.x;
     if (pix >= r.n)
@@ -988,9 +1016,40 @@ __global__ __launch_bounds__(256, 2) void k_sp_start(PtData d, RsData r)
         aux[2 * i] = 0.0f;
         aux[2 * i + 1] = -1.0f;
     }
+    const int32_t start = valid_M == 0 ? K : 0;
+    // The centre's sample at every neighbour's surface, then every neighbour's
+    // sample at the centre. Two loops: one that holds the centre's view terms
+    // across a neighbour's evaluation spills 96 registers (1.66 ms a pass of
+    // five neighbours at 1080p, for 1.23 in two).
+    if (update_mc)
+    {
+        pt::Xorshift32 nrng{nseed};
+        for (int32_t i = start; i < K; i++)
+        {
+            if (!(cache & (1u << i)))
+            {
+                nrng.next();
+                nrng.next();
+                continue;
+            }
+            const int32_t np = spatial_neighbor(d, r, cx, cy, nrng);
+            if (np == -1)
+                continue;
+            const float res_M = cw ? (float)__float_as_int(r.in[2 * (size_t)np + 1].x) : 1.0f;
+            const Surface ns = surface_current(d, (uint32_t)np);
+            f3 dir;
+            float dist;
+            const float tf_csn = target_function(d, ns, center.point, center.tri, center.flags, dir, dist);
+            const float conf_mult = cw ? (conf_sum == 0.0f ? 0.0f : res_M / conf_sum) : 1.0f;
+            aux[2 * i] = tf_csn;
+            aux[2 * i + 1] = conf_mult;
+            if (tf_csn != 0.0f)
+                write_ray(r.rays, (size_t)i * r.n + pix, ns.p, ns.prim, dir, dist - 1.0e-4f);
+        }
+    }
+    const pt::ViewTerms ct = surface_terms(d, cs);
     Res out = res_empty();
     pt::Xorshift32 nrng{nseed};
-    const int32_t start = valid_M == 0 ? K : 0;
     for (int32_t i = start; i < K; i++)
     {
         if (!(cache & (1u << i)))
@@ -1008,25 +1067,13 @@ __global__ __launch_bounds__(256, 2) void k_sp_start(PtData d, RsData r)
         {
             f3 dir;
             float dist;
-            tf_center = target_function(d, cs, nres.point, nres.tri, nres.flags, dir, dist);
+            tf_center = target_function(d, cs, [&]() -> const pt::ViewTerms& { return ct; }, nres.point, nres.tri, nres.flags, dir, dist);
         }
         // ReSTIRSpatialResamplingMISWeight<PAIRWISE_MIS> (SpatialMISWeight.h:118-234), neighbour
         const float res_M = cw ? (float)nres.M : 1.0f;
         const float nume = nres.target * res_M;
         const float denom = nres.target * conf_sum + tf_center / vdt * center_M;
         const float mi = denom == 0.0f ? 0.0f : nume / denom;
-        if (update_mc)
-        {
-            const Surface ns = surface_current(d, (uint32_t)np);
-            f3 dir;
-            float dist;
-            const float tf_csn = target_function(d, ns, center.point, center.tri, center.flags, dir, dist);
-            const float conf_mult = cw ? (conf_sum == 0.0f ? 0.0f : res_M / conf_sum) : 1.0f;
-            aux[2 * i] = tf_csn;
-            aux[2 * i + 1] = conf_mult;
-            if (tf_csn != 0.0f)
-                write_ray(r.rays, (size_t)i * r.n + pix, ns.p, ns.prim, dir, dist - 1.0e-4f);
-        }
         if (combine_with(out, nres, mi / vdt, tf_center, 1.0f, rng))
             out.flags &= ~pt::RESTIR_FLAG_UNOCCLUDED;
     }
@@ -1318,6 +1365,7 @@ __global__ __launch_bounds__(256, 2) void k_fst_combine(PtData d, RsData r)
         if (combine_with(out, tn, mi / vdt, tf_center, 1.0f, rng))
             out.flags |= pt::RESTIR_FLAG_UNOCCLUDED;
     }
+    const pt::ViewTerms ct = surface_terms(d, cs);
     pt::Xorshift32 nrng{nseed};
     const int32_t start = valid_M == 0 ? K : 0;
     for (int32_t i = start; i < K + 1; i++)
@@ -1341,7 +1389,7 @@ __global__ __launch_bounds__(256, 2) void k_fst_combine(PtData d, RsData r)
             {
                 f3 dir;
                 float dist;
-                tf_center = target_function(d, cs, nres.point, nres.tri, nres.flags, dir, dist);
+                tf_center = target_function(d, cs, [&]() -> const pt::ViewTerms& { return ct; }, nres.point, nres.tri, nres.flags, dir, dist);
             }
         }
         float w;

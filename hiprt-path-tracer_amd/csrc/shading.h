@@ -277,25 +277,37 @@ PT_HD float lut_fetch(const float* lut, int n, float u, float v)
 }
 
 // MicrofacetEnergyCompensation.h:27-45; thresholds of BSDFsData.h (0, -1).
-PT_HD Color ggx_energy_compensation_conductor(const BsdfGlobals& g, Color F0, float roughness, bool do_ec, f3 lv)
+PT_HD bool conductor_compensated(float roughness, bool do_ec, float NoV)
 {
-    bool smooth_enough = roughness <= 0.0f;
-    bool invalid = lv.z < 0.0f;
-    if (!do_ec || smooth_enough || invalid)
-        return col(1.0f);
-    float u = maxf_(0.0f, lv.z);
+    return do_ec && !(roughness <= 0.0f) && !(NoV < 0.0f);
+}
+PT_HD float conductor_kms(const BsdfGlobals& g, float roughness, float NoV)
+{
+    float u = maxf_(0.0f, NoV);
     float v = 1.0f - roughness;
     float ess = lut_fetch(g.ggx_conductor_ess, g.lut_size, u, v);
-    float kms = (1.0f - ess) / ess;
-    return col(1.0f) + kms * F0;
+    return (1.0f - ess) / ess;
+}
+
+// What a reflection lobe needs that depends on the roughness and the view alone.
+struct LobeView {
+    float roughness, ax, ay, G1V;
+};
+
+PT_HD LobeView lobe_view(float roughness, float anisotropy, f3 lv)
+{
+    LobeView l;
+    l.roughness = roughness;
+    get_alphas(roughness, anisotropy, l.ax, l.ay);
+    l.G1V = 1.0f / (1.0f + smith_lambda(l.ax, l.ay, lv));
+    return l;
 }
 
 // Microfacet.h:103-178 (single scattering, height-uncorrelated Smith G2).
-PT_HD Color ggx_eval_reflect_ss(float roughness, float anisotropy, Color F, f3 lv, f3 ll, f3 lh, float& pdf,
-                                DeltaSampled delta)
+PT_HD Color ggx_eval_reflect_ss(const LobeView& l, Color F, f3 lv, f3 ll, f3 lh, float& pdf, DeltaSampled delta)
 {
     pdf = 0.0f;
-    if (is_perfectly_smooth(roughness))
+    if (is_perfectly_smooth(l.roughness))
     {
         if (delta == SPECULAR_PEAK_NOT_SAMPLED)
             return col(0.0f);
@@ -309,43 +321,17 @@ PT_HD Color ggx_eval_reflect_ss(float roughness, float anisotropy, Color F, f3 l
     }
     if (ll.z < 0.0f)
         return col(0.0f);
-    float ax, ay;
-    get_alphas(roughness, anisotropy, ax, ay);
-    float D = ggx_d(ax, ay, lh);
-    float lambda_v = smith_lambda(ax, ay, lv);
-    float G1V = 1.0f / (1.0f + lambda_v);
-    float Dvis = ggx_vndf(D, G1V, lv, lh);
+    float D = ggx_d(l.ax, l.ay, lh);
+    float Dvis = ggx_vndf(D, l.G1V, lv, lh);
     float NoV = maxf_(GGX_DOT_CLAMP, fabsf(lv.z));
     float NoL = maxf_(GGX_DOT_CLAMP, fabsf(ll.z));
     pdf = Dvis / (4.0f * dot(lv, lh));
     if (pdf == 0.0f)
         return col(0.0f);
-    float lambda_l = smith_lambda(ax, ay, ll);
+    float lambda_l = smith_lambda(l.ax, l.ay, ll);
     float G1L = 1.0f / (1.0f + lambda_l);
-    float G2 = G1V * G1L;
+    float G2 = l.G1V * G1L;
     return F * D * G2 / (4.0f * NoL * NoV);
-}
-
-// Microfacet.h:227-287
-PT_HD float ggx_pdf_reflect(float roughness, float anisotropy, f3 lv, f3 ll, f3 lh, DeltaSampled delta)
-{
-    if (is_perfectly_smooth(roughness))
-    {
-        if (delta == SPECULAR_PEAK_NOT_SAMPLED)
-            return 0.0f;
-        if (dot(reflect_ray(lv, mk(0.0f, 0.0f, 1.0f)), ll) < DELTA_ALIGN_THRESHOLD)
-            return 0.0f;
-        return DELTA_HIGH_VALUE;
-    }
-    if (ll.z < 0.0f)
-        return 0.0f;
-    float ax, ay;
-    get_alphas(roughness, anisotropy, ax, ay);
-    float D = ggx_d(ax, ay, lh);
-    float lambda_v = smith_lambda(ax, ay, lv);
-    float G1V = 1.0f / (1.0f + lambda_v);
-    float Dvis = ggx_vndf(D, G1V, lv, lh);
-    return Dvis / (4.0f * dot(lv, lh));
 }
 
 // Heitz 2018 VNDF sampling (Microfacet.h:398-424).
@@ -389,16 +375,19 @@ PT_HD float pow6(float x)
 }
 
 // Fresnel.h:138-168 (Adobe F82-tint).
-PT_HD Color f82_tint_fresnel(Color F0, Color F82, Color F90, float falloff, float cos_theta)
+PT_HD Color f82_tint_scale(Color F0, Color F82, Color F90, float falloff)
+{
+    const float cos_theta_max = 1.0f / 7.0f;
+    const float denom_a = cos_theta_max * pow6(1.0f - cos_theta_max);
+    Color nume_a = (F0 + (F90 - F0) * pow_fixed(1.0f - cos_theta_max, falloff)) * (col(1.0f) - F82);
+    return nume_a / denom_a;
+}
+PT_HD Color f82_tint_fresnel(Color F0, Color F90, float falloff, Color a, float cos_theta)
 {
     Color base = F0 + (F90 - F0) * pow_fixed(1.0f - cos_theta, falloff);
     if (max_component(base) < 1.0e-8f)
         return col(0.0f);
     float lazanyi = cos_theta * pow6(1.0f - cos_theta);
-    const float cos_theta_max = 1.0f / 7.0f;
-    const float denom_a = cos_theta_max * pow6(1.0f - cos_theta_max);
-    Color nume_a = (F0 + (F90 - F0) * pow_fixed(1.0f - cos_theta_max, falloff)) * (col(1.0f) - F82);
-    Color a = nume_a / denom_a;
     Color F = base - a * lazanyi;
     return col(clampf_(0.0f, 1.0f, F.r), clampf_(0.0f, 1.0f, F.g), clampf_(0.0f, 1.0f, F.b));
 }
@@ -418,32 +407,23 @@ struct BsdfCtx {
 // Principled.h:125-153
 PT_HD Color thin_film_fresnel(const Material& m, float ambient_ior, float HoL);
 
-PT_HD Color metallic_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, float roughness, float anisotropy,
+PT_HD Color metallic_eval(const Material& m, const BsdfCtx& c, const LobeView& l, float kms, Color f82_a,
                           float incident_ior, f3 lv, f3 ll, f3 lh, float& pdf)
 {
-    float rr = regularize_reflection(g, c.reg, roughness, c.path_roughness);
-    DeltaSampled ds = delta_reflection_sampled(m, rr, anisotropy, c.info);
+    DeltaSampled ds = delta_reflection_sampled(m, l.roughness, m.anisotropy, c.info);
     if (ds == SPECULAR_PEAK_NOT_SAMPLED)
     {
         pdf = 0.0f;
         return col(0.0f);
     }
     float HoL = clampf_(1.0e-8f, 1.0f, dot(lh, ll));
-    Color F_metal = f82_tint_fresnel(m.base_color, m.metallic_F82, m.metallic_F90, m.metallic_F90_falloff_exponent, HoL);
+    Color F_metal = f82_tint_fresnel(m.base_color, m.metallic_F90, m.metallic_F90_falloff_exponent, f82_a, HoL);
     Color F = lerpc(F_metal, thin_film_fresnel(m, incident_ior, HoL), m.thin_film);
-    Color ms = ggx_energy_compensation_conductor(g, F, rr, (m.flags & MAT_METALLIC_EC) != 0, lv);
-    Color ss = ggx_eval_reflect_ss(rr, anisotropy, F, lv, ll, lh, pdf, ds);
+    Color ms = col(1.0f);
+    if (conductor_compensated(l.roughness, (m.flags & MAT_METALLIC_EC) != 0, lv.z))
+        ms = col(1.0f) + kms * F;
+    Color ss = ggx_eval_reflect_ss(l, F, lv, ll, lh, pdf, ds);
     return ss * ms;
-}
-
-PT_HD float metallic_pdf(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, float roughness, float anisotropy,
-                         f3 lv, f3 ll, f3 lh)
-{
-    float rr = regularize_reflection(g, c.reg, roughness, c.path_roughness);
-    DeltaSampled ds = delta_reflection_sampled(m, rr, anisotropy, c.info);
-    if (ds == SPECULAR_PEAK_NOT_SAMPLED)
-        return 0.0f;
-    return ggx_pdf_reflect(rr, anisotropy, lv, ll, lh, ds);
 }
 
 // ---------------------------------------------------------------------------
@@ -723,24 +703,16 @@ PT_HD float energy_compensation_clearcoat(const BsdfGlobals& g, const Material& 
 }
 
 // Principled.h:292-313
-PT_HD Color specular_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, float relative_ior, f3 lv, f3 ll,
+PT_HD Color specular_eval(const Material& m, const BsdfCtx& c, const LobeView& l, float relative_ior, f3 lv, f3 ll,
                           f3 lh, float& pdf)
 {
-    float rr = regularize_reflection(g, c.reg, m.roughness, c.path_roughness);
-    DeltaSampled ds = delta_reflection_sampled(m, rr, m.anisotropy, c.info);
+    DeltaSampled ds = delta_reflection_sampled(m, l.roughness, m.anisotropy, c.info);
     Color F = specular_fresnel(m, relative_ior, dot(ll, lh));
-    return ggx_eval_reflect_ss(rr, m.anisotropy, F, lv, ll, lh, pdf, ds);
-}
-
-PT_HD float specular_pdf(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, f3 lv, f3 ll, f3 lh)
-{
-    float rr = regularize_reflection(g, c.reg, m.roughness, c.path_roughness);
-    DeltaSampled ds = delta_reflection_sampled(m, rr, m.anisotropy, c.info);
-    return ggx_pdf_reflect(rr, m.anisotropy, lv, ll, lh, ds);
+    return ggx_eval_reflect_ss(l, F, lv, ll, lh, pdf, ds);
 }
 
 // Principled.h:1272-1303 (OpenPBR's TIR darkening with a diffuse base).
-PT_HD Color specular_darkening(const Material& m, float relative_eta, float view_dir_fresnel)
+PT_HD Color specular_darkening(const Material& m, float relative_eta)
 {
     if (m.specular_darkening == 0.0f)
         return col(1.0f);
@@ -755,21 +727,13 @@ PT_HD Color specular_darkening(const Material& m, float relative_eta, float view
 // Coat layer
 // ---------------------------------------------------------------------------
 // Principled.h:49-73
-PT_HD Color coat_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, f3 lv, f3 ll, f3 lh,
+PT_HD Color coat_eval(const Material& m, const BsdfCtx& c, const LobeView& l, f3 lv, f3 ll, f3 lh,
                       float incident_medium_ior, float& pdf)
 {
     float HoL = clampf_(1.0e-8f, 1.0f, dot(lh, ll));
-    float rr = regularize_reflection(g, c.reg, m.coat_roughness, c.path_roughness);
-    DeltaSampled ds = delta_reflection_sampled(m, rr, m.coat_anisotropy, c.info);
+    DeltaSampled ds = delta_reflection_sampled(m, l.roughness, m.coat_anisotropy, c.info);
     Color F = col(fresnel_dielectric(HoL, incident_medium_ior, m.coat_ior));
-    return ggx_eval_reflect_ss(rr, m.coat_anisotropy, F, lv, ll, lh, pdf, ds);
-}
-
-PT_HD float coat_pdf(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, f3 lv, f3 ll, f3 lh)
-{
-    float rr = regularize_reflection(g, c.reg, m.coat_roughness, c.path_roughness);
-    DeltaSampled ds = delta_reflection_sampled(m, rr, m.coat_anisotropy, c.info);
-    return ggx_pdf_reflect(rr, m.coat_anisotropy, lv, ll, lh, ds);
+    return ggx_eval_reflect_ss(l, F, lv, ll, lh, pdf, ds);
 }
 
 // Principled.h:890-950 (OpenPBR coat darkening).
@@ -826,40 +790,41 @@ PT_HD float get_phi(f3 d)
     return p;
 }
 
-// SheenLTC.h:75-81: rotation of vec by angle around axis (Rodrigues).
-PT_HD f3 rotate_vector(f3 vec, f3 axis, float angle)
+// SheenLTC.h:75-81: rotation of vec around axis (Rodrigues) by the angle of
+// sine s and cosine co.
+PT_HD f3 rotate_vector(f3 vec, f3 axis, float s, float co)
 {
-    float s, co;
-    sincos_fixed(angle, s, co);
     return (vmul(vec, co) + vmul(vmul(axis, dot(vec, axis)), 1.0f - co)) + vmul(cross(axis, vec), s);
 }
 
+// The sheen's fit and the rotation that takes the view's azimuth to 0.
+struct SheenView {
+    Color AiBiRi;
+    float s, co;
+};
+
+PT_HD SheenView sheen_view(const BsdfGlobals& g, const Material& m, f3 lv)
+{
+    SheenView v;
+    v.AiBiRi = sheen_ltc_params(g, m.sheen_roughness, lv.z);
+    sincos_fixed(-get_phi(lv), v.s, v.co);
+    return v;
+}
+
 // SheenLTC.h:88-125; lv, ll in the (unrotated) local shading frame.
-PT_HD Color sheen_eval(const BsdfGlobals& g, const Material& m, f3 lv, f3 ll, float& pdf, float& reflectance)
+PT_HD Color sheen_eval(const Material& m, const SheenView& v, f3 lv, f3 ll, float& pdf, float& reflectance)
 {
     if (lv.z <= 0.0f || ll.z <= 0.0f)
     {
         pdf = 0.0f;
-        reflectance = lv.z > 0.0f ? sheen_ltc_params(g, m.sheen_roughness, lv.z).b : 0.0f;
+        reflectance = lv.z > 0.0f ? v.AiBiRi.b : 0.0f;
         return col(0.0f);
     }
-    float phi = get_phi(lv);
-    f3 l_std = rotate_vector(ll, mk(0.0f, 0.0f, 1.0f), -phi);
-    Color AiBiRi = sheen_ltc_params(g, m.sheen_roughness, lv.z);
-    float Do = eval_ltc(l_std, AiBiRi);
+    f3 l_std = rotate_vector(ll, mk(0.0f, 0.0f, 1.0f), v.s, v.co);
+    float Do = eval_ltc(l_std, v.AiBiRi);
     pdf = Do;
-    reflectance = AiBiRi.b;
-    return m.sheen_color * AiBiRi.b * Do / ll.z;
-}
-
-PT_HD float sheen_pdf(const BsdfGlobals& g, const Material& m, f3 lv, f3 ll)
-{
-    if (lv.z <= 0.0f || ll.z <= 0.0f)
-        return 0.0f;
-    float phi = get_phi(lv);
-    f3 l_std = rotate_vector(ll, mk(0.0f, 0.0f, 1.0f), -phi);
-    Color AiBiRi = sheen_ltc_params(g, m.sheen_roughness, lv.z);
-    return eval_ltc(l_std, AiBiRi);
+    reflectance = v.AiBiRi.b;
+    return m.sheen_color * v.AiBiRi.b * Do / ll.z;
 }
 
 // Sampling.h:210-220
@@ -883,7 +848,9 @@ PT_HD f3 sheen_sample(const BsdfGlobals& g, const Material& m, f3 lv, Xorshift32
     float Ai_inv = 1.0f / AiBiRi.r;
     float Bi = AiBiRi.g;
     f3 d = normalize(mk(cs.x * Ai_inv - cs.z * Bi * Ai_inv, cs.y * Ai_inv, cs.z));
-    return rotate_vector(d, mk(0.0f, 0.0f, 1.0f), get_phi(lv));
+    float s, co;
+    sincos_fixed(get_phi(lv), s, co);
+    return rotate_vector(d, mk(0.0f, 0.0f, 1.0f), s, co);
 }
 
 // ---------------------------------------------------------------------------
@@ -1101,26 +1068,6 @@ PT_HD Color ggx_eval_refract(const Material& m, float roughness, float relative_
     return color;
 }
 
-PT_HD float ggx_pdf_refract(const Material& m, float roughness, float relative_eta, f3 lv, f3 ll, f3 lh, uint32_t info)
-{
-    float NoV = lv.z;
-    float HoL = dot(ll, lh), HoV = dot(lv, lh);
-    if (is_perfectly_smooth(roughness))
-    {
-        bool perfect = dot(refract_ray(lv, mk(0.0f, 0.0f, 1.0f), relative_eta), ll) > DELTA_ALIGN_THRESHOLD;
-        return info == FROM_GLASS_REFRACT && perfect ? DELTA_HIGH_VALUE : 0.0f;
-    }
-    float dot_prod = HoL + HoV / relative_eta;
-    float dot_prod2 = dot_prod * dot_prod;
-    float ax, ay;
-    get_alphas(roughness, m.anisotropy, ax, ay);
-    float D = ggx_d(ax, ay, lh);
-    float G1_V = 1.0f / (1.0f + smith_lambda(ax, ay, lv));
-    float dwm_dwi = fabsf(HoL) / dot_prod2;
-    float D_pdf = G1_V / fabsf(NoV) * D * fabsf(HoV);
-    return dwm_dwi * D_pdf;
-}
-
 // IORs on both sides of the interface (Principled.h:374-380): the materials
 // of the incident / outgoing media (1 for the air) at the sampled wavelength.
 PT_HD float medium_ior(const BsdfGlobals& g, int32_t medium)
@@ -1210,7 +1157,7 @@ PT_HD Color glass_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c
         else if (g.regularize && c.reg == REGULARIZATION_CLASSIC)
             rr = regularize_reflection(g, c.reg, scaled, c.path_roughness);
         DeltaSampled ds = delta_reflection_sampled(m, scaled, m.anisotropy, c.info);
-        color = ggx_eval_reflect_ss(rr, m.anisotropy, F, lv, ll, lh, pdf, ds);
+        color = ggx_eval_reflect_ss(lobe_view(rr, m.anisotropy, lv), F, lv, ll, lh, pdf, ds);
         float compensation = glass_energy_compensation(g, m, m.roughness, v.inside != 0, eta_t, eta_i, relative_eta,
                                                        lv.z);
         color = color / compensation;
@@ -1244,49 +1191,6 @@ PT_HD Color glass_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c
         }
     }
     return color;
-}
-
-// principled_glass_pdf (Principled.h:560-724)
-PT_HD float glass_pdf(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, f3 lv, f3 ll)
-{
-    float NoV = lv.z, NoL = ll.z;
-    if (fabsf(NoL) < 1.0e-8f)
-        return 0.0f;
-    bool reflecting = NoL * NoV > 0.0f;
-    const VolumeState& v = *c.vs;
-    float eta_i, eta_t, relative_eta;
-    glass_etas(g, m, v, eta_i, eta_t, relative_eta);
-    const bool thin = (m.flags & MAT_THIN_WALLED) != 0;
-    float scaled = thin_walled_roughness(thin, m.roughness, relative_eta);
-    f3 lh = glass_half_vector(g, reflecting, thin, scaled, relative_eta, lv, ll);
-    float HoL = dot(ll, lh), HoV = dot(lv, lh);
-    if (HoL * NoL < 0.0f || HoV * NoV < 0.0f)
-        return 0.0f;
-    float reflect_proba;
-    glass_fresnel(m, thin, scaled, eta_i, relative_eta, HoV, reflect_proba);
-    float pdf;
-    if (reflecting)
-    {
-        float rr = scaled;
-        if (g.regularize && c.reg == REGULARIZATION_MIS)
-            rr = regularize_mix(g, c.reg, scaled, c.path_roughness, eta_i, eta_t);
-        else if (g.regularize && c.reg == REGULARIZATION_CLASSIC)
-            rr = regularize_reflection(g, c.reg, scaled, c.path_roughness);
-        DeltaSampled ds = delta_reflection_sampled(m, scaled, m.anisotropy, c.info);
-        pdf = ggx_pdf_reflect(rr, m.anisotropy, lv, ll, lh, ds);
-        pdf *= reflect_proba;
-    }
-    else
-    {
-        float rr = scaled;
-        if (g.regularize && c.reg == REGULARIZATION_MIS)
-            rr = regularize_mix(g, c.reg, scaled, c.path_roughness, eta_i, eta_t);
-        else if (g.regularize && c.reg == REGULARIZATION_CLASSIC)
-            rr = regularize_refraction(g, c.reg, scaled, c.path_roughness, eta_i, eta_t);
-        pdf = ggx_pdf_refract(m, rr, relative_eta, lv, ll, lh, c.info);
-        pdf *= 1.0f - reflect_proba;
-    }
-    return pdf;
 }
 
 // principled_glass_sample (Principled.h:726-830): a microfacet normal from the
@@ -1329,7 +1233,7 @@ PT_HD f3 glass_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& c, f3 lv
     return refract_ray(lv, mn, relative_eta);
 }
 
-// principled_diffuse_transmission_eval / _pdf (Principled.h:832-873).
+// principled_diffuse_transmission_eval (Principled.h:832-851).
 PT_HD Color dtrans_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, f3 lv, f3 ll, float& pdf)
 {
     pdf = 0.0f;
@@ -1350,13 +1254,6 @@ PT_HD Color dtrans_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& 
     }
     pdf = fabsf(ll.z * INV_PI_F);
     return color;
-}
-
-PT_HD float dtrans_pdf(f3 lv, f3 ll)
-{
-    if (lv.z * ll.z > 0.0f)
-        return 0.0f;
-    return fabsf(ll.z * INV_PI_F);
 }
 
 // ---------------------------------------------------------------------------
@@ -1385,69 +1282,130 @@ PT_HD LobeWeights lobe_weights(const Material& m, bool outside_object)
     return w;
 }
 
-// Principled.h:1556-1618 (no Fresnel-based lobe sampling: both options off).
-PT_HD LobeWeights lobe_probas(const LobeWeights& w)
+// Principled.h:1556-1618 (no Fresnel-based lobe sampling: both options off):
+// the probability of a lobe is its weight times this.
+PT_HD float lobe_proba_scale(const LobeWeights& w)
 {
-    float nf = 1.0f / (w.coat + w.sheen + w.metal1 + w.metal2 + w.specular + w.diffuse + w.glass + w.dtrans);
-    LobeWeights p;
-    p.coat = w.coat * nf;
-    p.sheen = w.sheen * nf;
-    p.metal1 = w.metal1 * nf;
-    p.metal2 = w.metal2 * nf;
-    p.specular = w.specular * nf;
-    p.diffuse = w.diffuse * nf;
-    p.glass = w.glass * nf;
-    p.dtrans = w.dtrans * nf;
-    return p;
+    return 1.0f / (w.coat + w.sheen + w.metal1 + w.metal2 + w.specular + w.diffuse + w.glass + w.dtrans);
 }
 
-// The three local frames of one evaluation (Principled.h:1633-1645).
+// The part of an evaluation that depends on the vertex and the view alone: a
+// vertex that evaluates several directions computes it once. One evaluation is
+// about 1500 instructions of a wave for a glossy material, nearly half of them
+// in here (pow and table lookup of the energy compensation, the frames, the
+// view's Fresnel terms and masking, the F82 fit), and the candidate loops are
+// bound by instruction issue. The media (c.vs->incident, ->inside) are those at
+// construction; popping the interior stack afterwards does not change them.
+struct ViewTerms {
+    f3 T, B, lv;    // unrotated ONB and the view in it
+    f3 TR, BR, lvr; // ONB rotated by anisotropy_rotation * pi
+    LobeWeights w;
+    float proba_scale;
+    float incident_ior;
+    LobeView base, metal2, coat;    // specular and first metal; second metal; coat
+    float kms1, kms2;               // conductor compensation of the metals
+    Color f82_a;
+    SheenView sheen;
+    float coat_fresnel;             // view Fresnel of the coat
+    Color coat_darkening;
+    float specular_ior;
+    Color specular_fresnel, specular_darkening;
+    float glossy_compensation, coat_compensation;
+};
+
+// The lobes' terms follow the regularisation mode and the path's roughness.
+PT_HD void view_lobes(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, ViewTerms& t)
+{
+    if (t.w.specular > 0.0f || t.w.metal1 > 0.0f)
+        t.base = lobe_view(regularize_reflection(g, c.reg, m.roughness, c.path_roughness), m.anisotropy, t.lvr);
+    if (t.w.metal1 > 0.0f)
+        t.kms1 = conductor_kms(g, t.base.roughness, t.lvr.z);
+    if (t.w.metal2 > 0.0f)
+    {
+        t.metal2 =
+            lobe_view(regularize_reflection(g, c.reg, m.second_roughness, c.path_roughness), m.anisotropy, t.lvr);
+        t.kms2 = conductor_kms(g, t.metal2.roughness, t.lvr.z);
+    }
+    if (t.w.coat > 0.0f)
+        t.coat =
+            lobe_view(regularize_reflection(g, c.reg, m.coat_roughness, c.path_roughness), m.coat_anisotropy, t.lv);
+}
+
+PT_HD ViewTerms view_terms(const BsdfGlobals& g, const Material& m, const BsdfCtx& c)
+{
+    ViewTerms t{};
+    build_onb(c.sn, t.T, t.B);
+    t.lv = world_to_local(t.T, t.B, c.sn, c.view);
+    build_rotated_onb(c.sn, t.TR, t.BR, m.anisotropy_rotation * PI_F);
+    t.lvr = world_to_local(t.TR, t.BR, c.sn, c.view);
+    t.w = lobe_weights(m, !c.vs->inside);
+    t.proba_scale = lobe_proba_scale(t.w);
+    t.incident_ior = medium_ior(g, c.vs->incident);
+    view_lobes(g, m, c, t);
+    if (t.w.metal1 > 0.0f || t.w.metal2 > 0.0f)
+        t.f82_a = f82_tint_scale(m.base_color, m.metallic_F82, m.metallic_F90, m.metallic_F90_falloff_exponent);
+    if (t.w.coat > 0.0f)
+    {
+        t.coat_fresnel = fresnel_dielectric(fabsf(t.lv.z), t.incident_ior, m.coat_ior);
+        t.coat_darkening = coat_darkening(m, m.coat_ior / t.incident_ior, t.coat_fresnel);
+    }
+    if (t.w.sheen != 0.0f && t.lv.z > 0.0f)
+        t.sheen = sheen_view(g, m, t.lv);
+    if (t.w.specular > 0.0f)
+    {
+        t.specular_ior = specular_relative_ior(m, t.incident_ior);
+        t.specular_fresnel = specular_fresnel(m, t.specular_ior, fabsf(t.lvr.z));
+        t.specular_darkening = specular_darkening(m, t.specular_ior);
+    }
+    t.glossy_compensation = energy_compensation_glossy_base(g, m, t.incident_ior, t.lv.z);
+    t.coat_compensation = energy_compensation_clearcoat(g, m, t.incident_ior, t.lv.z);
+    return t;
+}
+
+// The local frames of one evaluation (Principled.h:1633-1645).
 struct LocalFrames {
     f3 lv, ll, lh;    // unrotated ONB
     f3 lvr, llr, lhr; // ONB rotated by anisotropy_rotation * pi
 };
 
-PT_HD LocalFrames local_frames(const Material& m, const BsdfCtx& c)
+PT_HD LocalFrames local_frames(const ViewTerms& t, const BsdfCtx& c)
 {
     LocalFrames f;
-    f3 T, B;
-    build_onb(c.sn, T, B);
-    f.lv = world_to_local(T, B, c.sn, c.view);
-    f.ll = world_to_local(T, B, c.sn, c.to_light);
+    f.lv = t.lv;
+    f.ll = world_to_local(t.T, t.B, c.sn, c.to_light);
     f.lh = normalize(f.lv + f.ll);
-    f3 TR, BR;
-    build_rotated_onb(c.sn, TR, BR, m.anisotropy_rotation * PI_F);
-    f.lvr = world_to_local(TR, BR, c.sn, c.view);
-    f.llr = world_to_local(TR, BR, c.sn, c.to_light);
+    f.lvr = t.lvr;
+    f.llr = world_to_local(t.TR, t.BR, c.sn, c.to_light);
     f.lhr = normalize(f.lvr + f.llr);
     return f;
 }
+
+// x / 1 is x for every x: the usual compensation costs no division.
+PT_HD Color compensated(Color x, float compensation) { return compensation == 1.0f ? x : x / compensation; }
 
 // ---------------------------------------------------------------------------
 // Layers (Principled.h:955-1512), evaluated top to bottom; `layers` is the
 // energy left for the layers below.
 // ---------------------------------------------------------------------------
 // Principled.h:955-1058
-PT_HD Color eval_coat_layer(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const LocalFrames& f,
-                            float incident_ior, bool refracting, float weight, float proba, Color& layers,
-                            float& pdf)
+PT_HD Color eval_coat_layer(const Material& m, const BsdfCtx& c, const ViewTerms& t, const LocalFrames& f,
+                            bool refracting, float weight, float proba, Color& layers, float& pdf)
 {
-    float coat_ior = m.coat_ior;
+    const float coat_ior = m.coat_ior, incident_ior = t.incident_ior;
     if (weight > 0.0f && ((f.lv.z > 0.0f && f.ll.z > 0.0f) || refracting))
     {
         float cpdf = 0.0f;
         Color contribution = col(0.0f);
         if (!refracting)
         {
-            contribution = coat_eval(g, m, c, f.lv, f.ll, f.lh, incident_ior, cpdf);
+            contribution = coat_eval(m, c, t.coat, f.lv, f.ll, f.lh, incident_ior, cpdf);
             contribution = contribution * weight;
             contribution = contribution * layers;
         }
         pdf += cpdf * proba;
         Color below = col(1.0f);
         below = below * (1.0f - fresnel_dielectric(fabsf(f.ll.z), incident_ior, coat_ior));
-        float view_dir_fresnel = fresnel_dielectric(fabsf(f.lv.z), incident_ior, coat_ior);
-        below = below * (1.0f - view_dir_fresnel);
+        below = below * (1.0f - t.coat_fresnel);
         if (!is_white(m.coat_medium_absorption))
         {
             float in_angle = maxf_(1.0e-6f, sqrtf(1.0f - (1.0f - f.ll.z * f.ll.z) / (coat_ior * coat_ior)));
@@ -1459,7 +1417,7 @@ PT_HD Color eval_coat_layer(const BsdfGlobals& g, const Material& m, const BsdfC
             Color e = (col(0.0f) - (col(1.0f) - p)) * m.coat_medium_thickness;
             below = below * col(exp_fixed(e.r), exp_fixed(e.g), exp_fixed(e.b));
         }
-        below = below * coat_darkening(m, coat_ior / incident_ior, view_dir_fresnel);
+        below = below * t.coat_darkening;
         below = lerpc(col(1.0f), below, m.coat);
         layers = layers * below;
         return contribution;
@@ -1467,27 +1425,14 @@ PT_HD Color eval_coat_layer(const BsdfGlobals& g, const Material& m, const BsdfC
     return col(0.0f);
 }
 
-PT_HD float pdf_coat_layer(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const LocalFrames& f,
-                           bool refracting, float weight, float proba)
-{
-    if (weight > 0.0f && ((f.lv.z > 0.0f && f.ll.z > 0.0f) || refracting))
-    {
-        float cpdf = 0.0f;
-        if (!refracting)
-            cpdf = coat_pdf(g, m, c, f.lv, f.ll, f.lh);
-        return cpdf * proba;
-    }
-    return 0.0f;
-}
-
 // Principled.h:1088-1113
-PT_HD Color eval_sheen_layer(const BsdfGlobals& g, const Material& m, const LocalFrames& f, bool refracting,
-                             float weight, float proba, Color& layers, float& pdf)
+PT_HD Color eval_sheen_layer(const Material& m, const ViewTerms& t, const LocalFrames& f, bool refracting, float weight,
+                             float proba, Color& layers, float& pdf)
 {
     if ((weight > 0.0f && f.lv.z > 0.0f && f.ll.z > 0.0f) || refracting)
     {
         float reflectance, spdf;
-        Color contribution = sheen_eval(g, m, f.lv, f.ll, spdf, reflectance);
+        Color contribution = sheen_eval(m, t.sheen, f.lv, f.ll, spdf, reflectance);
         contribution = contribution * weight;
         contribution = contribution * layers;
         pdf += spdf * proba;
@@ -1497,23 +1442,14 @@ PT_HD Color eval_sheen_layer(const BsdfGlobals& g, const Material& m, const Loca
     return col(0.0f);
 }
 
-PT_HD float pdf_sheen_layer(const BsdfGlobals& g, const Material& m, const LocalFrames& f, bool refracting,
-                            float weight, float proba)
-{
-    if ((weight > 0.0f && f.lv.z > 0.0f && f.ll.z > 0.0f) || refracting)
-        return sheen_pdf(g, m, f.lv, f.ll) * proba;
-    return 0.0f;
-}
-
 // Principled.h:1129-1157 (the metal lobe has nothing below it).
-PT_HD Color eval_metal_layer(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const LocalFrames& f,
-                             float roughness, float incident_ior, float weight, float proba, const Color& layers,
-                             float& pdf)
+PT_HD Color eval_metal_layer(const Material& m, const BsdfCtx& c, const ViewTerms& t, const LocalFrames& f,
+                             const LobeView& l, float kms, float weight, float proba, const Color& layers, float& pdf)
 {
     if (weight > 0.0f && f.lvr.z > 0.0f && f.llr.z > 0.0f)
     {
         float mpdf = 0.0f;
-        Color contribution = metallic_eval(g, m, c, roughness, m.anisotropy, incident_ior, f.lvr, f.llr, f.lhr, mpdf);
+        Color contribution = metallic_eval(m, c, l, kms, t.f82_a, t.incident_ior, f.lvr, f.llr, f.lhr, mpdf);
         contribution = contribution * weight;
         contribution = contribution * layers;
         pdf += mpdf * proba;
@@ -1522,48 +1458,29 @@ PT_HD Color eval_metal_layer(const BsdfGlobals& g, const Material& m, const Bsdf
     return col(0.0f);
 }
 
-PT_HD float pdf_metal_layer(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const LocalFrames& f,
-                            float roughness, float weight, float proba)
-{
-    if (weight > 0.0f && f.lvr.z > 0.0f && f.llr.z > 0.0f)
-        return metallic_pdf(g, m, c, roughness, m.anisotropy, f.lvr, f.llr, f.lhr) * proba;
-    return 0.0f;
-}
-
 // Principled.h:1305-1405, in the rotated frame.
-PT_HD Color eval_specular_layer(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const LocalFrames& f,
-                                float incident_ior, float weight, bool refracting, float proba, Color& layers,
-                                float& pdf)
+PT_HD Color eval_specular_layer(const Material& m, const BsdfCtx& c, const ViewTerms& t, const LocalFrames& f,
+                                float weight, bool refracting, float proba, Color& layers, float& pdf)
 {
     if (weight > 0.0f && ((f.lvr.z > 0.0f && f.llr.z > 0.0f) || (refracting && c.info == FROM_DIFFUSE_TRANSMISSION)))
     {
-        float relative_ior = specular_relative_ior(m, incident_ior);
         float spdf = 0.0f;
-        Color contribution = specular_eval(g, m, c, relative_ior, f.lvr, f.llr, f.lhr, spdf);
+        Color contribution = specular_eval(m, c, t.base, t.specular_ior, f.lvr, f.llr, f.lhr, spdf);
         contribution = contribution * lerpc(col(1.0f), m.specular_tint * m.specular_color, m.specular);
         contribution = contribution * weight;
         contribution = contribution * layers;
         Color below = col(1.0f);
-        Color light_dir_fresnel = specular_fresnel(m, relative_ior, fabsf(f.llr.z));
+        Color light_dir_fresnel = specular_fresnel(m, t.specular_ior, fabsf(f.llr.z));
         light_dir_fresnel = light_dir_fresnel * (1.0f - m.diffuse_transmission);
         below = below * (col(1.0f) - light_dir_fresnel);
-        Color view_dir_fresnel = specular_fresnel(m, relative_ior, fabsf(f.lvr.z));
-        below = below * (col(1.0f) - view_dir_fresnel);
-        below = below * specular_darkening(m, relative_ior, luminance(view_dir_fresnel));
+        below = below * (col(1.0f) - t.specular_fresnel);
+        below = below * t.specular_darkening;
         below = lerpc(col(1.0f), below, m.specular);
         layers = layers * below;
         pdf += spdf * proba;
         return contribution;
     }
     return col(0.0f);
-}
-
-PT_HD float pdf_specular_layer(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const LocalFrames& f,
-                               float weight, bool refracting, float proba)
-{
-    if (weight > 0.0f && ((f.lvr.z > 0.0f && f.llr.z > 0.0f) || (refracting && c.info == FROM_DIFFUSE_TRANSMISSION)))
-        return specular_pdf(g, m, c, f.lvr, f.llr, f.lhr) * proba;
-    return 0.0f;
 }
 
 // Principled.h:1436-1469 (Lambertian diffuse, Lambertian.h:14-38).
@@ -1587,35 +1504,25 @@ PT_HD Color eval_diffuse_layer(const Material& m, const LocalFrames& f, float we
     return col(0.0f);
 }
 
-PT_HD float pdf_diffuse_layer(const LocalFrames& f, float weight, float proba)
-{
-    if (weight > 0.0f && f.lv.z > 0.0f && f.ll.z > 0.0f)
-        return (f.ll.z > 0.0f ? f.ll.z * INV_PI_F : 0.0f) * proba;
-    return 0.0f;
-}
-
 // ---------------------------------------------------------------------------
 // Principled BSDF (Principled.h:1620-1939)
 // ---------------------------------------------------------------------------
 // Principled.h:1556-1618 and :1620-1715
-PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, float& pdf)
+PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, const ViewTerms& t, float& pdf)
 {
     pdf = 0.0f;
-    const VolumeState& v = *c.vs;
-    bool outside = !v.inside;
-    bool refracting = dot(c.sn, c.to_light) < 0.0f && outside;
-    LocalFrames f = local_frames(m, c);
-    const float incident_ior = medium_ior(g, v.incident);
-    LobeWeights w = lobe_weights(m, outside);
-    LobeWeights p = lobe_probas(w);
+    const bool refracting = dot(c.sn, c.to_light) < 0.0f && !c.vs->inside;
+    const LocalFrames f = local_frames(t, c);
+    const LobeWeights& w = t.w;
+    const float nf = t.proba_scale;
     Color layers = col(1.0f);
     Color final_color = col(0.0f);
-    final_color = final_color + eval_coat_layer(g, m, c, f, incident_ior, refracting, w.coat, p.coat, layers, pdf);
-    final_color = final_color + eval_sheen_layer(g, m, f, refracting, w.sheen, p.sheen, layers, pdf);
-    final_color = final_color + eval_metal_layer(g, m, c, f, m.roughness, incident_ior, w.metal1 * (float)!refracting,
-                                                 p.metal1, layers, pdf);
-    final_color = final_color + eval_metal_layer(g, m, c, f, m.second_roughness, incident_ior,
-                                                 w.metal2 * (float)!refracting, p.metal2, layers, pdf);
+    final_color = final_color + eval_coat_layer(m, c, t, f, refracting, w.coat, w.coat * nf, layers, pdf);
+    final_color = final_color + eval_sheen_layer(m, t, f, refracting, w.sheen, w.sheen * nf, layers, pdf);
+    final_color = final_color + eval_metal_layer(m, c, t, f, t.base, t.kms1, w.metal1 * (float)!refracting,
+                                                 w.metal1 * nf, layers, pdf);
+    final_color = final_color + eval_metal_layer(m, c, t, f, t.metal2, t.kms2, w.metal2 * (float)!refracting,
+                                                 w.metal2 * nf, layers, pdf);
     // glass layer (Principled.h:1177-1200), rotated frame
     if (w.glass > 0.0f)
     {
@@ -1623,14 +1530,14 @@ PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfC
         Color contribution = glass_eval(g, m, c, f.lvr, f.llr, gpdf);
         contribution = contribution * w.glass;
         contribution = contribution * layers;
-        pdf += gpdf * p.glass;
+        pdf += gpdf * (w.glass * nf);
         final_color = final_color + contribution;
     }
     // glossy base: specular layer over the diffuse layer (Principled.h:1474-1492)
     Color glossy = col(0.0f);
-    glossy = glossy + eval_specular_layer(g, m, c, f, incident_ior, w.specular, refracting, p.specular, layers, pdf);
-    glossy = glossy + eval_diffuse_layer(m, f, w.diffuse * (float)!refracting, p.diffuse, layers, pdf);
-    final_color = final_color + glossy / energy_compensation_glossy_base(g, m, incident_ior, f.lv.z);
+    glossy = glossy + eval_specular_layer(m, c, t, f, w.specular, refracting, w.specular * nf, layers, pdf);
+    glossy = glossy + eval_diffuse_layer(m, f, w.diffuse * (float)!refracting, w.diffuse * nf, layers, pdf);
+    final_color = final_color + compensated(glossy, t.glossy_compensation);
     // diffuse transmission layer (Principled.h:1219-1241)
     if (w.dtrans > 0.0f && f.ll.z < 0.0f)
     {
@@ -1638,64 +1545,41 @@ PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfC
         Color contribution = dtrans_eval(g, m, c, f.lv, f.ll, dpdf);
         contribution = contribution * w.dtrans;
         contribution = contribution * layers;
-        pdf += dpdf * p.dtrans;
+        pdf += dpdf * (w.dtrans * nf);
         final_color = final_color + contribution;
     }
-    return final_color / energy_compensation_clearcoat(g, m, incident_ior, f.lv.z);
+    return compensated(final_color, t.coat_compensation);
 }
 
-// Principled.h:1717-1800
-PT_HD float principled_pdf(const BsdfGlobals& g, const Material& m, const BsdfCtx& c)
+PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, float& pdf)
 {
-    float pdf = 0.0f;
-    const VolumeState& v = *c.vs;
-    bool outside = !v.inside;
-    bool refracting = dot(c.sn, c.to_light) < 0.0f && outside;
-    LocalFrames f = local_frames(m, c);
-    LobeWeights w = lobe_weights(m, outside);
-    LobeWeights p = lobe_probas(w);
-    pdf += pdf_coat_layer(g, m, c, f, refracting, w.coat, p.coat);
-    pdf += pdf_sheen_layer(g, m, f, refracting, w.sheen, p.sheen);
-    pdf += pdf_metal_layer(g, m, c, f, m.roughness, w.metal1 * (float)!refracting, p.metal1);
-    pdf += pdf_metal_layer(g, m, c, f, m.second_roughness, w.metal2 * (float)!refracting, p.metal2);
-    if (w.glass > 0.0f)
-        pdf += glass_pdf(g, m, c, f.lvr, f.llr) * p.glass;
-    float glossy = 0.0f;
-    glossy += pdf_specular_layer(g, m, c, f, w.specular, refracting, p.specular);
-    glossy += pdf_diffuse_layer(f, w.diffuse * (float)!refracting, p.diffuse);
-    pdf += glossy;
-    if (w.dtrans > 0.0f && f.ll.z < 0.0f)
-        pdf += dtrans_pdf(f.lv, f.ll) * p.dtrans;
-    return pdf;
+    return principled_eval(g, m, c, view_terms(g, m, c), pdf);
 }
 
 // Principled.h:1802-1939. Returns the BSDF value of the sampled direction;
 // pdf = 0 when the sample is invalid. `c.info` receives the sampled lobe
 // (the sheen lobe leaves it as it was). With c.update, a reflection pops the
 // material of the vertex from the interior stack (the path stays outside).
-PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& c, f3& out_dir, float& pdf,
-                              Xorshift32& rng)
+PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& c, const ViewTerms& t, f3& out_dir,
+                              float& pdf, Xorshift32& rng)
 {
     pdf = 0.0f;
     VolumeState& v = *c.vs;
-    bool outside = !v.inside;
-    LobeWeights w = lobe_weights(m, outside);
-    LobeWeights p = lobe_probas(w);
-    float cdf0 = p.coat;
-    float cdf1 = cdf0 + p.sheen;
-    float cdf2 = cdf1 + p.metal1;
-    float cdf3 = cdf2 + p.metal2;
-    float cdf4 = cdf3 + p.specular;
-    float cdf5 = cdf4 + p.diffuse;
-    float cdf6 = cdf5 + p.dtrans;
+    const LobeWeights& w = t.w;
+    const float nf = t.proba_scale;
+    float cdf0 = w.coat * nf;
+    float cdf1 = cdf0 + w.sheen * nf;
+    float cdf2 = cdf1 + w.metal1 * nf;
+    float cdf3 = cdf2 + w.metal2 * nf;
+    float cdf4 = cdf3 + w.specular * nf;
+    float cdf5 = cdf4 + w.diffuse * nf;
+    float cdf6 = cdf5 + w.dtrans * nf;
     float rand_1 = rng();
     bool sampling_dt = rand_1 > cdf5 && rand_1 < cdf6;
     bool sampling_glass = rand_1 > cdf6;
     if (c.update && !sampling_glass && !sampling_dt)
         vol_pop(v, false);
-    f3 TR, BR;
-    build_rotated_onb(c.sn, TR, BR, m.anisotropy_rotation * PI_F);
-    f3 lvr = world_to_local(TR, BR, c.sn, c.view);
+    const f3 TR = t.TR, BR = t.BR, lvr = t.lvr;
     if (rand_1 < cdf0)
     {
         f3 TC, BC;
@@ -1707,10 +1591,7 @@ PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& 
     }
     else if (rand_1 < cdf1)
     {
-        f3 T, B;
-        build_onb(c.sn, T, B);
-        f3 lv = world_to_local(T, B, c.sn, c.view);
-        out_dir = local_to_world(T, B, c.sn, sheen_sample(g, m, lv, rng));
+        out_dir = local_to_world(t.T, t.B, c.sn, sheen_sample(g, m, t.lv, rng));
     }
     else if (rand_1 < cdf2)
     {
@@ -1745,7 +1626,13 @@ PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& 
     if (dot(out_dir, c.gn) < 0.0f && !sampling_glass && !sampling_dt)
         return col(0.0f);
     c.to_light = out_dir;
-    return principled_eval(g, m, c, pdf);
+    return principled_eval(g, m, c, t, pdf);
+}
+
+PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& c, f3& out_dir, float& pdf,
+                              Xorshift32& rng)
+{
+    return principled_sample(g, m, c, view_terms(g, m, c), out_dir, pdf, rng);
 }
 
 // ---------------------------------------------------------------------------
