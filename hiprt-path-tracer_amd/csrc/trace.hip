@@ -17,7 +17,8 @@
 //     deeper than the LDS stack spill to a per-thread global array;
 //   * a persistent grid sized from occupancy; each wave takes batches of rays
 //     from a global counter and hands them to lanes whose ray is done, once
-//     REFILL_LANES of them are;
+//     REFILL_LANES of them are. When none are left, its last GROUPS rays get
+//     eight lanes each;
 //   * optionally the rays to trace come from segmented queues of slot
 //     indices (seglist.h) whose lengths are read on the device (the path
 //     passes enqueue only live rays); results go to the rays' own slots.
@@ -61,13 +62,12 @@ __global__ void k_reset_counter(uint32_t* c) { c[0] = 0u; }
 // without a ray that make it take more (8 to 24: the same).
 constexpr int LEAF_LANES = 8;
 constexpr int REFILL_LANES = 16;
-// Fewer rays than the grid has lanes are dealt to 2 waves per SIMD, at least
-// MIN_BATCH to a wave: a wave of few rays takes fewer different branches and
-// ends sooner, but more waves than that wait for each other's instructions
-// (120,000 bounce rays of the 1M-triangle scene: 195 us at 64 rays a wave,
-// 160 us at 24, 140 to 146 us dealt so).
+// Fewer rays than the grid has lanes are dealt to 3 waves per SIMD, at least
+// MIN_BATCH to a wave, one for each of its groups of eight lanes (120,000
+// bounce rays of the 1M-triangle scene: 120 us at 2 waves, 116 us at 3, 119 to
+// 126 us at 4 to 6; 1 to 8 rays a wave measure the same).
 constexpr uint32_t MIN_BATCH = 8;
-constexpr uint32_t FEW_WAVES_PER_CU = 8;
+constexpr uint32_t FEW_WAVES_PER_CU = 12;
 
 constexpr int32_t IDLE = 0x7fffffff; // no node or leaf to visit (node indices stay below)
 
@@ -94,6 +94,7 @@ struct TraceArgs {
     uint32_t* work_counter;
     uint32_t tile;
     uint32_t few_waves; // waves that fewer rays than the grid's lanes are dealt to
+    uint32_t last_tri;  // index of the last triangle record
 };
 
 __device__ __forceinline__ uint32_t med3(uint32_t a, uint32_t b, uint32_t c) { return max(min(a, b), min(max(a, b), c)); }
@@ -113,6 +114,47 @@ __device__ __forceinline__ void sort6(uint32_t k[6])
     k[3] = max(m, n);
     k[4] = max(q, y);
     k[5] = max(a2, b2);
+}
+
+// The last GROUPS rays of a wave are traced by eight lanes each, lane c of a
+// group taking child c of a node and triangle c of a leaf. What ends a launch is
+// its longest ray: a round of one lane to a ray issues about 300 instructions
+// (four cycles each) after waiting for its node, a round of eight lanes about
+// 200 for a node and a leaf whose loads are under way together. 61 camera rays:
+// 21.6 us with one lane to a ray, 15.3 us so; 12,513 bounce rays 59.6 us and
+// 41 us, 120,000 (which end one lane to a ray until eight are left in a wave)
+// 142 us and 116 us; 2,073,600 516 us and 506 us. Eight rays is what the lanes
+// hold; a wave with more has enough to issue.
+constexpr int GROUP = 8;
+constexpr int GROUPS = 64 / GROUP;
+
+// Value of the lane whose index in the group of eight is lane ^ X.
+template <int X> __device__ __forceinline__ uint32_t group_xor(uint32_t v)
+{
+    constexpr int QUAD = X & 4 ? 3 - (X & 3) : X; // half-row mirror is ^ 7
+    int r = (int)v;
+    if (X & 4)
+        r = __builtin_amdgcn_mov_dpp(r, 0x141, 0xf, 0xf, true); // row_half_mirror
+    if (QUAD == 1)
+        r = __builtin_amdgcn_mov_dpp(r, 0xb1, 0xf, 0xf, true); // quad_perm 1 0 3 2
+    else if (QUAD == 2)
+        r = __builtin_amdgcn_mov_dpp(r, 0x4e, 0xf, 0xf, true); // quad_perm 2 3 0 1
+    else if (QUAD == 3)
+        r = __builtin_amdgcn_mov_dpp(r, 0x1b, 0xf, 0xf, true); // quad_perm 3 2 1 0
+    return (uint32_t)r;
+}
+
+__device__ __forceinline__ uint32_t group_min(uint32_t v)
+{
+    v = min(v, group_xor<1>(v));
+    v = min(v, group_xor<2>(v));
+    return min(v, group_xor<7>(v));
+}
+
+// Lanes of the group (bit c for lane c) that vote yes.
+__device__ __forceinline__ uint32_t group_ballot(bool yes, uint32_t group_shift)
+{
+    return (uint32_t)(__ballot(yes) >> group_shift) & 0xffu;
 }
 
 template <int I> __device__ __forceinline__ float byte_of(uint32_t w) { return (float)((w >> (8 * I)) & 0xffu); }
@@ -194,33 +236,40 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
     int32_t leaf = 0;    // leaf whose triangles wait to be tested, 0 for none
     int sp = 0;
 
+    auto write_result = [&]() {
+        if (any)
+        {
+            uint8_t* occ = a.job[0].occluded;
+            if (QUEUES)
+                occ = job == 0u ? a.job[0].occluded : (job == 1u ? a.job[1].occluded : a.job[2].occluded);
+            occ[slot] = best_prim >= 0 ? 1 : 0;
+        }
+        else
+        {
+            int4* hits = a.job[0].hits;
+            if (QUEUES)
+                hits = job == 0u ? a.job[0].hits : (job == 1u ? a.job[1].hits : a.job[2].hits);
+            hits[slot] = best_prim >= 0 ? make_int4(best_prim, __float_as_int(best_t), __float_as_int(best_u),
+                                                    __float_as_int(best_v))
+                                        : make_int4(-1, __float_as_int(-1.0f), 0, 0);
+            if (MODE == CLOSEST_COUNTED)
+                a.counts[slot] = make_uint2(n_nodes, n_tris);
+        }
+    };
+
+    // The instrumented variant counts a ray's visits one lane to a ray.
+    constexpr int LAST_RAYS = MODE == CLOSEST_COUNTED ? 0 : GROUPS;
     for (;;)
     {
         const uint64_t idle = __ballot(cur == IDLE && leaf == 0 && sp == 0);
-        if (idle == ~0ull || (more && __popcll(idle) >= REFILL_LANES))
+        const int live = 64 - __popcll(idle);
+        if (more ? live <= 64 - REFILL_LANES : live <= LAST_RAYS)
         {
             const bool free = cur == IDLE && leaf == 0 && sp == 0;
             if (free && has_ray)
             {
                 has_ray = false;
-                if (any)
-                {
-                    uint8_t* occ = a.job[0].occluded;
-                    if (QUEUES)
-                        occ = job == 0u ? a.job[0].occluded : (job == 1u ? a.job[1].occluded : a.job[2].occluded);
-                    occ[slot] = best_prim >= 0 ? 1 : 0;
-                }
-                else
-                {
-                    int4* hits = a.job[0].hits;
-                    if (QUEUES)
-                        hits = job == 0u ? a.job[0].hits : (job == 1u ? a.job[1].hits : a.job[2].hits);
-                    hits[slot] = best_prim >= 0 ? make_int4(best_prim, __float_as_int(best_t), __float_as_int(best_u),
-                                                            __float_as_int(best_v))
-                                                : make_int4(-1, __float_as_int(-1.0f), 0, 0);
-                    if (MODE == CLOSEST_COUNTED)
-                        a.counts[slot] = make_uint2(n_nodes, n_tris);
-                }
+                write_result();
             }
             if (more && next >= batch_end)
             {
@@ -298,7 +347,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
                 }
                 next += min((uint32_t)__popcll(idle), left);
             }
-            else if (idle == ~0ull)
+            else if (live <= LAST_RAYS)
                 break;
         }
 
@@ -439,6 +488,194 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
             }
         }
     }
+
+    // The wave's last rays, eight lanes to each.
+    const uint64_t live_lanes = __ballot(has_ray);
+    if (MODE == CLOSEST_COUNTED || live_lanes == 0ull)
+        return;
+    const uint32_t c = lane & 7u, group = lane >> 3, group_shift = lane & 56u;
+    uint64_t mine = live_lanes;
+#pragma unroll
+    for (uint32_t i = 0; i + 1 < GROUPS; i++)
+        mine = i < group ? mine & (mine - 1ull) : mine;
+    const int owner = mine ? __ffsll((unsigned long long)mine) - 1 : (int)lane;
+    auto from_owner_f = [&](float v) { return __shfl(v, owner); };
+    auto from_owner_i = [&](int32_t v) { return __shfl(v, owner); };
+    o = pt::mk(from_owner_f(o.x), from_owner_f(o.y), from_owner_f(o.z));
+    d = pt::mk(from_owner_f(d.x), from_owner_f(d.y), from_owner_f(d.z));
+    inv_nx = from_owner_f(inv_nx);
+    inv_ny = from_owner_f(inv_ny);
+    inv_nz = from_owner_f(inv_nz);
+    inv_fx = from_owner_f(inv_fx);
+    inv_fy = from_owner_f(inv_fy);
+    inv_fz = from_owner_f(inv_fz);
+    best_t = from_owner_f(best_t);
+    best_u = from_owner_f(best_u);
+    best_v = from_owner_f(best_v);
+    best_prim = from_owner_i(best_prim);
+    last_prim = from_owner_i(last_prim);
+    slot = (uint32_t)from_owner_i((int32_t)slot);
+    job = (uint32_t)from_owner_i((int32_t)job);
+    any = from_owner_i(any ? 1 : 0) != 0;
+    cur = mine ? from_owner_i(cur) : IDLE;
+    leaf = mine ? from_owner_i(leaf) : 0;
+    sp = mine ? from_owner_i(sp) : 0;
+    if (!mine)
+    {
+        cur = IDLE;
+        leaf = 0;
+        sp = 0;
+    }
+    // the ray's stack stays in its owner's columns
+    uint2* const column = stack + ((threadIdx.x & ~63u) + (uint32_t)owner);
+    uint2* const deep = a.spill + (gtid - lane + (uint32_t)owner);
+    const bool bx = inv_nx < 0.0f, by = inv_ny < 0.0f, bz = inv_nz < 0.0f;
+    // children 4 and 5 have their planes in the tail words: entry planes in
+    // bytes 0 and 1, exit planes in bytes 2 and 3, swapped by the direction
+    const bool tail = c >= 4u;
+    const uint32_t lo_shift = tail ? 8u * (c & 1u) : 8u * c, hi_shift = tail ? lo_shift + 16u : lo_shift;
+    const uint32_t nx_shift = bx ? hi_shift : lo_shift, fx_shift = bx ? lo_shift : hi_shift;
+    const uint32_t ny_shift = by ? hi_shift : lo_shift, fy_shift = by ? lo_shift : hi_shift;
+    const uint32_t nz_shift = bz ? hi_shift : lo_shift, fz_shift = bz ? lo_shift : hi_shift;
+
+    auto put_leaf_aside = [&]() {
+        if (cur < 0 && leaf == 0)
+        {
+            leaf = cur;
+            cur = IDLE;
+        }
+    };
+    // Stack entries written by one lane of a group are read by the others: the
+    // lanes of a wave run in step and its memory operations stay in order, so
+    // only the compiler has to keep that order.
+    auto stack_fence = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    stack_fence();
+    for (;;)
+    {
+        // The eight topmost entries at once: the first in reach of the closest
+        // hit is next, those above it are dropped.
+        auto pop = [&]() {
+            if (cur == IDLE && sp > 0)
+            {
+                const int at = sp - 1 - (int)c;
+                uint2 e = make_uint2(0x7f800001u, 0u); // NaN: out of reach
+                if (at >= 0)
+                    e = at < STACK ? column[at * BLOCK] : deep[(size_t)(at - STACK) * a.spill_stride];
+                const uint32_t in_reach = group_ballot(__uint_as_float(e.x) <= best_t * WIDEN_HI, group_shift);
+                const int first = in_reach ? __ffs((int)in_reach) - 1 : 0;
+                const int32_t ref = __shfl((int32_t)e.y, (int)group_shift + first);
+                if (in_reach)
+                {
+                    cur = ref;
+                    sp -= first + 1;
+                }
+                else
+                    sp = max(sp - GROUP, 0);
+            }
+        };
+        put_leaf_aside();
+        pop();
+        put_leaf_aside();
+        if (!__any(cur != IDLE || leaf != 0 || sp > 0))
+            break;
+        // both loads go out together; a group without a node or leaf reads the
+        // first one
+        const bool at_node = (uint32_t)cur < (uint32_t)IDLE;
+        const WideNode* np = a.nodes + (at_node ? cur : 0);
+        const float4 org = np->origin;
+        const uint4 refs = np->refs, qxy = np->qxy, qz = np->qz;
+        const TriRecord* tr = a.tris + (leaf != 0 ? min(((uint32_t)leaf & ~WIDE_LEAF) + c, a.last_tri) : 0u);
+        const float4 v0 = tr->v0, e1 = tr->e1, e2 = tr->e2;
+
+        if (leaf != 0)
+        {
+            // lanes past the leaf's last triangle have nothing
+            const uint32_t lasts = group_ballot(__float_as_int(e1.w) != 0, group_shift);
+            const bool in_leaf = (((lasts ^ (lasts - 1u)) >> c) & 1u) != 0u;
+            leaf = lasts ? 0 : leaf + GROUP;
+            const int32_t prim = __float_as_int(v0.w);
+            float t, u, v;
+            const bool hit = in_leaf &&
+                             pt::mt_intersect(pt::mk(v0.x, v0.y, v0.z), pt::mk(e1.x, e1.y, e1.z),
+                                              pt::mk(e2.x, e2.y, e2.z), o, d, t, u, v) &&
+                             prim != last_prim && (t < best_t || (t == best_t && prim < best_prim));
+            // positive floats order as their bits
+            const uint32_t tb = hit ? __float_as_uint(t) : ~0u;
+            const uint32_t t_min = group_min(tb);
+            const bool nearest = hit && tb == t_min;
+            const uint32_t p_min = group_min(nearest ? (uint32_t)prim : ~0u);
+            const uint32_t winner = group_ballot(nearest && (uint32_t)prim == p_min, group_shift);
+            if (winner)
+            {
+                const int src = (int)group_shift + __ffs((int)winner) - 1;
+                best_u = __shfl(u, src);
+                best_v = __shfl(v, src);
+                best_t = __uint_as_float(t_min);
+                best_prim = (int32_t)p_min;
+                if (any)
+                {
+                    cur = IDLE;
+                    leaf = 0;
+                    sp = 0;
+                }
+            }
+        }
+        if ((uint32_t)cur < (uint32_t)IDLE)
+        {
+            const uint32_t ex = (uint32_t)__float_as_int(org.w);
+            const float sx = __uint_as_float(ex << 23), sy = __uint_as_float((ex << 14) & 0x7f800000u),
+                        sz = __uint_as_float(ex & 0x7f800000u);
+            const float px = org.x - o.x, py = org.y - o.y, pz = org.z - o.z;
+            const uint32_t wnx = tail ? refs.w : (bx ? qxy.y : qxy.x), wfx = tail ? refs.w : (bx ? qxy.x : qxy.y);
+            const uint32_t wny = tail ? qz.z : (by ? qxy.w : qxy.z), wfy = tail ? qz.z : (by ? qxy.z : qxy.w);
+            const uint32_t wnz = tail ? qz.w : (bz ? qz.y : qz.x), wfz = tail ? qz.w : (bz ? qz.x : qz.y);
+            auto plane = [](uint32_t w, uint32_t shift) { return (float)__builtin_amdgcn_ubfe(w, shift, 8u); };
+            const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(plane(wnx, nx_shift), sx * inv_nx, px * inv_nx),
+                                               __builtin_fmaf(plane(wny, ny_shift), sy * inv_ny, py * inv_ny)),
+                                         __builtin_fmaf(plane(wnz, nz_shift), sz * inv_nz, pz * inv_nz)),
+                                   0.0f);
+            const float tf = fminf(fminf(fminf(__builtin_fmaf(plane(wfx, fx_shift), sx * inv_fx, px * inv_fx),
+                                               __builtin_fmaf(plane(wfy, fy_shift), sy * inv_fy, py * inv_fy)),
+                                         __builtin_fmaf(plane(wfz, fz_shift), sz * inv_fz, pz * inv_fz)),
+                                   best_t * WIDEN_HI);
+            const bool hit = tn <= tf && c < ((ex >> 17) & 7u);
+            const uint32_t key = hit ? ((__float_as_uint(tn) & ~31u) | (5u * c + 1u)) : ~0u;
+            // children nearer than this lane's: keys differ by their child
+            uint32_t rank = 0u;
+            rank += group_xor<1>(key) < key ? 1u : 0u;
+            rank += group_xor<2>(key) < key ? 1u : 0u;
+            rank += group_xor<3>(key) < key ? 1u : 0u;
+            rank += group_xor<4>(key) < key ? 1u : 0u;
+            rank += group_xor<5>(key) < key ? 1u : 0u;
+            rank += group_xor<6>(key) < key ? 1u : 0u;
+            rank += group_xor<7>(key) < key ? 1u : 0u;
+            const uint32_t nearest = group_min(key);
+            const int hits = __popc(group_ballot(hit, group_shift));
+            auto ref_of = [&](uint32_t k) {
+                const uint32_t m = __builtin_amdgcn_ubfe(refs.z, k, 5u);
+                return (m < 16u ? refs.y : refs.x) + m;
+            };
+            const int top = sp + hits - 1;
+            if (hit && rank > 0u)
+            {
+                const int at = top - (int)rank;
+                const uint2 e = make_uint2(key, ref_of(key));
+                if (at < STACK)
+                    column[at * BLOCK] = e;
+                else
+                    deep[(size_t)(at - STACK) * a.spill_stride] = e;
+            }
+            stack_fence();
+            cur = IDLE;
+            if (hits > 0)
+            {
+                sp = top;
+                cur = (int32_t)ref_of(nearest);
+            }
+        }
+    }
+    if (mine && c == 0u)
+        write_result();
 }
 
 __global__ void k_all_miss(int4* __restrict__ hits, uint8_t* __restrict__ occluded, uint32_t n)
@@ -565,6 +802,7 @@ TraceArgs trace_args(Ctx& ctx, uint32_t threads, const Scratch& sc)
     a.work_counter = sc.counter;
     a.tile = (uint32_t)ctx.trace_cfg.queue_tile;
     a.few_waves = (uint32_t)ctx.cu_count * FEW_WAVES_PER_CU;
+    a.last_tri = (uint32_t)ctx.bvh.triangle_count - 1u;
     return a;
 }
 

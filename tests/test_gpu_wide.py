@@ -91,3 +91,47 @@ def test_ray_batches(mipt_mod, oracle_mod, torch_mod, scene1, n, block, stack):
     ctx.set_trace_config(block, stack)
     _assert_hits_equal(ctx.trace_closest_host(rays[:n]), want[:n])
     ctx.close()
+
+
+@pytest.mark.parametrize("crowd", [False, True])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 17, 63, 64, 129])
+def test_last_rays(mipt_mod, oracle_mod, torch_mod, n, crowd):
+    """The rays that eight lanes share: slivers through one point, whose boxes
+    all overlap (stacks past the LDS entries, in the columns of the lanes that
+    the rays began in), alone in their waves and as the rest of larger batches
+    (`crowd`: the others miss at once); with the triangle that each hits
+    excluded, so that the next one of its leaf counts."""
+    rng = np.random.default_rng(n)
+    k = 3000
+    d = rng.normal(size=(k, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    off = rng.normal(size=(k, 3)) * 0.02
+    V = np.stack([-3 * d + off, 3 * d + off, 3 * d - off + rng.normal(size=(k, 3)) * 0.05], 1).astype(np.float32)
+    V = V.reshape(-1, 3)
+    I = np.arange(3 * k, dtype=np.int32).reshape(k, 3)
+    ctx = _ctx(mipt_mod, mipt_mod.Scene(V, I), mipt_mod.MIPT_BVH_SAH_BINNED)
+    rays = np.zeros(n, mipt_mod.RAY_DTYPE)
+    o = rng.normal(size=(n, 3))
+    o = (4 * o / np.linalg.norm(o, axis=1, keepdims=True)).astype(np.float32)
+    aim = rng.normal(size=(n, 3)) * 0.3 - o
+    rays["o"] = o
+    rays["d"] = (aim / np.linalg.norm(aim, axis=1, keepdims=True)).astype(np.float32)
+    rays["last_prim"] = -1
+    rays["tmax"] = np.inf
+    rays["last_prim"] = oracle_mod.trace_brute(V, I, rays)["prim"]
+    want = oracle_mod.trace_brute(V, I, rays)
+    at = np.arange(n)
+    if crowd:
+        many = np.zeros(40 * n, mipt_mod.RAY_DTYPE)
+        many["o"] = (50, 50, 50)
+        many["d"] = (1, 0, 0)
+        many["last_prim"] = -1
+        many["tmax"] = np.inf
+        at = np.sort(rng.choice(many.size, n, replace=False))
+        many[at] = rays
+        rays = many
+    got = ctx.trace_closest_host(rays)
+    _assert_hits_equal(got[at], want)
+    assert np.all(np.delete(got["prim"], at) == -1)
+    assert np.array_equal(ctx.trace_any_host(rays)[at].astype(bool), want["prim"] >= 0)
+    ctx.close()
