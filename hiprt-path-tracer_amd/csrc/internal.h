@@ -310,21 +310,25 @@ void autotune_trace(Ctx& ctx, const mipt_ray* rays, uint32_t n, int32_t repeats,
 // address noalloc_scratch_init looks up (once per device, device current).
 void noalloc_scratch_init(int device);
 void trace_closest_noalloc(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint32_t n, hipStream_t stream);
-// Trace the rays whose slots a segmented queue lists (seglist.h; length read
-// on the device, at most capacity rays); results go to the same slots.
-void trace_closest_queue(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, const SegList& queue, uint32_t capacity,
-                         hipStream_t stream);
-void trace_any_queue(Ctx& ctx, const mipt_ray* rays, uint8_t* occluded, const SegList& queue, uint32_t capacity,
-                     hipStream_t stream);
-// Up to three queued ray sets in one launch: a set with `occluded` is traced
-// any-hit (shadow rays), the others closest-hit into `hits`.
+// Up to three ray sets in one launch, each the rays whose slots a segmented
+// queue lists (seglist.h; lengths read on the device, at most `capacity`
+// rays, whose slots are below it); results go to the same slots. A set with `occluded` is traced any-hit
+// (shadow rays), the others closest-hit into `hits`. `counter` is 0 when the
+// launch begins: one of trace_counters, which the passes that enqueue the rays
+// reset in kernels that they launch anyway.
 struct TraceQueue {
     const mipt_ray* rays;
     mipt_hit* hits;
     uint8_t* occluded;
     const SegList* queue;
+    uint32_t capacity;
 };
-void trace_queues(Ctx& ctx, const TraceQueue* queues, int count, uint32_t capacity, hipStream_t stream);
+void trace_queues(Ctx& ctx, const TraceQueue* queues, int count, uint32_t* counter, hipStream_t stream);
+// Work counters for launches over queues, free for use between two other
+// trace launches of the context.
+constexpr uint32_t TRACE_COUNTERS = 1u + (uint32_t)MAX_SKIP_ROUNDS;
+uint32_t* trace_counters(Ctx& ctx);
+
 
 // camera.hip
 void camera_rays(Ctx& ctx, const mipt_camera& cam, int32_t w, int32_t h, uint32_t sample_number,

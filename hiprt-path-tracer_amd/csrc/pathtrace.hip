@@ -68,6 +68,40 @@ struct RayQueues {
     SegList skip[2];
 };
 
+// Counters of a path pass that are 0 before their kernels run. k_pass_reset
+// clears all of them once a pass; within the bounces each is cleared by the
+// last kernel before its users that does not use it itself (k_shade the skip
+// lists, the next bounce's list, the sort's and the trace launches', k_resolve
+// the ray lists). A reset kernel of its own took 4.6 us before each use: 18 of
+// them in a pass of four bounces, 83 us of the 682 of a 129 x 97 sample.
+struct PassCounters {
+    uint32_t* rays;  // shadow, BSDF, continuation, the two skip lists, the two live ones: back to back
+    uint32_t* next;  // list of the next bounce's paths
+    uint32_t* sort;  // counters and cursors of the sort, null without it
+    uint32_t* trace; // TRACE_COUNTERS, one per trace launch of a bounce
+};
+constexpr uint32_t RAY_LISTS = 3, SKIP_LISTS = 2, LIVE_LISTS = 2;
+
+__device__ __forceinline__ void reset_lists(uint32_t* counts, uint32_t lists)
+{
+    for (uint32_t i = threadIdx.x; i < lists * SEG_COUNT; i += blockDim.x)
+        counts[i * SEG_STRIDE] = 0u;
+}
+
+__device__ __forceinline__ void reset_sort(uint32_t* counts)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 2u * SHADE_SORT_COUNTERS; i += gridDim.x * blockDim.x)
+        counts[i * SEG_STRIDE] = 0u;
+}
+
+__global__ __launch_bounds__(256) void k_pass_reset(PassCounters c)
+{
+    if (blockIdx.x == 0)
+        reset_lists(c.rays, RAY_LISTS + SKIP_LISTS + LIVE_LISTS);
+    if (c.sort)
+        reset_sort(c.sort);
+}
+
 // Zeroes the counters of `lists` segmented lists stored back to back.
 __global__ void k_seg_reset(uint32_t* counts, uint32_t lists)
 {
@@ -630,13 +664,6 @@ __device__ __forceinline__ uint32_t shade_class(const PtData& d, uint32_t pix)
     return (uint32_t)d.mat_class[mi] | ((flags & FLAG_VOL) ? 32u : 0u);
 }
 
-__global__ void k_sort_reset(uint32_t* counts)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2u * SHADE_SORT_COUNTERS)
-        counts[i * SEG_STRIDE] = 0u;
-}
-
 __global__ __launch_bounds__(256) void k_sort_hist(PtData d, SegList live, uint32_t* __restrict__ counts)
 {
     __shared__ uint32_t h[SHADE_SORT_CLASSES];
@@ -726,8 +753,18 @@ __global__ __launch_bounds__(256) void k_sort_scatter(PtData d, SegList live, co
 // SIMD) beats spilling to scratch at 4 waves (11.08 vs 11.74 ms per 1080p
 // config-1 sample).
 __global__ __launch_bounds__(256, 2) void k_shade(PtData d, int32_t bounce, RayQueues q, SegList live,
-                                                  const uint32_t* __restrict__ sorted, float4* __restrict__ thr_prev)
+                                                  const uint32_t* __restrict__ sorted, float4* __restrict__ thr_prev,
+                                                  PassCounters c)
 {
+    if (blockIdx.x == 0)
+    {
+        reset_lists(c.rays + RAY_LISTS * SEG_COUNTER_WORDS, SKIP_LISTS);
+        reset_lists(c.next, 1u);
+        if (threadIdx.x < TRACE_COUNTERS)
+            c.trace[threadIdx.x] = 0u;
+    }
+    if (c.sort)
+        reset_sort(c.sort);
     const LiveIndex li = live_index(live);
     if (li.wave_empty)
         return;
@@ -951,8 +988,10 @@ __device__ __forceinline__ int resolve_path(const PtData& d, int32_t bounce, con
 // Over the paths shaded this bounce: those at a new vertex go to `next`, those
 // whose continuation ray skipped a boundary to `skip`.
 __global__ void k_resolve(PtData d, int32_t bounce, const float4* __restrict__ thr_prev, SegList live, SegList skip,
-                          SegList next)
+                          SegList next, PassCounters c)
 {
+    if (blockIdx.x == 0)
+        reset_lists(c.rays, RAY_LISTS);
     const LiveIndex li = live_index(live);
     if (li.wave_empty)
         return;
@@ -971,7 +1010,8 @@ __global__ void k_resolve_skip(PtData d, SegList in, SegList out, SegList next)
     if (li.wave_empty)
         return;
     const int st = li.valid ? next_vertex(d, li.pix, d.flags[li.pix]) : PATH_ENDED;
-    seg_append(out, st == PATH_SKIPPING, li.pix);
+    if (out.slots) // null in the last round: the path ends
+        seg_append(out, st == PATH_SKIPPING, li.pix);
     seg_append(next, st == PATH_AT_VERTEX, li.pix);
 }
 
@@ -1397,7 +1437,9 @@ void path_trace_pass(Ctx& ctx, uint32_t sample_number, uint32_t random_number, h
     // opaque scenes it costs its two kernels (config 1: 9.03 -> 9.32 ms).
     const bool sort_paths = R.shade_order == MIPT_SHADE_ORDER_MATERIAL ||
                             (R.shade_order == MIPT_SHADE_ORDER_AUTO && R.scene_volumes);
-    hipLaunchKernelGGL(k_seg_reset, dim3(1), dim3(SEG_COUNT), 0, s, live[0].counts, 1u);
+    PassCounters counters{qc, nullptr, sort_paths ? R.sort_counts.as<uint32_t>() : nullptr, trace_counters(ctx)};
+    hipLaunchKernelGGL(k_pass_reset, dim3(sort_paths ? blocks_for(2 * SHADE_SORT_COUNTERS, 256) : 1u), dim3(256), 0, s,
+                       counters);
     hipLaunchKernelGGL(k_path_init, dim3(g), dim3(256), 0, s, d, live[0]);
     int cur = 0;
     SegList cur_list = live[0];
@@ -1411,49 +1453,37 @@ void path_trace_pass(Ctx& ctx, uint32_t sample_number, uint32_t random_number, h
             cur_list = cv.train_list; // the paths that go on
         }
         const SegList next = live[cur ^ 1];
-        hipLaunchKernelGGL(k_seg_reset, dim3(1), dim3(4 * SEG_COUNT), 0, s, qc, 4u);
-        hipLaunchKernelGGL(k_seg_reset, dim3(1), dim3(SEG_COUNT), 0, s, next.counts, 1u);
+        counters.next = next.counts;
         const uint32_t* sorted = nullptr;
         if (sort_paths)
         {
             uint32_t* sc = R.sort_counts.as<uint32_t>();
             uint32_t* cursors = sc + (size_t)SHADE_SORT_COUNTERS * SEG_STRIDE;
-            hipLaunchKernelGGL(k_sort_reset, dim3(blocks_for(2 * SHADE_SORT_COUNTERS, 256)), dim3(256), 0, s, sc);
             hipLaunchKernelGGL(k_sort_hist, dim3(g), dim3(256), 0, s, d, cur_list, sc);
             hipLaunchKernelGGL(k_sort_scatter, dim3(g), dim3(256), 0, s, d, cur_list, (const uint32_t*)sc, cursors,
                                R.shade_sorted.as<uint32_t>());
             sorted = R.shade_sorted.as<uint32_t>();
         }
-        hipLaunchKernelGGL(k_shade, dim3(g), dim3(256), 0, s, d, bounce, q, cur_list, sorted, thr_prev);
-        // Shadow (any hit), BSDF-to-light and continuation rays. At bounce 0
-        // every pixel has its rays: one launch per kind, at the single-kind
-        // kernel's higher occupancy. Later bounces carry fewer paths, where a
-        // launch costs about its longest ray's latency: one launch for all.
-        const bool cont_rays = bounce < R.settings.nb_bounces;
-        if (bounce == 0)
-        {
-            trace_any_queue(ctx, R.shadow_rays.as<mipt_ray>(), R.shadow_occ.as<uint8_t>(), q.shadow,
-                            shadow_slots * n, s);
-            trace_closest_queue(ctx, R.bsdf_rays.as<mipt_ray>(), R.bsdf_hits.as<mipt_hit>(), q.bsdf, n, s);
-            if (cont_rays)
-                trace_closest_queue(ctx, R.cont_rays.as<mipt_ray>(), R.cont_hits.as<mipt_hit>(), q.cont, n, s);
-        }
-        else
-        {
-            const TraceQueue tq[3] = {
-                {R.shadow_rays.as<mipt_ray>(), nullptr, R.shadow_occ.as<uint8_t>(), &q.shadow},
-                {R.bsdf_rays.as<mipt_ray>(), R.bsdf_hits.as<mipt_hit>(), nullptr, &q.bsdf},
-                {R.cont_rays.as<mipt_ray>(), R.cont_hits.as<mipt_hit>(), nullptr, &q.cont}};
-            trace_queues(ctx, tq, cont_rays ? 3 : 2, n, s);
-        }
+        hipLaunchKernelGGL(k_shade, dim3(g), dim3(256), 0, s, d, bounce, q, cur_list, sorted, thr_prev,
+                           counters);
+        // Shadow (any hit), BSDF-to-light and continuation rays in one launch:
+        // its end, which lasts as long as its longest ray, is paid once
+        // (bounce 0 in three launches, its rays being many: 659 us for 577 a
+        // 129 x 97 sample, 1.32 ms for 1.26 at 512 x 512, 3.46 ms for 3.26 a
+        // layered one at 960 x 541, 25 us more at 1080p with ReSTIR).
+        const TraceQueue tq[3] = {{R.shadow_rays.as<mipt_ray>(), nullptr, R.shadow_occ.as<uint8_t>(), &q.shadow,
+                                   shadow_slots * n},
+                                  {R.bsdf_rays.as<mipt_ray>(), R.bsdf_hits.as<mipt_hit>(), nullptr, &q.bsdf, n},
+                                  {R.cont_rays.as<mipt_ray>(), R.cont_hits.as<mipt_hit>(), nullptr, &q.cont, n}};
+        trace_queues(ctx, tq, bounce < R.settings.nb_bounces ? 3 : 2, counters.trace, s);
         hipLaunchKernelGGL(k_resolve, dim3(g), dim3(256), 0, s, d, bounce, (const float4*)thr_prev, cur_list, q.skip[0],
-                           next);
+                           next, counters);
         for (int32_t k = 0; k < skip_rounds && bounce < R.settings.nb_bounces; k++)
         {
             const SegList& in = q.skip[k & 1];
-            const SegList& out = q.skip[(k + 1) & 1];
-            hipLaunchKernelGGL(k_seg_reset, dim3(1), dim3(SEG_COUNT), 0, s, out.counts, 1u);
-            trace_closest_queue(ctx, R.cont_rays.as<mipt_ray>(), R.cont_hits.as<mipt_hit>(), in, n, s);
+            const SegList out = k + 1 < skip_rounds ? q.skip[(k + 1) & 1] : SegList{};
+            const TraceQueue skipping{R.cont_rays.as<mipt_ray>(), R.cont_hits.as<mipt_hit>(), nullptr, &in, n};
+            trace_queues(ctx, &skipping, 1, counters.trace + 1 + k, s);
             hipLaunchKernelGGL(k_resolve_skip, dim3(g), dim3(256), 0, s, d, in, out, next);
         }
         cur ^= 1;

@@ -116,6 +116,15 @@ __device__ __forceinline__ void sort6(uint32_t k[6])
     k[5] = max(a2, b2);
 }
 
+// Rays that a wave takes at a time.
+__host__ __device__ __forceinline__ uint32_t wave_batch(uint32_t total, uint32_t waves, uint32_t tile, uint32_t few_waves)
+{
+    if (total >= waves * 64u)
+        return 64u * tile;
+    const uint32_t share = (total + few_waves - 1u) / few_waves;
+    return share <= MIN_BATCH ? MIN_BATCH : (share < 64u ? share : 64u);
+}
+
 // The last GROUPS rays of a wave are traced by eight lanes each, lane c of a
 // group taking child c of a node and triangle c of a leaf. What ends a launch is
 // its longest ray: a round of one lane to a ray issues about 300 instructions
@@ -217,9 +226,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
     // lanes the batches shrink, down to MIN_BATCH rays: more waves, each with
     // fewer different paths through the tree, end sooner.
     const uint32_t waves = gridDim.x * (BLOCK / 64u);
-    uint32_t batch = 64u * a.tile;
-    if (total < waves * 64u)
-        batch = min(64u, max(MIN_BATCH, (total + a.few_waves - 1u) / a.few_waves));
+    const uint32_t batch = wave_batch(total, waves, a.tile, a.few_waves);
     uint32_t next = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64u) + threadIdx.x / 64u) * batch;
     uint32_t batch_end = min(next + batch, total);
     bool more = next < total;
@@ -782,7 +789,7 @@ Scratch trace_scratch(Ctx& ctx, uint32_t threads)
     // per CU), not for this launch's grid, so that launches of different grids
     // on one stream never reallocate the buffer under queued kernels.
     const int spill_depth = ctx.bvh.wide_stack - ctx.trace_cfg.lds_stack;
-    const size_t spill_off = 256; // work counter lives at the front
+    const size_t spill_off = 256; // work counters live at the front
     const size_t columns = std::max<size_t>(threads, (size_t)ctx.cu_count * 32u * 64u);
     size_t spill_bytes = spill_off;
     if (spill_depth > 0)
@@ -804,6 +811,15 @@ TraceArgs trace_args(Ctx& ctx, uint32_t threads, const Scratch& sc)
     a.few_waves = (uint32_t)ctx.cu_count * FEW_WAVES_PER_CU;
     a.last_tri = (uint32_t)ctx.bvh.triangle_count - 1u;
     return a;
+}
+
+// Whether a launch of n rays gives any wave more than the batch that it takes
+// by its index. Without, the work counter is not read and needs no reset: its
+// kernel is 4.5 us of a launch of 61 rays' 15.
+bool takes_from_counter(const TraceArgs& a, unsigned grid, uint32_t n, int block)
+{
+    const uint32_t waves = grid * (uint32_t)(block / 64);
+    return (uint64_t)waves * wave_batch(n, waves, a.tile, a.few_waves) < n;
 }
 
 bool trace_ready(Ctx& ctx)
@@ -835,7 +851,8 @@ void launch(Ctx& ctx, int mode, const mipt_ray* rays, mipt_hit* hits, uint8_t* o
     a.job[0].occluded = occluded;
     a.counts = reinterpret_cast<uint2*>(counts);
     a.n = n;
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
+    if (takes_from_counter(a, l.grid, n, block))
+        hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
     hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(block), 0, stream, a);
     HIP_CHECK(hipGetLastError());
 }
@@ -920,9 +937,16 @@ void trace_closest_noalloc(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint3
     a.job[0].rays = reinterpret_cast<const float4*>(rays);
     a.job[0].hits = reinterpret_cast<int4*>(hits);
     a.n = n;
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
+    if (takes_from_counter(a, grid, n, block))
+        hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
     hipLaunchKernelGGL(l.fn, dim3(grid), dim3(block), 0, stream, a);
     HIP_CHECK(hipGetLastError());
+}
+
+uint32_t* trace_counters(Ctx& ctx)
+{
+    static_assert(TRACE_COUNTERS <= 64, "they lie in front of the spill columns");
+    return trace_scratch(ctx, 0u).counter;
 }
 
 void trace_reserve(Ctx& ctx)
@@ -1011,35 +1035,24 @@ void trace_any(Ctx& ctx, const mipt_ray* rays, uint8_t* occluded, uint32_t n, hi
     launch(ctx, ANY, rays, nullptr, occluded, nullptr, n, stream);
 }
 
-void trace_closest_queue(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, const SegList& queue, uint32_t capacity,
-                         hipStream_t stream)
+void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t* counter, hipStream_t stream)
 {
-    const TraceQueue q{rays, hits, nullptr, &queue};
-    trace_queues(ctx, &q, 1, capacity, stream);
-}
-
-void trace_any_queue(Ctx& ctx, const mipt_ray* rays, uint8_t* occluded, const SegList& queue, uint32_t capacity,
-                     hipStream_t stream)
-{
-    const TraceQueue q{rays, nullptr, occluded, &queue};
-    trace_queues(ctx, &q, 1, capacity, stream);
-}
-
-void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t capacity, hipStream_t stream)
-{
-    if (capacity == 0 || count == 0)
+    uint64_t capacity = 0;
+    for (int k = 0; k < count; k++)
+        capacity += q[k].capacity;
+    if (capacity == 0)
         return;
     if (count > 3)
         fail(MIPT_ERR_INVALID_ARGUMENT, "trace_queues: at most 3 queues");
     if (!trace_ready(ctx))
     {
         for (int k = 0; k < count; k++)
-            hipLaunchKernelGGL(k_all_miss, dim3((capacity + 255) / 256), dim3(256), 0, stream,
-                               reinterpret_cast<int4*>(q[k].hits), q[k].occluded, capacity);
+            hipLaunchKernelGGL(k_all_miss, dim3((q[k].capacity + 255) / 256), dim3(256), 0, stream,
+                               reinterpret_cast<int4*>(q[k].hits), q[k].occluded, q[k].capacity);
         HIP_CHECK(hipGetLastError());
         return;
     }
-    const Launch l = plan(ctx, QUEUED, (uint32_t)std::min<uint64_t>((uint64_t)capacity * count, 0xffffffffull));
+    const Launch l = plan(ctx, QUEUED, (uint32_t)std::min<uint64_t>(capacity, 0xffffffffull));
     const int block = ctx.trace_cfg.block_size;
     const uint32_t threads = l.grid * (uint32_t)block;
     const Scratch sc = trace_scratch(ctx, threads);
@@ -1054,7 +1067,7 @@ void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t capacity, h
         j.counts = q[k].queue->counts;
         j.seg_cap = q[k].queue->seg_cap;
     }
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, sc.counter);
+    a.work_counter = counter;
     hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(block), 0, stream, a);
     HIP_CHECK(hipGetLastError());
 }
