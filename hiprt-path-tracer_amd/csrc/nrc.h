@@ -26,7 +26,7 @@ struct RowSel {
 #ifdef __HIPCC__
     __device__ uint32_t rows() const
     {
-        const uint32_t c = *count;
+        const uint32_t c = count ? *count : limit; // null: as many as the caller's limit
         const uint32_t r = c > offset ? (c - offset + stride - 1) / stride : 0u;
         return r < limit ? r : limit;
     }

@@ -120,14 +120,10 @@ __device__ __forceinline__ void normalized_position(const NrcDev& P, const float
 //
 // k_nrc_inputs reads each record once: the inputs that are not grid features,
 // and the position in the grid's cube.
-__global__ __launch_bounds__(256) void k_nrc_inputs(NrcDev P, const float4* __restrict__ queries, RowSel sel,
-                                                    uint32_t n, uint32_t pad, EncDev E)
+// A row's inputs that are not the grid's; zeros for a row of padding.
+__device__ __forceinline__ void write_inputs(const NrcDev& P, const float4* __restrict__ queries, const RowSel& sel,
+                                             uint32_t row, uint32_t rows, const EncDev& E)
 {
-    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t rows = sel.rows();
-    const uint32_t padded = (rows + pad - 1) / pad * pad;
-    if (row >= n || row >= padded)
-        return;
     uint4* out = reinterpret_cast<uint4*>(E.misc + (size_t)row * NRC_MISC);
     if (row >= rows)
     {
@@ -166,6 +162,17 @@ __global__ __launch_bounds__(256) void k_nrc_inputs(NrcDev P, const float4* __re
     }
 }
 
+__global__ __launch_bounds__(256) void k_nrc_inputs(NrcDev P, const float4* __restrict__ queries, RowSel sel,
+                                                    uint32_t n, uint32_t pad, EncDev E)
+{
+    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t rows = sel.rows();
+    const uint32_t padded = (rows + pad - 1) / pad * pad;
+    if (row >= n || row >= padded)
+        return;
+    write_inputs(P, queries, sel, row, rows, E);
+}
+
 // k_nrc_grid interpolates one level for one row per thread. Workgroups go to
 // the 8 XCDs round-robin, so block b runs on XCD b % 8: it takes level
 // b % 8 for every row first and level b % 8 + 8 after that, so that an XCD's L2
@@ -181,25 +188,9 @@ __global__ __launch_bounds__(256) void k_nrc_inputs(NrcDev P, const float4* __re
 // 1,000,003 rows x 16 levels took 800 us that way.
 constexpr uint32_t NRC_XCDS = 8;
 
-__global__ __launch_bounds__(256) void k_nrc_grid(NrcDev P, RowSel sel, uint32_t n, uint32_t pad, uint32_t chunks,
-                                                  EncDev E)
+// A row's two features of level l at its normalised position.
+__device__ __forceinline__ uint32_t grid_features(const NrcDev& P, int l, const float pos[3])
 {
-    const uint32_t turn = blockIdx.x / NRC_XCDS;
-    const int l = (int)(blockIdx.x % NRC_XCDS + NRC_XCDS * (turn / chunks));
-    const uint32_t row = (turn % chunks) * blockDim.x + threadIdx.x;
-    const uint32_t rows = sel.rows();
-    const uint32_t padded = (rows + pad - 1) / pad * pad;
-    if (l >= P.levels || row >= n || row >= padded)
-        return;
-    uint32_t* out = E.feat + (size_t)l * E.stride + row;
-    if (row >= rows)
-    {
-        *out = 0u;
-        return;
-    }
-    float pos[3];
-    for (int i = 0; i < 3; i++)
-        pos[i] = E.pos[(size_t)i * E.stride + row];
     const uint32_t tmask = (1u << P.log2_table) - 1u;
     const NrcGridLevel& L = P.level[l];
     const uint32_t* table = reinterpret_cast<const uint32_t*>(P.grid_f16) + ((size_t)l << P.log2_table);
@@ -222,7 +213,58 @@ __global__ __launch_bounds__(256) void k_nrc_grid(NrcDev P, RowSel sel, uint32_t
         f0 += w[cc] * (float)__builtin_bit_cast(_Float16, (uint16_t)(pair[cc] & 0xffffu));
         f1 += w[cc] * (float)__builtin_bit_cast(_Float16, (uint16_t)(pair[cc] >> 16));
     }
-    *out = (uint32_t)to_bf16(f0) | ((uint32_t)to_bf16(f1) << 16);
+    return (uint32_t)to_bf16(f0) | ((uint32_t)to_bf16(f1) << 16);
+}
+
+__global__ __launch_bounds__(256) void k_nrc_grid(NrcDev P, RowSel sel, uint32_t n, uint32_t pad, uint32_t chunks,
+                                                  EncDev E)
+{
+    const uint32_t turn = blockIdx.x / NRC_XCDS;
+    const int l = (int)(blockIdx.x % NRC_XCDS + NRC_XCDS * (turn / chunks));
+    const uint32_t row = (turn % chunks) * blockDim.x + threadIdx.x;
+    const uint32_t rows = sel.rows();
+    const uint32_t padded = (rows + pad - 1) / pad * pad;
+    if (l >= P.levels || row >= n || row >= padded)
+        return;
+    uint32_t* out = E.feat + (size_t)l * E.stride + row;
+    if (row >= rows)
+    {
+        *out = 0u;
+        return;
+    }
+    float pos[3];
+    for (int i = 0; i < 3; i++)
+        pos[i] = E.pos[(size_t)i * E.stride + row];
+    *out = grid_features(P, l, pos);
+}
+
+// Both in one launch for few rows: block row l of the levels, then one for the
+// other inputs. A level's block reads the whole record for its position, which
+// costs bandwidth that few rows leave free.
+__global__ __launch_bounds__(256) void k_nrc_encode_few(NrcDev P, const float4* __restrict__ queries, RowSel sel,
+                                                        uint32_t n, uint32_t pad, EncDev E)
+{
+    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
+    const int l = (int)blockIdx.y;
+    const uint32_t rows = sel.rows();
+    const uint32_t padded = (rows + pad - 1) / pad * pad;
+    if (row >= n || row >= padded)
+        return;
+    if (l == P.levels)
+    {
+        write_inputs(P, queries, sel, row, rows, E);
+        return;
+    }
+    uint32_t f = 0u;
+    if (row < rows)
+    {
+        const float4 a = queries[4 * sel.record(row)];
+        const float q[3] = {a.x, a.y, a.z};
+        float pos[3];
+        normalized_position(P, q, pos);
+        f = grid_features(P, l, pos);
+    }
+    E.feat[(size_t)l * E.stride + row] = f;
 }
 
 // Rows of NRC_WIDTH inputs as the network counts them: the grid features,
@@ -256,10 +298,23 @@ EncDev enc_buffer(Nrc& C, uint32_t n)
     return E;
 }
 
+// Up to here one launch encodes faster (16 levels of 2^19, 7 of 2^14): 300 rows
+// 13.9 us an inference for 17.7 in two launches, 5000 rows 18.6 for 19.7; past it
+// the order of levels over the XCDs counts: 20,000 rows 32.9 us (16.4) for 26.6
+// (19.2), 60,000 61.5 us for 43.8, a million 478 us for 463. (The weights' loads
+// going out together then took 1 to 2 us off every one of these.)
+constexpr uint32_t FEW_ROWS = 16384;
+
 void encode_launch(const NrcDev& P, const float* d_queries, const RowSel& sel, uint32_t n, uint32_t pad,
                    const EncDev& E, hipStream_t s)
 {
     const unsigned chunks = (n + 255u) / 256u;
+    if (n <= FEW_ROWS)
+    {
+        hipLaunchKernelGGL(k_nrc_encode_few, dim3(chunks, (unsigned)P.levels + 1u), dim3(256), 0, s, P,
+                           reinterpret_cast<const float4*>(d_queries), sel, n, pad, E);
+        return;
+    }
     const unsigned turns = ((unsigned)P.levels + NRC_XCDS - 1) / NRC_XCDS;
     hipLaunchKernelGGL(k_nrc_inputs, dim3(chunks), dim3(256), 0, s, P, reinterpret_cast<const float4*>(d_queries), sel,
                        n, pad, E);
@@ -312,25 +367,40 @@ __global__ __launch_bounds__(256, 3) void k_nrc_forward(const uint16_t* __restri
 {
     __shared__ uint4 frag[FWD_FRAGS * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t rows = *count < n ? *count : n;
+    const uint32_t rows = count && *count < n ? *count : n;
     if (blockIdx.x * 4u * 64u >= rows)
         return;
-    for (int f = wave; f < FWD_FRAGS; f += 4)
+    // Every weight is on its way before the first is stored: with few rows the
+    // launch is mostly this wait.
+    uint4 v[(FWD_FRAGS + 3) / 4];
+#pragma unroll
+    for (int i = 0; i < (FWD_FRAGS + 3) / 4; i++)
     {
-        const int layer = f < 40 ? f / 8 : 5, mb = f < 40 ? (f % 8) / 2 : 0, s = f % 2;
+        const int f = wave + 4 * i < FWD_FRAGS ? wave + 4 * i : FWD_FRAGS - 1;
+        const int layer = f < 40 ? f / 8 : 5, mb = f < 40 ? (f % 8) / 2 : 0, k_step = f % 2;
         const int g = lane >> 4;
         const uint16_t* w = wt_global + NRC_WOFF(layer) + (size_t)(16 * mb + (lane & 15)) * NRC_WIDTH;
-        uint16_t v[8];
-        for (int j = 0; j < 8; j++)
+        if (i >= 2) // layers past the first: two runs of four weights
         {
-            // layer 0 takes the grid features in k-step 0 and the other inputs in step 1
-            const int slot = 8 * g + j;
-            const int k = layer > 0 ? 16 * (2 * s + (j >> 2)) + 4 * g + (j & 3) : (s == 0 ? slot : 2 * levels + slot);
-            v[j] = k < NRC_WIDTH && (layer > 0 || s == 1 || slot < 2 * levels) ? w[k] : (uint16_t)0;
+            const uint2 lo = *reinterpret_cast<const uint2*>(w + 32 * k_step + 4 * g);
+            const uint2 hi = *reinterpret_cast<const uint2*>(w + 32 * k_step + 16 + 4 * g);
+            v[i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
         }
-        frag[f * 64 + lane] = make_uint4((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16),
-                                         (uint32_t)v[4] | ((uint32_t)v[5] << 16), (uint32_t)v[6] | ((uint32_t)v[7] << 16));
+        else
+        {
+            // layer 0 takes the grid features in k-step 0 and the other inputs
+            // in step 1: pairs of weights, none past either's end
+            const int first = k_step == 0 ? 8 * g : 2 * levels + 8 * g, end = k_step == 0 ? 2 * levels : NRC_WIDTH;
+            uint32_t pair[4];
+            for (int p = 0; p < 4; p++)
+                pair[p] = first + 2 * p < end ? *reinterpret_cast<const uint32_t*>(w + first + 2 * p) : 0u;
+            v[i] = make_uint4(pair[0], pair[1], pair[2], pair[3]);
+        }
     }
+#pragma unroll
+    for (int i = 0; i < (FWD_FRAGS + 3) / 4; i++)
+        if (wave + 4 * i < FWD_FRAGS)
+            frag[(wave + 4 * i) * 64 + lane] = v[i];
     __syncthreads();
     const uint32_t tiles = (rows + 63) / 64;
     const int col = lane & 15, g = lane >> 4;
@@ -1117,12 +1187,6 @@ void nrc_infer(Ctx& ctx, const float* d_queries, const uint32_t* d_count, uint32
     if (n == 0)
         return;
     const EncDev E = enc_buffer(C, n);
-    C.count.reserve(4);
-    if (!d_count)
-    {
-        hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, C.count.as<uint32_t>(), n);
-        d_count = C.count.as<uint32_t>();
-    }
     const NrcDev P = nrc_dev(ctx);
     encode_launch(P, d_queries, RowSel{d_count, 1u, 0u, n}, n, 1u, E, s);
     const unsigned grid = (unsigned)std::min<size_t>(blocks_for((n + 63) / 64, 4), (size_t)ctx.cu_count * 3);
@@ -1138,10 +1202,8 @@ void nrc_encode(Ctx& ctx, const float* d_queries, uint32_t n, uint16_t* d_out, h
         fail(MIPT_ERR_INVALID_ARGUMENT, "radiance cache not configured: call mipt_set_radiance_cache first");
     if (n == 0)
         return;
-    C.count.reserve(4);
-    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, C.count.as<uint32_t>(), n);
     const EncDev E = enc_buffer(C, n);
-    encode_launch(nrc_dev(ctx), d_queries, RowSel{C.count.as<uint32_t>(), 1u, 0u, n}, n, 1u, E, s);
+    encode_launch(nrc_dev(ctx), d_queries, RowSel{nullptr, 1u, 0u, n}, n, 1u, E, s);
     hipLaunchKernelGGL(k_nrc_rows, dim3(blocks_for((size_t)n * (NRC_WIDTH / 2), 256)), dim3(256), 0, s, E,
                        (int)C.settings.grid_levels, n, reinterpret_cast<uint32_t*>(d_out));
     HIP_CHECK(hipGetLastError());
