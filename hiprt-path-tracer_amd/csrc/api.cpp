@@ -197,6 +197,7 @@ void prepare_scene_for_render(Ctx& ctx)
     upload(R.lut_glass_exponent, glass_exponent_data(), 2 * 10 * 11 * 4);
     upload(R.lut_sheen, sheen_ltc_data(), 32 * 32 * 3);
     build_power_alias_table(ctx);
+    build_light_records(ctx);
     R.scene_ready = true;
 }
 

@@ -132,6 +132,8 @@ struct RenderState {
     DeviceBuffer frame_params;  // FrameParams
     uint32_t graph_replays = 0;
     DeviceBuffer areas;         // float[T]
+    DeviceBuffer tri_info;      // float4[T]: unit normal, material index
+    DeviceBuffer light_info;    // float4[4 E]: what a light sample reads of its triangle (pt_device.h)
     DeviceBuffer lut_conductor; // float[128*128]
     DeviceBuffer lut_glossy, lut_glass, lut_glass_inv, lut_thin_glass, lut_glass_exponent, lut_sheen;
     // tables set with mipt_set_lut (MIPT_LUT_GGX_CONDUCTOR .. MIPT_LUT_GGX_THIN_GLASS), empty: the shipped one
@@ -291,6 +293,9 @@ void build_sah_binned(Ctx& ctx);
 
 // bvh_wide.hip: the 6-wide tree from the finished binary one.
 void build_wide(Ctx& ctx);
+
+// pathtrace.hip: fills tri_info and light_info from the scene's geometry.
+void build_light_records(Ctx& ctx);
 
 // trace.hip
 void trace_closest(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint32_t* counts, uint32_t n,

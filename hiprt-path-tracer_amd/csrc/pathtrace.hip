@@ -333,8 +333,9 @@ __device__ __forceinline__ Color restir_final_shading(const PtData& d, uint32_t 
     }
     else
     {
-        emission = d.mats[d.mat_idx[tri]].emission;
-        conv = cos_at_light(pt::normalize(tri_normal_unnormalized(d, tri)), -1.0f * dir);
+        const float4 info = d.tri_info[tri];
+        emission = d.mats[__float_as_int(info.w)].emission;
+        conv = cos_at_light(ld3(info), -1.0f * dir);
         conv /= dist * dist;
     }
     return (((f * ucw) * emission) * cosine) * conv;
@@ -884,9 +885,7 @@ __device__ __forceinline__ Color resolve_ris(const PtData& d, uint32_t pix, uint
                 const Color emission = d.mats[d.mat_idx[hp]].emission;
                 const float4 rb = d.bsdf_rays[2 * (size_t)pix + 1];
                 const f3 dir = pt::mk(rb.x, rb.y, rb.z);
-                f3 a, b, c;
-                tri_verts(d, hp, a, b, c);
-                const f3 hgn = pt::normalize(pt::normalize(pt::cross(b - a, c - a)));
+                const f3 hgn = pt::normalize(ld3(d.tri_info[hp]));
                 const float cos_at_light = pt::maxf_(0.0f, pt::dot(hgn, -1.0f * dir));
                 if (!pt::is_black(emission) && cos_at_light > 0.0f)
                 {
@@ -945,9 +944,7 @@ __device__ __forceinline__ int resolve_path(const PtData& d, int32_t bounce, con
                 const Color emission = d.mats[d.mat_idx[hp]].emission;
                 const float4 rb = d.bsdf_rays[2 * (size_t)pix + 1];
                 const f3 dir = pt::mk(rb.x, rb.y, rb.z);
-                f3 a, b, c;
-                tri_verts(d, hp, a, b, c);
-                const f3 hgn = pt::normalize(pt::normalize(pt::cross(b - a, c - a)));
+                const f3 hgn = pt::normalize(ld3(d.tri_info[hp]));
                 const float cos_l = pt::maxf_(0.0f, pt::dot(hgn, -1.0f * dir));
                 if (!pt::is_black(emission) && cos_l > 0.0f)
                 {
@@ -1231,6 +1228,33 @@ CacheView make_cache_view(Ctx& ctx, uint32_t sample_number, uint32_t every)
     return cv;
 }
 
+__global__ void k_tri_info(PtData d, float4* __restrict__ info, int32_t count)
+{
+    const int32_t t = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t < count)
+        info[t] = st3(pt::normalize(tri_normal_unnormalized(d, t)), __int_as_float(d.mat_idx[t]));
+}
+
+// The operations of sample_one_emissive_triangle_* that depend on the triangle
+// alone (LightUtils.h:163-199), in its order.
+__global__ void k_light_info(PtData d, const int32_t* __restrict__ emissive, float4* __restrict__ info, int32_t count)
+{
+    const int32_t e = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (e >= count)
+        return;
+    const int32_t t = emissive[e];
+    f3 A, B, C;
+    tri_verts(d, t, A, B, C);
+    const f3 AB = B - A, AC = C - A;
+    const f3 nrm = pt::cross(AB, AC);
+    const float len = sqrtf(pt::dot(nrm, nrm));
+    const float area = 0.5f * len;
+    info[4 * (size_t)e] = st3(A, __int_as_float(t));
+    info[4 * (size_t)e + 1] = st3(AB, __int_as_float(d.mat_idx[t]));
+    info[4 * (size_t)e + 2] = st3(AC, area);
+    info[4 * (size_t)e + 3] = st3(pt::vdiv(nrm, len), 1.0f / area);
+}
+
 } // namespace
 
 // MicrofacetRegularization::consistent_tau (MicrofacetRegularization.h:148-161),
@@ -1243,6 +1267,29 @@ float consistent_tau(float tau_0, uint32_t sample_number)
     float p = powf((float)(int)(sample_number + 1), -1.0f / 6.0f);
     float inner = p * sqrtf(four_pi * tau_0 - 1.0f) / (two_pi * tau_0 - 1.0f);
     return 1.0f / (2.0f * pi * (1.0f - cosf(atanf(inner))));
+}
+
+void build_light_records(Ctx& ctx)
+{
+    RenderState& R = ctx.render;
+    if (ctx.triangle_count == 0)
+        return;
+    PtData d{};
+    d.verts = ctx.vertices.as<float>();
+    d.idx = ctx.indices.as<int32_t>();
+    d.mat_idx = ctx.material_indices.as<int32_t>();
+    const int32_t T = ctx.triangle_count, E = ctx.emissive_count;
+    R.tri_info.reserve(sizeof(float4) * (size_t)T);
+    hipLaunchKernelGGL(k_tri_info, dim3(blocks_for((uint32_t)T, 256)), dim3(256), 0, nullptr, d, R.tri_info.as<float4>(),
+                       T);
+    if (E > 0)
+    {
+        R.light_info.reserve(4 * sizeof(float4) * (size_t)E);
+        hipLaunchKernelGGL(k_light_info, dim3(blocks_for((uint32_t)E, 256)), dim3(256), 0, nullptr, d,
+                           ctx.emissive_prims.as<int32_t>(), R.light_info.as<float4>(), E);
+    }
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(nullptr)); // the passes run on any stream
 }
 
 PtData make_pt_data(Ctx& ctx, uint32_t sample_number, uint32_t random_number)
@@ -1260,8 +1307,9 @@ PtData make_pt_data(Ctx& ctx, uint32_t sample_number, uint32_t random_number)
     const bool smooth = R.settings.do_normal_mapping && ctx.has_normals.ptr && ctx.vertex_normals.ptr;
     d.has_normals = smooth ? ctx.has_normals.as<uint8_t>() : nullptr;
     d.vnormals = smooth ? ctx.vertex_normals.as<float>() : nullptr;
-    d.emissive = ctx.emissive_prims.as<int32_t>();
     d.areas = R.areas.as<float>();
+    d.tri_info = R.tri_info.as<float4>();
+    d.light_info = R.light_info.as<float4>();
     d.emissive_count = ctx.emissive_count;
     d.light_base = R.settings.direct_light_sampling_base_strategy;
     d.alias_probas = R.alias_probas.as<float>();

@@ -28,8 +28,15 @@ struct PtData {
     int32_t view_count;
     // graph replay: per-sample values in device memory (null: the fields below)
     const FrameParams* frame;
-    const int32_t* emissive;
     const float* areas;
+    // What a light sample and a target function need of a triangle, laid out
+    // once per scene: a lookup by index, corners and material took four
+    // dependent loads and a root, now one, or two with the emission. A triangle:
+    // unit normal, material index. An emissive triangle, 64 bytes: corner A,
+    // index; AB, material index; AC, area; unit normal, 1 / area. Emission stays
+    // with the materials, which may change.
+    const float4* tri_info;
+    const float4* light_info;
     // smooth shading (get_shading_normal): per-vertex flag and normals, null
     // when the scene has none or do_normal_mapping is 0
     const uint8_t* has_normals;
@@ -341,9 +348,9 @@ __device__ __forceinline__ LightSample sample_emissive_with(const PtData& d, int
             e = d.alias_alias[e];
     }
     LightSample s;
-    s.tri = d.emissive[e];
-    f3 A, B, C;
-    tri_verts(d, s.tri, A, B, C);
+    const float4* l = d.light_info + 4 * (size_t)e;
+    const float4 la = l[0], lb = l[1], lc = l[2], ln = l[3];
+    s.tri = __float_as_int(la.w);
     float r1 = rng();
     float r2 = rng();
     if (r2 > r1)
@@ -356,14 +363,11 @@ __device__ __forceinline__ LightSample sample_emissive_with(const PtData& d, int
         r2 *= 0.5f;
         r1 -= r2;
     }
-    const f3 AB = B - A, AC = C - A;
-    const f3 nrm = pt::cross(AB, AC);
-    const float len = sqrtf(pt::dot(nrm, nrm));
-    s.point = (A + r1 * AB) + r2 * AC;
-    s.normal = pt::vdiv(nrm, len);
-    s.area = 0.5f * len;
-    s.emission = d.mats[d.mat_idx[s.tri]].emission;
-    s.area_pdf = 1.0f / s.area;
+    s.point = (pt::mk(la.x, la.y, la.z) + r1 * pt::mk(lb.x, lb.y, lb.z)) + r2 * pt::mk(lc.x, lc.y, lc.z);
+    s.normal = pt::mk(ln.x, ln.y, ln.z);
+    s.area = lc.w;
+    s.emission = d.mats[__float_as_int(lb.w)].emission;
+    s.area_pdf = ln.w;
     if (strategy == MIPT_LSS_BASE_POWER)
         s.area_pdf *= (luminance(s.emission) * s.area) / d.alias_sum;
     else

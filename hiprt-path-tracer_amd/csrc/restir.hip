@@ -308,8 +308,9 @@ __device__ __forceinline__ float target_function(const PtData& d, const Surface&
     }
     else
     {
-        emission = d.mats[d.mat_idx[tri]].emission;
-        geometry = cos_at_light(pt::normalize(tri_normal_unnormalized(d, tri)), -1.0f * dir);
+        const float4 info = d.tri_info[tri];
+        emission = d.mats[__float_as_int(info.w)].emission;
+        geometry = cos_at_light(ld3(info), -1.0f * dir);
         geometry /= dist * dist;
     }
     return luminance(((f * emission) * cosine) * geometry);
@@ -634,7 +635,7 @@ __global__ __launch_bounds__(256, 3) void k_ic_bsdf(PtData d, RsData r)
             f3 tdir;
             float tdist;
             const float target = target_function(d, s, point, hp, flags, tdir, tdist);
-            const f3 hgn = pt::normalize(pt::normalize(tri_normal_unnormalized(d, hp)));
+            const f3 hgn = pt::normalize(ld3(d.tri_info[hp]));
             const float cos_l = cos_at_light(hgn, -1.0f * dir);
             float lpdf = 0.0f;
             // with presampling, the light sampler is the presampling's
