@@ -196,6 +196,7 @@ def main():
     # launch configuration; null when the configuration differs.
     traffic = None
     l2_hit_rate = None
+    valu_busy = None
     prof_source = None
     for name in ("trace_closest_config2_rinc.json", "trace_closest_config2_rinc_sah.json"):
         prof = os.path.join(ROOT, "profiles", name)
@@ -206,6 +207,7 @@ def main():
         if pj.get("bvh", "LBVH") == bvh_name:
             traffic = pj.get("traffic_bytes_per_launch")
             l2_hit_rate = pj.get("l2_hit_rate")
+            valu_busy = pj.get("valu_issue_busy")
             prof_source = pj.get("summary")
     # What bounds the kernel, from the counters: the algorithmic bytes are an
     # effective bandwidth (they grow with node visits, most of which L2 and
@@ -216,10 +218,12 @@ def main():
     if traffic:
         hbm_gbs = traffic / mean_launch_s / 1e9
         measured = {"hbm_gbs": round(hbm_gbs, 1), "hbm_frac": round(hbm_gbs / HBM_PEAK_GBS, 4),
-                    "traffic_over_algorithmic": round(traffic / (n * b_ray), 4), "l2_hit_rate": l2_hit_rate}
+                    "traffic_over_algorithmic": round(traffic / (n * b_ray), 4), "l2_hit_rate": l2_hit_rate,
+                    "valu_issue_busy": valu_busy}
         limiter = ("hbm bandwidth" if hbm_gbs / HBM_PEAK_GBS >= 0.5 else
-                   f"dependent node-fetch latency and L2 (HBM traffic is {traffic / (n * b_ray) * 100:.1f} % of the "
-                   f"algorithmic bytes and {hbm_gbs / HBM_PEAK_GBS * 100:.1f} % of HBM peak; L2 hit rate "
+                   f"instruction issue: vector units {(valu_busy or 0) * 100:.0f} % busy "
+                   f"(HBM traffic is {traffic / (n * b_ray) * 100:.1f} % of the algorithmic bytes "
+                   f"and {hbm_gbs / HBM_PEAK_GBS * 100:.1f} % of HBM peak; L2 hit rate "
                    f"{(l2_hit_rate or 0) * 100:.1f} %)")
 
     if not args.no_render:
