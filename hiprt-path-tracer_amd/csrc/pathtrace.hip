@@ -750,9 +750,10 @@ __global__ __launch_bounds__(256) void k_sort_scatter(PtData d, SegList live, co
 // or stopped paths) and enqueues the slots of the rays they emitted; keeps
 // the throughput before the vertex for the direct-light estimate. With
 // `sorted`, the list's paths are taken in that order (k_sort_scatter).
-// The layered BSDF with every lobe needs ~140 VGPRs: allowing them (3 waves per
-// SIMD) beats spilling to scratch at 4 waves (11.08 vs 11.74 ms per 1080p
-// config-1 sample).
+// The layered BSDF with every lobe and its view terms fills the 256 VGPRs of two
+// waves a SIMD; three waves spill (314 us a launch for 260, layered materials at
+// 960 x 541). Issue is 59 % busy in the first bounce there, 25 % at 512 x 512 with
+// simple materials: the rest waits on dependent loads.
 __global__ __launch_bounds__(256, 2) void k_shade(PtData d, int32_t bounce, RayQueues q, SegList live,
                                                   const uint32_t* __restrict__ sorted, float4* __restrict__ thr_prev,
                                                   PassCounters c)

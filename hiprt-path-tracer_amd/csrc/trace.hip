@@ -173,12 +173,12 @@ template <int I> __device__ __forceinline__ float byte_of(uint32_t w) { return (
 // the grid busy when the queues are short (a launch costs about the traversal
 // latency of its longest ray, whatever its length).
 //
-// Bound by instruction issue: the vector units are busy 83 % of the time over
+// Bound by instruction issue: the vector units are busy 85 % of the time over
 // 2,073,600 incoherent rays on 1,040,384 triangles (17 nodes and 4.6 triangles
 // a ray, 45 of 64 lanes at a node in a mean node step, about 210 instructions;
 // the 64-byte record costs 4 loads, the L2 serves 2.4 GB). A binary tree of
 // 64-byte nodes with float boxes took 43.8 nodes a ray, and the same 4
-// loads for each: 910 us, now 514 us; 700,001 shadow rays 564 us, now 300 us.
+// loads for each: 910 us, now 506 us; 700,001 shadow rays 564 us, now 296 us.
 // Reading the nodes by groups of four lanes through LDS (a quarter of the cache
 // accesses) cost more in instructions and LDS than it saved (680 us), a second
 // put-aside leaf per lane let culling lag (552 us).
