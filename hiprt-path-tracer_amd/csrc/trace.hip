@@ -14,7 +14,10 @@
 //     wait until LEAF_LANES of them are there (or no lane is at a node): the
 //     wave then pays for the triangle test once for many;
 //   * the per-lane stack lives in LDS, laid out [depth][lane]; entries
-//     deeper than the LDS stack spill to a per-thread global array;
+//     deeper than the LDS stack spill to a per-thread global array, without
+//     their distances: few do, and the arrays, sized for the deepest stack a
+//     tree allows, are half as large (two million bounce rays: 509 us a launch,
+//     511 us with the distances);
 //   * a persistent grid sized from occupancy; each wave takes batches of rays
 //     from a global counter and hands them to lanes whose ray is done, once
 //     REFILL_LANES of them are. When none are left, its last GROUPS rays get
@@ -69,6 +72,8 @@ constexpr int REFILL_LANES = 16;
 constexpr uint32_t MIN_BATCH = 8;
 constexpr uint32_t FEW_WAVES_PER_CU = 12;
 
+constexpr int MAX_LDS_STACK = 32;
+
 constexpr int32_t IDLE = 0x7fffffff; // no node or leaf to visit (node indices stay below)
 
 // A ray set: `rays` indexed by slot; with `occluded` it is traced any-hit
@@ -89,7 +94,7 @@ struct TraceArgs {
     QueueJob job[3];
     uint2* counts;      // nodes and triangles per ray (instrumented variant)
     uint32_t n;         // rays without a queue
-    uint2* spill;       // stack entries past the LDS ones, a column per thread
+    uint32_t* spill;    // references of stack entries past the LDS ones, a column per thread
     uint32_t spill_stride;
     uint32_t* work_counter;
     uint32_t tile;
@@ -429,7 +434,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
                         if (top - k < STACK)
                             stack[(top - k) * BLOCK + threadIdx.x] = e;
                         else
-                            a.spill[(size_t)(top - k - STACK) * a.spill_stride + gtid] = e;
+                            a.spill[(size_t)(top - k - STACK) * a.spill_stride + gtid] = e.y;
                     }
             }
             cur = IDLE;
@@ -454,11 +459,11 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
         if (cur == IDLE && sp > 0)
         {
             sp--;
-            uint2 e;
+            uint2 e = make_uint2(0u, 0u); // a spilled entry: distance 0, always in reach
             if (sp < STACK)
                 e = stack[sp * BLOCK + threadIdx.x];
             else
-                e = a.spill[(size_t)(sp - STACK) * a.spill_stride + gtid];
+                e.y = a.spill[(size_t)(sp - STACK) * a.spill_stride + gtid];
             // the entry's distance is already widened downwards
             if (__uint_as_float(e.x) <= best_t * WIDEN_HI)
                 cur = (int32_t)e.y;
@@ -535,7 +540,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
     }
     // the ray's stack stays in its owner's columns
     uint2* const column = stack + ((threadIdx.x & ~63u) + (uint32_t)owner);
-    uint2* const deep = a.spill + (gtid - lane + (uint32_t)owner);
+    uint32_t* const deep = a.spill + (gtid - lane + (uint32_t)owner);
     const bool bx = inv_nx < 0.0f, by = inv_ny < 0.0f, bz = inv_nz < 0.0f;
     // children 4 and 5 have their planes in the tail words: entry planes in
     // bytes 0 and 1, exit planes in bytes 2 and 3, swapped by the direction
@@ -566,8 +571,10 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
             {
                 const int at = sp - 1 - (int)c;
                 uint2 e = make_uint2(0x7f800001u, 0u); // NaN: out of reach
-                if (at >= 0)
-                    e = at < STACK ? column[at * BLOCK] : deep[(size_t)(at - STACK) * a.spill_stride];
+                if (at >= STACK)
+                    e = make_uint2(0u, deep[(size_t)(at - STACK) * a.spill_stride]);
+                else if (at >= 0)
+                    e = column[at * BLOCK];
                 const uint32_t in_reach = group_ballot(__uint_as_float(e.x) <= best_t * WIDEN_HI, group_shift);
                 const int first = in_reach ? __ffs((int)in_reach) - 1 : 0;
                 const int32_t ref = __shfl((int32_t)e.y, (int)group_shift + first);
@@ -670,7 +677,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a)
                 if (at < STACK)
                     column[at * BLOCK] = e;
                 else
-                    deep[(size_t)(at - STACK) * a.spill_stride] = e;
+                    deep[(size_t)(at - STACK) * a.spill_stride] = e.y;
             }
             stack_fence();
             cur = IDLE;
@@ -769,10 +776,10 @@ unsigned persistent_grid(Ctx& ctx, const void* fn, uint32_t n)
     return (unsigned)(g ? g : 1);
 }
 
-Launch plan(Ctx& ctx, int mode, uint32_t n)
+Launch plan(Ctx& ctx, int mode, uint32_t n, int lds_stack)
 {
     Launch l;
-    l.fn = pick(ctx.trace_cfg.block_size, ctx.trace_cfg.lds_stack, mode);
+    l.fn = pick(ctx.trace_cfg.block_size, lds_stack, mode);
     l.grid = persistent_grid(ctx, reinterpret_cast<const void*>(l.fn), n);
     return l;
 }
@@ -780,7 +787,7 @@ Launch plan(Ctx& ctx, int mode, uint32_t n)
 // Work counter and spill columns of a persistent grid of `threads` threads.
 struct Scratch {
     uint32_t* counter;
-    uint2* spill;
+    uint32_t* spill;
 };
 
 Scratch trace_scratch(Ctx& ctx, uint32_t threads)
@@ -793,10 +800,10 @@ Scratch trace_scratch(Ctx& ctx, uint32_t threads)
     const size_t columns = std::max<size_t>(threads, (size_t)ctx.cu_count * 32u * 64u);
     size_t spill_bytes = spill_off;
     if (spill_depth > 0)
-        spill_bytes = spill_off + sizeof(uint2) * (size_t)spill_depth * columns;
+        spill_bytes = spill_off + sizeof(uint32_t) * (size_t)spill_depth * columns;
     ctx.spill.reserve(spill_bytes);
     return Scratch{ctx.spill.as<uint32_t>(),
-                   reinterpret_cast<uint2*>(reinterpret_cast<char*>(ctx.spill.ptr) + spill_off)};
+                   reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ctx.spill.ptr) + spill_off)};
 }
 
 TraceArgs trace_args(Ctx& ctx, uint32_t threads, const Scratch& sc)
@@ -841,7 +848,7 @@ void launch(Ctx& ctx, int mode, const mipt_ray* rays, mipt_hit* hits, uint8_t* o
         HIP_CHECK(hipGetLastError());
         return;
     }
-    const Launch l = plan(ctx, mode, n);
+    const Launch l = plan(ctx, mode, n, ctx.trace_cfg.lds_stack);
     const int block = ctx.trace_cfg.block_size;
     const uint32_t threads = l.grid * (uint32_t)block;
     const Scratch sc = trace_scratch(ctx, threads);
@@ -910,29 +917,39 @@ void trace_closest_noalloc(Ctx& ctx, const mipt_ray* rays, mipt_hit* hits, uint3
         HIP_CHECK(hipGetLastError());
         return;
     }
-    const Launch l = plan(ctx, CLOSEST, n);
     const int block = ctx.trace_cfg.block_size;
-    // Spill columns of the persistent grid: when the tree is deep enough
-    // that the whole grid's columns do not fit, the grid shrinks to the
-    // blocks whose columns do (every wave takes rays from the work counter,
-    // so fewer blocks trace the same rays).
-    const int spill_depth = std::max(0, ctx.bvh.wide_stack - ctx.trace_cfg.lds_stack);
+    // Spill columns of the persistent grid: where the whole grid's columns do
+    // not fit, it shrinks to the blocks whose columns do (every wave takes
+    // rays from the work counter, so fewer blocks trace the same rays), or
+    // more of the stack stays in LDS: of the LDS depths from the context's on,
+    // the one that leaves the most blocks. 1,040,384 triangles, 2,073,600
+    // bounce rays, stacks of 57 (SAH) and 59 entries: 581 and 690 us with 16 and
+    // 24 LDS entries (plain call: 509 and 561), where spilled entries of 8 bytes
+    // behind 8 LDS ones left 668 and 642 of 3072 blocks: 1098 and 1366 us.
     const size_t room = MIPT_TRACE_NOALLOC_SCRATCH_BYTES - NOALLOC_COUNTER_BYTES;
-    unsigned grid = l.grid;
-    if (spill_depth > 0)
+    Launch l{nullptr, 0u};
+    for (int lds = ctx.trace_cfg.lds_stack; lds <= MAX_LDS_STACK; lds += 8)
     {
-        const size_t per_block = sizeof(uint2) * (size_t)spill_depth * (size_t)block;
-        const size_t fit = room / per_block;
-        if (fit == 0)
-            fail(MIPT_ERR_INVALID_ARGUMENT,
-                 "mipt_trace_closest_noalloc: a BVH of " + std::to_string(ctx.bvh.wide_stack) +
-                     " stack entries needs more than the " + std::to_string(MIPT_TRACE_NOALLOC_SCRATCH_BYTES) +
-                     "-byte scratch for one block's spill stack");
-        grid = (unsigned)std::min<size_t>(grid, fit);
+        Launch c = plan(ctx, CLOSEST, n, lds);
+        const unsigned whole = c.grid;
+        const size_t per_block =
+            sizeof(uint32_t) * (size_t)std::max(0, ctx.bvh.wide_stack - lds) * (size_t)block;
+        if (per_block > 0)
+            c.grid = (unsigned)std::min<size_t>(whole, room / per_block);
+        if (c.grid > l.grid)
+            l = c;
+        if (c.grid == whole)
+            break;
     }
+    if (l.grid == 0)
+        fail(MIPT_ERR_INVALID_ARGUMENT,
+             "mipt_trace_closest_noalloc: a BVH of " + std::to_string(ctx.bvh.wide_stack) +
+                 " stack entries needs more than the " + std::to_string(MIPT_TRACE_NOALLOC_SCRATCH_BYTES) +
+                 "-byte scratch for one block's spill stack");
+    const unsigned grid = l.grid;
     const uint32_t threads = grid * (uint32_t)block;
     const Scratch sc{reinterpret_cast<uint32_t*>(base),
-                     reinterpret_cast<uint2*>(reinterpret_cast<char*>(base) + NOALLOC_COUNTER_BYTES)};
+                     reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(base) + NOALLOC_COUNTER_BYTES)};
     TraceArgs a = trace_args(ctx, threads, sc);
     a.job[0].rays = reinterpret_cast<const float4*>(rays);
     a.job[0].hits = reinterpret_cast<int4*>(hits);
@@ -1052,7 +1069,7 @@ void trace_queues(Ctx& ctx, const TraceQueue* q, int count, uint32_t* counter, h
         HIP_CHECK(hipGetLastError());
         return;
     }
-    const Launch l = plan(ctx, QUEUED, (uint32_t)std::min<uint64_t>(capacity, 0xffffffffull));
+    const Launch l = plan(ctx, QUEUED, (uint32_t)std::min<uint64_t>(capacity, 0xffffffffull), ctx.trace_cfg.lds_stack);
     const int block = ctx.trace_cfg.block_size;
     const uint32_t threads = l.grid * (uint32_t)block;
     const Scratch sc = trace_scratch(ctx, threads);

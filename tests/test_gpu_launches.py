@@ -1,0 +1,121 @@
+"""What calls launch, read from a HIP graph that captures them (so the numbers
+are exact): the size of a grid, and how many kernels a call takes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_mod():
+    import torch
+
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    return torch
+
+
+class _Dim3(C.Structure):
+    _fields_ = [("x", C.c_uint32), ("y", C.c_uint32), ("z", C.c_uint32)]
+
+
+class _KernelNodeParams(C.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", _Dim3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", _Dim3),
+                ("params", C.c_void_p), ("lds", C.c_uint)]
+
+
+def _hip():
+    """The HIP runtime that the process has loaded."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    return C.CDLL(path)
+
+
+def kernels(torch, call):
+    """(blocks, threads a block) of every kernel that call(stream) launches, its buffers being
+    allocated by an earlier call."""
+    hip = _hip()
+    stream = torch.cuda.Stream()
+    s = C.c_void_p(stream.cuda_stream)
+    graph = C.c_void_p()
+    torch.cuda.synchronize()
+    assert hip.hipStreamBeginCapture(s, 2) == 0  # relaxed
+    try:
+        call(stream.cuda_stream)
+    finally:
+        assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+    count = C.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+    nodes = (C.c_void_p * max(count.value, 1))()
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(count)) == 0
+    out = []
+    for k in range(count.value):
+        node, kind = C.c_void_p(nodes[k]), C.c_int()
+        assert hip.hipGraphNodeGetType(node, C.byref(kind)) == 0
+        assert kind.value == 0, "a node that is not a kernel"
+        p = _KernelNodeParams()
+        assert hip.hipGraphKernelNodeGetParams(node, C.byref(p)) == 0
+        out.append((p.grid.x * p.grid.y * p.grid.z, p.block.x * p.block.y * p.block.z))
+    assert hip.hipGraphDestroy(graph) == 0
+    return out
+
+
+@pytest.mark.parametrize("builder", ["lbvh", "sah"])
+def test_noalloc_grid(mipt_mod, torch_mod, scene2, builder):
+    """The no-allocation closest hit keeps the GPU as busy as its scratch allows: on the
+    1,040,384-triangle scene, whose stacks do not fit for the whole grid, it
+    runs at least 0.45 of the plain call's threads (0.5 with a 24-entry LDS stack; one of 8
+    entries left it 0.22 and made it slower than a binary tree), with the same hits."""
+    n = 1920 * 1080
+    ctx = mipt_mod.Context(0)
+    ctx.set_scene(scene2)
+    ctx.build_bvh(mipt_mod.MIPT_BVH_SAH_BINNED if builder == "sah" else mipt_mod.MIPT_BVH_LBVH)
+    d_rays, d_rng = mipt_mod.empty_device(32 * n), mipt_mod.empty_device(4 * n)
+    d_hits, d_hits2 = mipt_mod.empty_device(16 * n), mipt_mod.empty_device(16 * n)
+    ctx.camera_rays(scene2.camera, 1920, 1080, 0, mipt_mod.host_random_number(0), 0, d_rays, d_rng)
+    ctx.trace_closest(d_rays, d_hits, n)
+    ctx.trace_closest_noalloc(d_rays, d_hits2, n)
+    torch_mod.cuda.synchronize()
+    assert torch_mod.equal(d_hits, d_hits2)
+    threads = [max(g * b for g, b in kernels(torch_mod, lambda s: fn(d_rays, d_hits, n, s)))
+               for fn in (ctx.trace_closest, ctx.trace_closest_noalloc)]
+    print(f"{builder}: {threads[0]} threads, without allocation {threads[1]}")
+    assert threads[1] >= 0.45 * threads[0]
+    ctx.close()
+
+
+@pytest.mark.parametrize("lds", [8, 16, 24, 32])
+@pytest.mark.parametrize("block", [64, 128, 256])
+def test_noalloc_deep_stacks(mipt_mod, oracle_mod, torch_mod, block, lds):
+    """Slivers through one point, whose boxes all overlap: stacks past the LDS entries at every
+    depth that the context or the no-allocation call takes, hits against brute force."""
+    rng = np.random.default_rng(5)
+    k, n = 3000, 3000
+    d = rng.normal(size=(k, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    off = rng.normal(size=(k, 3)) * 0.02
+    V = np.stack([-3 * d + off, 3 * d + off, 3 * d - off + rng.normal(size=(k, 3)) * 0.05], 1).astype(np.float32)
+    V = V.reshape(-1, 3)
+    I = np.arange(3 * k, dtype=np.int32).reshape(k, 3)
+    rays = np.zeros(n, mipt_mod.RAY_DTYPE)
+    o = rng.normal(size=(n, 3))
+    rays["o"] = 4 * o / np.linalg.norm(o, axis=1, keepdims=True)
+    aim = rng.normal(size=(n, 3)) * 0.3 - rays["o"]
+    rays["d"] = aim / np.linalg.norm(aim, axis=1, keepdims=True)
+    rays["last_prim"] = -1
+    rays["tmax"] = np.inf
+    want = oracle_mod.trace_brute(V, I, rays)
+    ctx = mipt_mod.Context(0)
+    ctx.set_scene(mipt_mod.Scene(V, I))
+    ctx.build_bvh()
+    ctx.set_trace_config(block, lds)
+    d_rays, d_hits = mipt_mod.to_device(rays), mipt_mod.empty_device(16 * n)
+    for fn in (ctx.trace_closest, ctx.trace_closest_noalloc):
+        d_hits.zero_()
+        fn(d_rays, d_hits, n)
+        torch_mod.cuda.synchronize()
+        got = mipt_mod.from_device(d_hits, mipt_mod.HIT_DTYPE)[:n]
+        assert np.array_equal(got["prim"], want["prim"])
+        assert np.array_equal(got["t"].view(np.uint32), want["t"].view(np.uint32))
+    ctx.close()
