@@ -28,10 +28,14 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // Rows from which the grid gradient is binned instead of added by global
-// atomics. A whole training step, atomics against bins: 2048 rows 214 / 234 us
-// at 2^19 entries a level, 99 / 101 us at 2^14; 4096 rows 247 / 238 and 128 / 113;
-// 65,536 rows 1146 / 489 and 1006 / 309.
-constexpr uint32_t GRAD_BIN_MIN_ROWS = 4096;
+// atomics: the bins' five launches cost the same with few levels as with many,
+// the atomics by the level. A whole training step, atomics against bins, tables
+// of 2^14 (2^19) entries a level: 16 levels 3000 rows 121 / 116 us (237 / 236),
+// 4096 rows 138 / 117 (255 / 238); 7 levels 4096 rows 106 / 112 (143 / 152),
+// 6000 rows 125 / 118 (163 / 154); 3 levels 6000 rows 109 / 114 (124 / 132), 8192 rows
+// 123 / 117 (137 / 134); 1 level 10,000 rows 123 / 132 (126 / 141), 16,384 rows
+// 132 / 125 (136 / 134). 65,536 rows of 16 levels: 1188 / 314 (1384 / 492).
+constexpr uint32_t grad_bin_min_rows(uint32_t levels) { return std::max(4096u, 3072u + 12288u / levels); }
 constexpr uint32_t GRAD_MAX_RANGES = 1u << (24 - 13); // per level (log2_table is at most 24)
 constexpr uint32_t GRAD_BIN_ROWS = 1u << 16;          // rows binned at a time: 100 MB of updates at most
 constexpr int TILE_LD = NRC_WIDTH + 8; // LDS row stride (bf16) of an activation tile
@@ -879,7 +883,7 @@ void grid_grad_launch(Nrc& C, const NrcDev& P, const NrcTrainDev& T, uint32_t ba
 {
     const int lt = P.log2_table;
     const unsigned levels = (unsigned)P.levels;
-    if (batch < GRAD_BIN_MIN_ROWS || lt < 10)
+    if (batch < grad_bin_min_rows(levels) || lt < 10)
     {
         hipLaunchKernelGGL(k_nrc_grid_grad, dim3((batch + 127u) / 128u, levels), dim3(128), 0, s, P, T);
         return;

@@ -119,3 +119,22 @@ def test_noalloc_deep_stacks(mipt_mod, oracle_mod, torch_mod, block, lds):
         assert np.array_equal(got["prim"], want["prim"])
         assert np.array_equal(got["t"].view(np.uint32), want["t"].view(np.uint32))
     ctx.close()
+
+
+def _train_kernels(mipt_mod, torch_mod, scene, levels, log2_table, rows):
+    ctx = mipt_mod.Context(0)
+    ctx.set_scene(scene)
+    ctx.set_radiance_cache(mipt_mod.default_radiance_cache_settings(grid_levels=levels, grid_log2_table=log2_table))
+    q, y = torch_mod.rand(rows, 16, device="cuda"), torch_mod.rand(rows, 4, device="cuda")
+    ctx.cache_train_step(q, y, rows, False)
+    found = kernels(torch_mod, lambda s: ctx.cache_train_step(q, y, rows, False, s))
+    ctx.close()
+    return len(found)
+
+
+@pytest.mark.parametrize("levels,rows", [(16, 4096), (7, 4827), (3, 7168), (2, 9216), (1, 15360)])
+def test_gradient_bins_start_where_they_pay(mipt_mod, torch_mod, scene1, levels, rows):
+    """The grid gradient's bins take four launches more than its atomics, which few
+    levels repay later: two levels of 4096 rows took 113 us binned and 92 us with atomics."""
+    few, many = (_train_kernels(mipt_mod, torch_mod, scene1, levels, 14, n) for n in (rows - 1, rows))
+    assert many == few + 4

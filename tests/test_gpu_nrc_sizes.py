@@ -4,8 +4,8 @@ working.
 - Inference: a row's answer does not depend on the rows beside it, so row
   counts around a wave's 64 rows and a block's 256 give the same bits as one
   large call.
-- Grid and weight gradients: from 4096 rows on the corner updates are binned,
-  below they are added by atomics. A batch's gradient is the row-weighted mean
+- Grid and weight gradients: from 4096 rows on (16 levels; 15,360 with one) the corner
+  updates are binned, below they are added by atomics. A batch's gradient is the row-weighted mean
   of its halves' (the terms are the same 32-bit products, up to the scale
   1 / (3 rows) and the order of the sums): with at most 2^17 addends of random
   sign per entry the two agree to 1e-5 in the 2-norm.
@@ -39,8 +39,11 @@ def test_rows_are_independent(mipt_mod, torch_mod, scene1, levels):
     ctx.close()
 
 
-@pytest.mark.parametrize("levels,log2_table", [(16, 9), (16, 10), (7, 14), (16, 15), (16, 19), (3, 21)])
-@pytest.mark.parametrize("rows", [4096, 4097, 6000])
+FEW_LEVELS = [(4827, 7, 14), (7168, 3, 21), (15360, 1, 10)]  # the first binned batch of 7, 3 and 1 levels
+
+
+@pytest.mark.parametrize("rows,levels,log2_table", [(r, *c) for c in [(16, 9), (16, 10), (7, 14), (16, 15), (16, 19), (3, 21)]
+                                                    for r in (4096, 4097, 6000)] + FEW_LEVELS)
 def test_binned_gradient_is_the_mean_of_its_halves(mipt_mod, torch_mod, scene1, rows, levels, log2_table):
     rng = np.random.default_rng(rows + log2_table)
     ctx, cs = _make(mipt_mod, scene1, grid_levels=levels, grid_log2_table=log2_table)
