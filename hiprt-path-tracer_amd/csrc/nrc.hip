@@ -707,9 +707,11 @@ __global__ __launch_bounds__(128) void k_nrc_grid_grad(NrcDev P, NrcTrainDev T)
 }
 
 // The same without global atomics on the gradient, which the memory side serves at
-// 18 G/s however they are ordered: the corner updates are binned by ranges
-// of 2^log2_e table entries of a level (count, prefix sums, scatter), then a
-// block adds the updates of one range in LDS and writes the range once.
+// 18 G/s however they are ordered, and slower where they meet in few entries
+// (a step of 65,536 rows, 16 levels: 12.9 ms at 2^4 entries a level, 1.25 ms at
+// 2^9; binned 0.32 ms both): the corner updates are binned by ranges of 2^log2_e
+// table entries of a level (count, prefix sums, scatter), then a block adds the
+// updates of one range in LDS and writes the range once.
 struct GradBins {
     uint32_t* counts;  // [levels][ranges]
     uint32_t* cursors; // [levels][ranges]: first free place of each bin
@@ -720,6 +722,7 @@ struct GradBins {
     uint32_t places;   // rows * 8: places of a level
     uint32_t first_row, rows; // this pass's rows
     int log2_e;
+    uint32_t ranges;   // per level
 };
 
 // The 8 corners of a row at a level.
@@ -753,7 +756,7 @@ __global__ __launch_bounds__(GRAD_BIN_BLOCK) void k_nrc_bin(NrcDev P, NrcTrainDe
 {
     __shared__ uint32_t hist[GRAD_MAX_RANGES], base[GRAD_MAX_RANGES];
     const int l = (int)blockIdx.y;
-    const uint32_t ranges = 1u << (P.log2_table - B.log2_e);
+    const uint32_t ranges = B.ranges;
     const uint32_t rows = T.sel.rows();
     const uint32_t end = min(B.first_row + B.rows, rows);
     const uint32_t row = B.first_row + blockIdx.x * GRAD_BIN_BLOCK + threadIdx.x;
@@ -842,7 +845,7 @@ __global__ __launch_bounds__(GRAD_ADD_BLOCK) void k_nrc_bin_add(NrcDev P, NrcTra
         return;
     const uint2 item = B.items[blockIdx.x];
     const uint32_t bin = item.x; // level * ranges + range
-    const uint32_t ranges = 1u << (P.log2_table - LOG2_E);
+    const uint32_t ranges = B.ranges;
     const int l = (int)(bin / ranges);
     const uint32_t count = B.counts[bin], end = min(item.y + GRAD_SHARE, count);
     for (uint32_t i = threadIdx.x; i < ENTRIES / 2; i += GRAD_ADD_BLOCK)
@@ -883,15 +886,23 @@ void grid_grad_launch(Nrc& C, const NrcDev& P, const NrcTrainDev& T, uint32_t ba
 {
     const int lt = P.log2_table;
     const unsigned levels = (unsigned)P.levels;
-    if (batch < grad_bin_min_rows(levels) || lt < 10)
+    if (batch < grad_bin_min_rows(levels))
     {
         hipLaunchKernelGGL(k_nrc_grid_grad, dim3((batch + 127u) / 128u, levels), dim3(128), 0, s, P, T);
         return;
     }
     GradBins B{};
+    // Both range sizes are within 6 % of each other from 2^15 to 2^19 entries
+    // (16 levels of 37,000 rows, 2^10 against 2^13: 264 / 273 us and 381 / 376).
+    // Below, the larger one leaves a level few blocks and sums in LDS that no
+    // update reaches (2^14: 238 / 273); above, the smaller one splits the updates over
+    // more ranges than there are blocks at a time (2^21: 792 / 745), and a level of
+    // 2^24 has as many ranges of 2^13 as the histograms hold. A table smaller than a
+    // range is one range, whose other sums stay 0.
     B.log2_e = lt <= 14 ? 10 : 13;
-    const uint32_t ranges = 1u << (lt - B.log2_e);
+    const uint32_t ranges = lt > B.log2_e ? 1u << (lt - B.log2_e) : 1u;
     const uint32_t pass = std::min<uint32_t>(batch, GRAD_BIN_ROWS);
+    B.ranges = ranges;
     const size_t bins = (size_t)levels * ranges, places = (size_t)8 * pass;
     const size_t max_items = bins + places * levels / GRAD_SHARE;
     C.grad_bins.reserve(8 * bins + 12 * places * levels + 8 * max_items + 8);

@@ -138,3 +138,11 @@ def test_gradient_bins_start_where_they_pay(mipt_mod, torch_mod, scene1, levels,
     levels repay later: two levels of 4096 rows took 113 us binned and 92 us with atomics."""
     few, many = (_train_kernels(mipt_mod, torch_mod, scene1, levels, 14, n) for n in (rows - 1, rows))
     assert many == few + 4
+
+
+@pytest.mark.parametrize("log2_table", [4, 9, 10])
+def test_small_tables_are_binned(mipt_mod, torch_mod, scene1, log2_table):
+    """Tables of any size are binned: atomics meet in the few entries of a small one (65,536
+    rows: 12.9 ms at 2^4 entries a level, 1.25 ms at 2^9)."""
+    few, many = (_train_kernels(mipt_mod, torch_mod, scene1, 16, log2_table, n) for n in (4095, 4096))
+    assert many == few + 4

@@ -42,7 +42,7 @@ def test_rows_are_independent(mipt_mod, torch_mod, scene1, levels):
 FEW_LEVELS = [(4827, 7, 14), (7168, 3, 21), (15360, 1, 10)]  # the first binned batch of 7, 3 and 1 levels
 
 
-@pytest.mark.parametrize("rows,levels,log2_table", [(r, *c) for c in [(16, 9), (16, 10), (7, 14), (16, 15), (16, 19), (3, 21)]
+@pytest.mark.parametrize("rows,levels,log2_table", [(r, *c) for c in [(16, 4), (16, 7), (16, 9), (16, 10), (7, 14), (16, 15), (16, 19), (3, 21)]
                                                     for r in (4096, 4097, 6000)] + FEW_LEVELS)
 def test_binned_gradient_is_the_mean_of_its_halves(mipt_mod, torch_mod, scene1, rows, levels, log2_table):
     rng = np.random.default_rng(rows + log2_table)
