@@ -118,30 +118,15 @@ __device__ __forceinline__ void normalized_position(const NrcDev& P, const float
         pos[a] = fminf(1.0f, fmaxf(0.0f, (q[a] - P.bmin[a]) * P.inv_extent));
 }
 
-// Query record (16 floats): position, direction, normal, roughness, albedo.
-// Encodes the selected rows into E rows [0, rows) and zero-fills the rows up
-// to the next multiple of pad (at most n rows in all), in two kernels.
-//
-// k_nrc_inputs reads each record once: the inputs that are not grid features,
-// and the position in the grid's cube.
-// A row's inputs that are not the grid's; zeros for a row of padding.
-__device__ __forceinline__ void write_inputs(const NrcDev& P, const float4* __restrict__ queries, const RowSel& sel,
-                                             uint32_t row, uint32_t rows, const EncDev& E)
+// The inputs of a query record (16 floats: position, direction, normal,
+// roughness, albedo) that are not the grid's, in pairs, and its position in the
+// grid's cube.
+__device__ __forceinline__ void record_inputs(const NrcDev& P, const float4* __restrict__ queries, size_t rec,
+                                              uint32_t pairs[NRC_MISC / 2], float pos[3])
 {
-    uint4* out = reinterpret_cast<uint4*>(E.misc + (size_t)row * NRC_MISC);
-    if (row >= rows)
-    {
-        for (int k = 0; k < NRC_MISC / 8; k++)
-            out[k] = make_uint4(0u, 0u, 0u, 0u);
-        return;
-    }
-    const size_t rec = sel.record(row);
     const float4 a = queries[4 * rec], b = queries[4 * rec + 1], c = queries[4 * rec + 2], d = queries[4 * rec + 3];
     const float q[16] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
-    float pos[3];
     normalized_position(P, q, pos);
-    for (int i = 0; i < 3; i++)
-        E.pos[(size_t)i * E.stride + row] = pos[i];
     uint16_t m[NRC_MISC];
     float u, v;
     oct_uv(q[3], q[4], q[5], u, v);
@@ -157,15 +142,32 @@ __device__ __forceinline__ void write_inputs(const NrcDev& P, const float4* __re
     m[5 * NRC_BLOB + 3] = to_bf16(1.0f);
     for (int k = 5 * NRC_BLOB + 4; k < NRC_MISC; k++)
         m[k] = 0;
-    for (int k = 0; k < NRC_MISC / 8; k++)
-    {
-        uint32_t w[4];
-        for (int i = 0; i < 4; i++)
-            w[i] = (uint32_t)m[8 * k + 2 * i] | ((uint32_t)m[8 * k + 2 * i + 1] << 16);
-        out[k] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
+    for (int k = 0; k < NRC_MISC / 2; k++)
+        pairs[k] = (uint32_t)m[2 * k] | ((uint32_t)m[2 * k + 1] << 16);
 }
 
+// A row's inputs that are not the grid's; zeros for a row of padding.
+__device__ __forceinline__ void write_inputs(const NrcDev& P, const float4* __restrict__ queries, const RowSel& sel,
+                                             uint32_t row, uint32_t rows, const EncDev& E)
+{
+    uint4* out = reinterpret_cast<uint4*>(E.misc + (size_t)row * NRC_MISC);
+    uint32_t m[NRC_MISC / 2] = {};
+    if (row < rows)
+    {
+        float pos[3];
+        record_inputs(P, queries, sel.record(row), m, pos);
+        for (int i = 0; i < 3; i++)
+            E.pos[(size_t)i * E.stride + row] = pos[i];
+    }
+    for (int k = 0; k < NRC_MISC / 8; k++)
+        out[k] = make_uint4(m[4 * k], m[4 * k + 1], m[4 * k + 2], m[4 * k + 3]);
+}
+
+// Encodes the selected rows into E rows [0, rows) and zero-fills the rows up
+// to the next multiple of pad (at most n rows in all), in two kernels.
+//
+// k_nrc_inputs reads each record once: the inputs that are not grid features,
+// and the position in the grid's cube.
 __global__ __launch_bounds__(256) void k_nrc_inputs(NrcDev P, const float4* __restrict__ queries, RowSel sel,
                                                     uint32_t n, uint32_t pad, EncDev E)
 {
@@ -272,7 +274,45 @@ __global__ __launch_bounds__(256) void k_nrc_encode_few(NrcDev P, const float4* 
 }
 
 // Rows of NRC_WIDTH inputs as the network counts them: the grid features,
-// the other inputs, zeros (a thread per pair of inputs).
+// the other inputs, zeros. In one launch for few rows: `chunks` blocks for the
+// other inputs, then the levels' in k_nrc_grid's order.
+__global__ __launch_bounds__(256) void k_nrc_encode_rows(NrcDev P, const float4* __restrict__ queries, uint32_t n,
+                                                         uint32_t chunks, uint32_t* __restrict__ out)
+{
+    const uint32_t turn = blockIdx.x / NRC_XCDS;
+    int l = (int)(blockIdx.x % NRC_XCDS + NRC_XCDS * (turn / chunks));
+    uint32_t chunk = turn % chunks;
+    const uint32_t grid_blocks = (uint32_t)(P.levels + NRC_XCDS - 1) / NRC_XCDS * NRC_XCDS * chunks;
+    if (blockIdx.x >= grid_blocks)
+    {
+        l = P.levels;
+        chunk = blockIdx.x - grid_blocks;
+    }
+    else if (l >= P.levels)
+        return;
+    const uint32_t row = chunk * blockDim.x + threadIdx.x;
+    if (row >= n)
+        return;
+    uint32_t* o = out + (size_t)row * (NRC_WIDTH / 2);
+    if (l == P.levels)
+    {
+        uint32_t m[NRC_MISC / 2];
+        float pos[3];
+        record_inputs(P, queries, row, m, pos);
+        for (int k = 0; k < NRC_MISC / 2; k++)
+            o[l + k] = m[k];
+        for (int k = l + NRC_MISC / 2; k < NRC_WIDTH / 2; k++)
+            o[k] = 0u;
+        return;
+    }
+    const float4 a = queries[4 * (size_t)row];
+    const float q[3] = {a.x, a.y, a.z};
+    float pos[3];
+    normalized_position(P, q, pos);
+    o[l] = grid_features(P, l, pos);
+}
+
+// The same from encoded planes (a thread per pair of inputs).
 __global__ void k_nrc_rows(EncDev E, int levels, uint32_t n, uint32_t* __restrict__ out)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -308,6 +348,12 @@ EncDev enc_buffer(Nrc& C, uint32_t n)
 // (19.2), 60,000 61.5 us for 43.8, a million 478 us for 463. (The weights' loads
 // going out together then took 1 to 2 us off every one of these.)
 constexpr uint32_t FEW_ROWS = 16384;
+// The same line for rows as the caller gets them (one launch against the planes'
+// launches and k_nrc_rows; 16 levels of 2^19, 7 of 2^14): 1 to 5000 rows 6.2 us
+// for 9.5 and 9.9, 20,000 rows 15.8 us (8.8) for 19.0 (14.2), 40,000 28.7 us (13.9) for
+// 29.9 (17.3), 65,536 42.5 us (21.9) for 42.0 (22.4); there each row's 128 bytes
+// are written 4 at a time from eight XCDs.
+constexpr uint32_t FEW_OUTPUT_ROWS = 49152;
 
 void encode_launch(const NrcDev& P, const float* d_queries, const RowSel& sel, uint32_t n, uint32_t pad,
                    const EncDev& E, hipStream_t s)
@@ -1217,8 +1263,17 @@ void nrc_encode(Ctx& ctx, const float* d_queries, uint32_t n, uint16_t* d_out, h
         fail(MIPT_ERR_INVALID_ARGUMENT, "radiance cache not configured: call mipt_set_radiance_cache first");
     if (n == 0)
         return;
+    const NrcDev P = nrc_dev(ctx);
+    if (n <= FEW_OUTPUT_ROWS)
+    {
+        const unsigned chunks = (n + 255u) / 256u, turns = ((unsigned)P.levels + NRC_XCDS - 1) / NRC_XCDS;
+        hipLaunchKernelGGL(k_nrc_encode_rows, dim3((NRC_XCDS * turns + 1u) * chunks), dim3(256), 0, s, P,
+                           reinterpret_cast<const float4*>(d_queries), n, chunks, reinterpret_cast<uint32_t*>(d_out));
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
     const EncDev E = enc_buffer(C, n);
-    encode_launch(nrc_dev(ctx), d_queries, RowSel{nullptr, 1u, 0u, n}, n, 1u, E, s);
+    encode_launch(P, d_queries, RowSel{nullptr, 1u, 0u, n}, n, 1u, E, s);
     hipLaunchKernelGGL(k_nrc_rows, dim3(blocks_for((size_t)n * (NRC_WIDTH / 2), 256)), dim3(256), 0, s, E,
                        (int)C.settings.grid_levels, n, reinterpret_cast<uint32_t*>(d_out));
     HIP_CHECK(hipGetLastError());

@@ -146,3 +146,16 @@ def test_small_tables_are_binned(mipt_mod, torch_mod, scene1, log2_table):
     rows: 12.9 ms at 2^4 entries a level, 1.25 ms at 2^9)."""
     few, many = (_train_kernels(mipt_mod, torch_mod, scene1, 16, log2_table, n) for n in (4095, 4096))
     assert many == few + 4
+
+
+@pytest.mark.parametrize("rows,count", [(1, 1), (49152, 1), (49153, 3)])
+def test_encode_launches(mipt_mod, torch_mod, scene1, rows, count):
+    """Few rows are encoded to the caller's layout by one kernel (two took 9.9 us for 6.2)."""
+    ctx = mipt_mod.Context(0)
+    ctx.set_scene(scene1)
+    ctx.set_radiance_cache(mipt_mod.default_radiance_cache_settings(grid_levels=16, grid_log2_table=14))
+    q = torch_mod.rand(rows, 16, device="cuda")
+    out = torch_mod.empty(rows, 64, dtype=torch_mod.int16, device="cuda")
+    ctx.cache_encode(q, rows, out)
+    assert len(kernels(torch_mod, lambda s: ctx.cache_encode(q, rows, out, s))) == count
+    ctx.close()

@@ -4,6 +4,7 @@ working.
 - Inference: a row's answer does not depend on the rows beside it, so row
   counts around a wave's 64 rows and a block's 256 give the same bits as one
   large call.
+- Encoded rows: one launch up to 49,152 rows, planes and a copy past it; the same bits.
 - Grid and weight gradients: from 4096 rows on (16 levels; 15,360 with one) the corner
   updates are binned, below they are added by atomics. A batch's gradient is the row-weighted mean
   of its halves' (the terms are the same 32-bit products, up to the scale
@@ -36,6 +37,24 @@ def test_rows_are_independent(mipt_mod, torch_mod, scene1, levels):
     assert np.isfinite(want).all() and (want[:, 3] == 0.0).all()
     for n in (1, 2, 63, 64, 65, 255, 256, 257, 4097, 49153):
         assert _infer(mipt_mod, torch_mod, ctx, q[:n]).tobytes() == want[:n].tobytes(), n
+    ctx.close()
+
+
+@pytest.mark.parametrize("levels", [1, 7, 8, 9, 16])
+def test_encoded_rows_are_independent(mipt_mod, torch_mod, scene1, levels):
+    rng = np.random.default_rng(levels)
+    ctx, cs = _make(mipt_mod, scene1, grid_levels=levels, grid_log2_table=13)
+    _randomize_grid(ctx, cs, rng)
+    n = 49153
+    d_q = mipt_mod.to_device(_queries(rng, scene1, n))
+    want = torch_mod.empty(n, 64, dtype=torch_mod.int16, device="cuda")
+    ctx.cache_encode(d_q, n, want)
+    assert (want[:, 2 * levels + 28:] == 0).all()
+    for k in (1, 2, 255, 256, 257, 16385, 49152):
+        got = torch_mod.full((k + 1, 64), -1, dtype=torch_mod.int16, device="cuda")
+        ctx.cache_encode(d_q, k, got)
+        assert torch_mod.equal(got[:k], want[:k]), k
+        assert (got[k] == -1).all(), "written past the last row"
     ctx.close()
 
 
