@@ -967,7 +967,7 @@ void build_sah_binned(Ctx& ctx)
     bvh.triangle_count = n;
     if (n <= 0)
     {
-        bvh.node_count = bvh.leaf_count = bvh.max_depth = bvh.max_leaf_size = 0;
+        bvh.node_count = bvh.leaf_count = bvh.max_depth = bvh.max_leaf_size = bvh.wide_stack = 0;
         bvh.valid = true;
         return;
     }

@@ -966,9 +966,10 @@ uint32_t* trace_counters(Ctx& ctx)
     return trace_scratch(ctx, 0u).counter;
 }
 
+// A scene without triangles has work counters too (the passes reset them).
 void trace_reserve(Ctx& ctx)
 {
-    if (ctx.bvh.valid && ctx.bvh.triangle_count > 0)
+    if (ctx.bvh.valid)
         (void)trace_scratch(ctx, 0u);
 }
 

@@ -159,3 +159,52 @@ def test_encode_launches(mipt_mod, torch_mod, scene1, rows, count):
     ctx.cache_encode(q, rows, out)
     assert len(kernels(torch_mod, lambda s: ctx.cache_encode(q, rows, out, s))) == count
     ctx.close()
+
+
+def _empty_scene(mipt_mod):
+    return mipt_mod.Scene(np.zeros((0, 3), np.float32), np.zeros((0, 3), np.int32),
+                          camera=mipt_mod.generate_scene(1, 64, 48).camera)
+
+
+def _empty_ctx(mipt_mod, first=None, builder=1):
+    ctx = mipt_mod.Context(0)
+    if first is not None:
+        ctx.set_scene(first)
+        ctx.build_bvh(builder)
+    scene = _empty_scene(mipt_mod)
+    ctx.set_scene(scene)
+    ctx.build_bvh(builder)
+    ctx.set_envmap(mipt_mod.generate_envmap(64, 32))
+    ctx.set_world_settings(mipt_mod.default_world_settings(ambient_light_type=mipt_mod.MIPT_AMBIENT_ENVMAP))
+    ctx.set_render_settings(mipt_mod.default_render_settings(width=64, height=48, nb_bounces=3))
+    ctx.set_camera(scene.camera)
+    return ctx
+
+
+@pytest.mark.parametrize("builder", [0, 1])
+def test_empty_scene_holds_no_stacks(mipt_mod, torch_mod, scene2, builder):
+    """The traversal's buffers are those of the tree at hand: a scene without triangles after one of
+    1,040,384 takes no stacks (its first sample allocated those of the tree that was gone)."""
+    ctx = _empty_ctx(mipt_mod, scene2, builder)
+    torch_mod.cuda.synchronize()
+    before = torch_mod.cuda.mem_get_info()[0]
+    ctx.render_sample(0)
+    torch_mod.cuda.synchronize()
+    assert before - torch_mod.cuda.mem_get_info()[0] <= 32 << 20  # tables and a 64 x 32 envmap
+    ctx.close()
+
+
+def test_empty_scene_graph(mipt_mod, torch_mod):
+    """An environment alone, replayed: every sample equals the eager one, also where the first
+    sample is the one that is captured (its buffers are allocated before)."""
+    graph, eager = _empty_ctx(mipt_mod), _empty_ctx(mipt_mod)
+    graph.set_graph_capture(True)
+    for k in range(1, 5):
+        graph.render_sample(k)
+        eager.render_sample(k)
+        torch_mod.cuda.synchronize()
+        assert graph.graph_replays() == k
+        a, b = graph.read_framebuffer(), eager.read_framebuffer()
+        assert a.tobytes() == b.tobytes() and np.isfinite(a).all() and (a > 0).any()
+    graph.close()
+    eager.close()
