@@ -81,6 +81,10 @@ struct PassCounters {
     uint32_t* trace; // TRACE_COUNTERS, one per trace launch of a bounce
 };
 constexpr uint32_t RAY_LISTS = 3, SKIP_LISTS = 2, LIVE_LISTS = 2;
+// The skip lists are cleared once a bounce, so each is filled once in it: by
+// k_resolve and by every round but the last. A third round would append to the
+// list that the first one read.
+static_assert((uint32_t)MAX_SKIP_ROUNDS <= SKIP_LISTS, "a skip list for every round of a bounce");
 
 __device__ __forceinline__ void reset_lists(uint32_t* counts, uint32_t lists)
 {
