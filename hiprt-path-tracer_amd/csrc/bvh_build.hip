@@ -547,6 +547,7 @@ void build_lbvh(Ctx& ctx)
     hipLaunchKernelGGL(bvhc::k_emit_tris, dim3(blocks(n, B)), dim3(B), 0, s, verts, idx, n, vals_sorted,
                        bvh.tris.as<TriRecord>());
     HIP_CHECK(hipGetLastError());
+    finalize_bvh(ctx, nodes, ninner);
     HIP_CHECK(hipEventRecord(ev1, s));
     HIP_CHECK(hipEventSynchronize(ev1));
     float ms = 0.0f;
@@ -554,9 +555,6 @@ void build_lbvh(Ctx& ctx)
     bvh.build_ms = ms;
     HIP_CHECK(hipEventDestroy(ev0));
     HIP_CHECK(hipEventDestroy(ev1));
-    // Statistics, validation and the depth-first layout: not part of the
-    // build time.
-    finalize_bvh(ctx, nodes, ninner);
 }
 
 } // namespace mipt

@@ -1135,6 +1135,8 @@ void build_sah_binned(Ctx& ctx)
     hipLaunchKernelGGL(bvhc::k_emit_tris, dim3(bvhc::blocks(n, 256)), dim3(256), 0, s, verts, idx, n,
                        ref, bvh.tris.as<TriRecord>());
     HIP_CHECK(hipGetLastError());
+    // every split makes a node, and a whole subtree takes its count - 1 ids: n - 1 in all
+    finalize_bvh(ctx, nodes, ninner);
     HIP_CHECK(hipEventRecord(ev1, s));
     HIP_CHECK(hipEventSynchronize(ev1));
     float ms = 0.0f;
@@ -1142,8 +1144,6 @@ void build_sah_binned(Ctx& ctx)
     bvh.build_ms = ms;
     HIP_CHECK(hipEventDestroy(ev0));
     HIP_CHECK(hipEventDestroy(ev1));
-    // every split makes a node, and a whole subtree takes its count - 1 ids: n - 1 in all
-    finalize_bvh(ctx, nodes, ninner);
 }
 
 } // namespace mipt

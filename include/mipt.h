@@ -166,9 +166,11 @@ typedef struct mipt_bvh_info {
     int32_t leaf_count;
     int32_t max_depth;         /* deepest leaf, root = 0 */
     int32_t max_leaf_size;
-    int64_t node_bytes;
-    int64_t triangle_bytes;
-    double build_ms;           /* device time of the build kernels */
+    int64_t node_bytes;        /* of the binary tree's nodes that mipt_read_bvh copies ... */
+    int64_t triangle_bytes;    /* ... and of its triangle records; the tree of up to six children a
+                                * node that rays walk is made from them and held beside them */
+    double build_ms;           /* device time from the first kernel of the build to the tree that rays
+                                * walk, with the gaps between kernels */
     double sah_cost;           /* SAH cost (C_node = 1, C_tri = 1), relative to root area */
 } mipt_bvh_info;
 

@@ -208,3 +208,22 @@ def test_empty_scene_graph(mipt_mod, torch_mod):
         assert a.tobytes() == b.tobytes() and np.isfinite(a).all() and (a > 0).any()
     graph.close()
     eager.close()
+
+
+@pytest.mark.parametrize("builder", [0, 1])
+def test_build_time_is_whole(mipt_mod, torch_mod, scene1, builder):
+    """bvh_info's build_ms reaches to the tree that rays walk: it is most of a repeated build's wall
+    time (the rest: allocations before the first kernel; 0.57 of an LBVH build of 102,428
+    triangles was counted when it ended at the binary tree)."""
+    import time
+
+    ctx = mipt_mod.Context(0)
+    ctx.set_scene(scene1)
+    share = []
+    for _ in range(9):
+        t = time.perf_counter()
+        ctx.build_bvh(builder)
+        share.append(ctx.bvh_info().build_ms * 1e-3 / (time.perf_counter() - t))
+    ctx.close()
+    print(f"builder {builder}: {sorted(share)[4]:.2f} of the wall time")
+    assert 0.75 <= sorted(share)[4] <= 1.0
