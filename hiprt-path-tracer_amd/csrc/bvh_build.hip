@@ -49,13 +49,24 @@ __device__ __forceinline__ uint64_t expand21(uint64_t v)
     return v;
 }
 
+// Codes, and what the later kernels find set: no visits, no parents, nothing
+// collapsed (four memsets, seven kernels, otherwise).
 __global__ void k_morton(const float4* __restrict__ lo, const float4* __restrict__ hi, int32_t n,
                          const uint32_t* __restrict__ bounds, uint64_t* __restrict__ keys,
-                         uint32_t* __restrict__ vals)
+                         uint32_t* __restrict__ vals, int32_t ninner, uint32_t* __restrict__ visits,
+                         int32_t* __restrict__ node_parent, int32_t* __restrict__ leaf_parent,
+                         uint8_t* __restrict__ collapse)
 {
     int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
+    leaf_parent[i] = -1;
+    if (i < ninner)
+    {
+        visits[i] = 0u;
+        node_parent[i] = -1;
+        collapse[i] = 0;
+    }
     float clo[3], cext[3];
     for (int k = 0; k < 3; k++)
     {
@@ -261,12 +272,9 @@ void write_single_triangle_root(BvhNode* d_node, const float4* d_lo, const float
 namespace {
 
 constexpr int CHECK_BLOCK = 256;
-
-// What a block of nodes adds up to; a last record holds the root's area in sah.
-struct TreeStats {
-    double sah; // sum of C_node area over interior children and C_tri count area over leaves
-    uint32_t inner, leaves, max_depth, max_leaf, errors, pad;
-};
+constexpr int TREE_BLOCK = 1024;
+// Triangles up to which one block checks and lays out the tree, in LDS.
+constexpr int32_t TREE_SMALL = 4096;
 
 __device__ __forceinline__ double box_area(float lx, float ly, float lz, float hx, float hy, float hz)
 {
@@ -274,6 +282,107 @@ __device__ __forceinline__ double box_area(float lx, float ly, float lz, float h
     if (dx < 0 || dy < 0 || dz < 0)
         return 0.0;
     return dx * dy + dy * dz + dz * dx;
+}
+
+__device__ __forceinline__ double root_box_area(const BvhNode& nd, int32_t n)
+{
+    return n == 1 ? box_area(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y)
+                  : box_area(fminf(nd.a.x, nd.b.z), fminf(nd.a.y, nd.b.w), fminf(nd.a.z, nd.c.x),
+                             fmaxf(nd.a.w, nd.c.y), fmaxf(nd.b.x, nd.c.z), fmaxf(nd.b.y, nd.c.w));
+}
+
+// Checks node j and its children and adds them up. start(begin, depth)
+// records a node whose range starts at triangle `begin`; see_node(r) and see_tri(q)
+// mark a node as referenced and a triangle as held, and say whether they were.
+template <class Start, class SeeNode, class SeeTri>
+__device__ __forceinline__ void check_node(const BvhNode* __restrict__ nodes, int32_t j, int32_t count, int32_t n,
+                                           TreeStats& t, const Start& start, const SeeNode& see_node,
+                                           const SeeTri& see_tri)
+{
+    const BvhNode nd = nodes[j];
+    const int32_t begin = nd.d.z, depth = nd.d.w;
+    if (depth == NODE_UNUSED)
+        return;
+    t.inner++;
+    if (begin < 0 || begin >= n || depth < 0 || (depth == 0) != (j == 0))
+    {
+        t.errors++;
+        return;
+    }
+    start(begin, depth);
+    const double area[2] = {box_area(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y),
+                            box_area(nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w)};
+    const int32_t refs[2] = {nd.d.x, nd.d.y};
+    for (int s = 0; s < (n == 1 ? 1 : 2); s++)
+    {
+        const int32_t r = refs[s];
+        if (r >= 0)
+        {
+            t.sah += SAH_C_NODE * area[s];
+            if (r >= count || nodes[r].d.w != depth + 1 || (s == 0 && nodes[r].d.z != begin) || see_node(r))
+                t.errors++;
+            continue;
+        }
+        const int32_t first = leaf_first(r), cnt = leaf_count(r);
+        t.leaves++;
+        t.max_leaf = max(t.max_leaf, (uint32_t)cnt);
+        t.max_depth = max(t.max_depth, (uint32_t)depth + 1u);
+        t.sah += SAH_C_TRI * cnt * area[s];
+        if (first < 0 || first + cnt > n || (s == 0 && first != begin))
+        {
+            t.errors++;
+            continue;
+        }
+        for (int32_t q = first; q < first + cnt; q++)
+            t.errors += see_tri(q) ? 1u : 0u;
+    }
+}
+
+// Sums over the block, in thread 0; `part` holds a record per wave.
+template <int BLOCK> __device__ __forceinline__ TreeStats block_sum(TreeStats t, TreeStats* part)
+{
+    for (int off = 32; off > 0; off >>= 1)
+    {
+        t.sah += __shfl_xor(t.sah, off, 64);
+        t.inner += __shfl_xor(t.inner, off, 64);
+        t.leaves += __shfl_xor(t.leaves, off, 64);
+        t.errors += __shfl_xor(t.errors, off, 64);
+        t.max_depth = max(t.max_depth, (uint32_t)__shfl_xor(t.max_depth, off, 64));
+        t.max_leaf = max(t.max_leaf, (uint32_t)__shfl_xor(t.max_leaf, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0)
+        part[threadIdx.x / 64] = t;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < BLOCK / 64; w++)
+        {
+            t.sah += part[w].sah;
+            t.inner += part[w].inner;
+            t.leaves += part[w].leaves;
+            t.errors += part[w].errors;
+            t.max_depth = max(t.max_depth, part[w].max_depth);
+            t.max_leaf = max(t.max_leaf, part[w].max_leaf);
+        }
+    return t;
+}
+
+// Nodes whose range starts at the same triangle are a chain of first children,
+// so a node's place in the depth-first order is the number of nodes that start
+// before it, plus its depth below the chain's top.
+__device__ __forceinline__ void lay_out(const BvhNode* __restrict__ nodes, int32_t j, int32_t n,
+                                        const uint32_t* before, const int32_t* top_depth, BvhNode* __restrict__ out)
+{
+    BvhNode nd = nodes[j];
+    if (nd.d.w == NODE_UNUSED)
+        return;
+    auto place = [&](const int4 d) { return (int32_t)before[d.z] + d.w - top_depth[d.z]; };
+    const int32_t at = place(nd.d);
+    if (nd.d.x >= 0)
+        nd.d.x = place(nodes[nd.d.x].d);
+    if (nd.d.y >= 0 && n > 1)
+        nd.d.y = place(nodes[nd.d.y].d);
+    nd.d.z = nd.d.w = 0;
+    out[at] = nd;
 }
 
 __global__ void k_check_init(uint32_t* __restrict__ tri_seen, uint32_t* __restrict__ starts,
@@ -290,11 +399,9 @@ __global__ void k_check_init(uint32_t* __restrict__ tri_seen, uint32_t* __restri
         node_seen[i] = 0u;
 }
 
-// Checks every node and its children, adds up the statistics per block, and
-// counts the nodes whose range starts at each triangle, with the depth of
-// the topmost: those nodes are a chain of first children, so a node's place
-// in the depth-first order is the number of nodes that start before it, plus its
-// depth below the chain's top.
+// Checks every node, adds up the statistics per block, and counts the nodes whose
+// range starts at each triangle, with the depth of the topmost. A last record holds
+// the root's area in sah.
 __global__ __launch_bounds__(CHECK_BLOCK) void k_tree_check(const BvhNode* __restrict__ nodes, int32_t count, int32_t n,
                                                             uint32_t* __restrict__ tri_seen,
                                                             uint32_t* __restrict__ node_seen,
@@ -305,76 +412,20 @@ __global__ __launch_bounds__(CHECK_BLOCK) void k_tree_check(const BvhNode* __res
     __shared__ TreeStats part[CHECK_BLOCK / 64];
     const int32_t j = blockIdx.x * CHECK_BLOCK + threadIdx.x;
     TreeStats t{};
-    if (j < count && nodes[j].d.w != NODE_UNUSED)
-    {
-        const BvhNode nd = nodes[j];
-        const int32_t begin = nd.d.z, depth = nd.d.w;
-        t.inner = 1u;
-        if (j == 0)
-            stats[gridDim.x].sah =
-                n == 1 ? box_area(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y)
-                       : box_area(fminf(nd.a.x, nd.b.z), fminf(nd.a.y, nd.b.w), fminf(nd.a.z, nd.c.x),
-                                  fmaxf(nd.a.w, nd.c.y), fmaxf(nd.b.x, nd.c.z), fmaxf(nd.b.y, nd.c.w));
-        if (begin < 0 || begin >= n || depth < 0 || (depth == 0) != (j == 0))
-            t.errors = 1u;
-        else
-        {
-            atomicAdd(&starts[begin], 1u);
-            atomicMin(&top_depth[begin], depth);
-            const double area[2] = {box_area(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y),
-                                    box_area(nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w)};
-            const int32_t refs[2] = {nd.d.x, nd.d.y};
-            for (int s = 0; s < (n == 1 ? 1 : 2); s++)
-            {
-                const int32_t r = refs[s];
-                if (r >= 0)
-                {
-                    t.sah += SAH_C_NODE * area[s];
-                    if (r >= count || nodes[r].d.w != depth + 1 || (s == 0 && nodes[r].d.z != begin) ||
-                        atomicAdd(&node_seen[r], 1u) != 0u)
-                        t.errors++;
-                    continue;
-                }
-                const int32_t first = leaf_first(r), cnt = leaf_count(r);
-                t.leaves++;
-                t.max_leaf = max(t.max_leaf, (uint32_t)cnt);
-                t.max_depth = max(t.max_depth, (uint32_t)depth + 1u);
-                t.sah += SAH_C_TRI * cnt * area[s];
-                if (first < 0 || first + cnt > n || (s == 0 && first != begin))
-                {
-                    t.errors++;
-                    continue;
-                }
-                for (int32_t q = first; q < first + cnt; q++)
-                    t.errors += atomicAdd(&tri_seen[q], 1u) != 0u;
-            }
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1)
-    {
-        t.sah += __shfl_xor(t.sah, off, 64);
-        t.inner += __shfl_xor(t.inner, off, 64);
-        t.leaves += __shfl_xor(t.leaves, off, 64);
-        t.errors += __shfl_xor(t.errors, off, 64);
-        t.max_depth = max(t.max_depth, (uint32_t)__shfl_xor(t.max_depth, off, 64));
-        t.max_leaf = max(t.max_leaf, (uint32_t)__shfl_xor(t.max_leaf, off, 64));
-    }
-    if ((threadIdx.x & 63) == 0)
-        part[threadIdx.x / 64] = t;
-    __syncthreads();
+    if (j == 0)
+        stats[gridDim.x].sah = root_box_area(nodes[0], n);
+    if (j < count)
+        check_node(
+            nodes, j, count, n, t,
+            [&](int32_t begin, int32_t depth) {
+                atomicAdd(&starts[begin], 1u);
+                atomicMin(&top_depth[begin], depth);
+            },
+            [&](int32_t r) { return atomicAdd(&node_seen[r], 1u) != 0u; },
+            [&](int32_t q) { return atomicAdd(&tri_seen[q], 1u) != 0u; });
+    t = block_sum<CHECK_BLOCK>(t, part);
     if (threadIdx.x == 0)
-    {
-        for (int w = 1; w < CHECK_BLOCK / 64; w++)
-        {
-            t.sah += part[w].sah;
-            t.inner += part[w].inner;
-            t.leaves += part[w].leaves;
-            t.errors += part[w].errors;
-            t.max_depth = max(t.max_depth, part[w].max_depth);
-            t.max_leaf = max(t.max_leaf, part[w].max_leaf);
-        }
         stats[blockIdx.x] = t;
-    }
 }
 
 // Every used node but the root is referenced (once: k_tree_check), every
@@ -396,77 +447,186 @@ __global__ void k_tree_layout(const BvhNode* __restrict__ nodes, int32_t count, 
                               BvhNode* __restrict__ out)
 {
     const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= count || nodes[j].d.w == NODE_UNUSED)
+    if (j < count)
+        lay_out(nodes, j, n, before, top_depth, out);
+}
+
+// The same for a tree of at most TREE_SMALL triangles in one block, without the
+// host between check and layout: a tree with errors is not laid out.
+__global__ __launch_bounds__(TREE_BLOCK) void k_tree_small(const BvhNode* __restrict__ nodes, int32_t count, int32_t n,
+                                                           BvhNode* __restrict__ out, TreeReport* __restrict__ report)
+{
+    __shared__ uint32_t starts[TREE_SMALL]; // nodes that start at a triangle, then before it
+    __shared__ int32_t top_depth[TREE_SMALL];
+    __shared__ uint32_t tri_seen[TREE_SMALL / 32], node_seen[TREE_SMALL / 32];
+    __shared__ TreeStats part[TREE_BLOCK / 64];
+    __shared__ uint32_t wave_total[TREE_BLOCK / 64];
+    __shared__ uint32_t missing, errors;
+    const int32_t tid = (int32_t)threadIdx.x;
+    for (int32_t i = tid; i < TREE_SMALL; i += TREE_BLOCK)
+    {
+        starts[i] = 0u;
+        top_depth[i] = 0x7fffffff;
+    }
+    if (tid < TREE_SMALL / 32)
+        tri_seen[tid] = node_seen[tid] = 0u;
+    if (tid == 0)
+        missing = 0u;
+    __syncthreads();
+    TreeStats t{};
+    auto see = [](uint32_t* bits, int32_t i) {
+        const uint32_t bit = 1u << (i & 31);
+        return (atomicOr(&bits[i >> 5], bit) & bit) != 0u;
+    };
+    for (int32_t j = tid; j < count; j += TREE_BLOCK)
+        check_node(
+            nodes, j, count, n, t,
+            [&](int32_t begin, int32_t depth) {
+                atomicAdd(&starts[begin], 1u);
+                atomicMin(&top_depth[begin], depth);
+            },
+            [&](int32_t r) { return see(node_seen, r); }, [&](int32_t q) { return see(tri_seen, q); });
+    __syncthreads();
+    for (int32_t i = tid; i < n; i += TREE_BLOCK)
+    {
+        bool bad = ((tri_seen[i >> 5] >> (i & 31)) & 1u) == 0u;
+        if (i < count && i > 0 && nodes[i].d.w != NODE_UNUSED)
+            bad |= ((node_seen[i >> 5] >> (i & 31)) & 1u) == 0u;
+        if (bad)
+            atomicAdd(&missing, 1u);
+    }
+    // exclusive scan of starts: four a thread
+    static_assert(TREE_SMALL == 4 * TREE_BLOCK, "four a thread");
+    uint32_t own[4], sum = 0u;
+    for (int k = 0; k < 4; k++)
+    {
+        own[k] = starts[4 * tid + k];
+        sum += own[k];
+    }
+    uint32_t incl = sum;
+    for (int off = 1; off < 64; off <<= 1)
+    {
+        const uint32_t v = __shfl_up(incl, off, 64);
+        if ((tid & 63) >= off)
+            incl += v;
+    }
+    if ((tid & 63) == 63)
+        wave_total[tid / 64] = incl;
+    __syncthreads();
+    uint32_t at = incl - sum;
+    for (int w = 0; w < tid / 64; w++)
+        at += wave_total[w];
+    for (int k = 0; k < 4; k++)
+    {
+        starts[4 * tid + k] = at;
+        at += own[k];
+    }
+    t = block_sum<TREE_BLOCK>(t, part);
+    if (tid == 0)
+    {
+        t.errors += missing;
+        errors = t.errors;
+        report->sums = t;
+        report->root_area = root_box_area(nodes[0], n);
+    }
+    __syncthreads();
+    if (errors != 0u)
         return;
-    auto place = [&](const int4 d) { return (int32_t)before[d.z] + d.w - top_depth[d.z]; };
-    BvhNode nd = nodes[j];
-    const int32_t at = place(nd.d);
-    if (nd.d.x >= 0)
-        nd.d.x = place(nodes[nd.d.x].d);
-    if (nd.d.y >= 0 && n > 1)
-        nd.d.y = place(nodes[nd.d.y].d);
-    nd.d.z = nd.d.w = 0;
-    out[at] = nd;
+    for (int32_t j = tid; j < count; j += TREE_BLOCK)
+        lay_out(nodes, j, n, starts, top_depth, out);
 }
 
 } // namespace
 
-void finalize_bvh(Ctx& ctx, const BvhNode* d_nodes, int32_t count)
+TreeScratch tree_scratch(BuildScratch& sc, int32_t n, int32_t count)
+{
+    TreeScratch t{};
+    const size_t N = (size_t)n, C = (size_t)count;
+    if (n > TREE_SMALL)
+    {
+        t.o_tri = sc.add(4 * N);
+        t.o_starts = sc.add(4 * N);
+        t.o_before = sc.add(4 * N);
+        t.o_top = sc.add(4 * N);
+        t.o_node = sc.add(4 * C);
+        t.o_stats = sc.add(sizeof(TreeStats) * (blocks(count, CHECK_BLOCK) + 1));
+        HIP_CHECK(rocprim::exclusive_scan(nullptr, t.scan_bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr, 0u, N,
+                                          rocprim::plus<uint32_t>(), (hipStream_t) nullptr));
+        t.o_scan = sc.add(t.scan_bytes > 0 ? t.scan_bytes : 1);
+    }
+    t.o_item_ref = sc.add(sizeof(int32_t) * C);
+    t.o_item_stack = sc.add(sizeof(uint32_t) * C);
+    t.o_tri_src = sc.add(sizeof(uint32_t) * N);
+    t.o_report = sc.add(sizeof(TreeReport));
+    return t;
+}
+
+void set_statistics(Ctx& ctx, const TreeStats& t, double root_area)
+{
+    Bvh& bvh = ctx.bvh;
+    if (t.errors != 0u)
+        fail(MIPT_ERR_HIP, "BVH validation failed: " + std::to_string(t.errors) +
+                               " nodes or triangles missing, out of range or in two places");
+    bvh.node_count = (int32_t)t.inner;
+    bvh.leaf_count = (int32_t)t.leaves;
+    bvh.max_depth = (int32_t)t.max_depth;
+    bvh.max_leaf_size = (int32_t)t.max_leaf;
+    bvh.sah_cost = root_area > 0 ? (t.sah + SAH_C_NODE * root_area) / root_area : 0.0;
+}
+
+void finalize_bvh(Ctx& ctx, const BuildScratch& sc, TreeScratch& t, const BvhNode* d_nodes, int32_t count)
 {
     Bvh& bvh = ctx.bvh;
     const int32_t n = bvh.triangle_count;
     const hipStream_t s = nullptr;
-    bvh.root = 0;
+    t.item_ref = sc.get<int32_t>(t.o_item_ref);
+    t.item_stack = sc.get<uint32_t>(t.o_item_stack);
+    t.tri_src = sc.get<uint32_t>(t.o_tri_src);
+    t.report = sc.get<TreeReport>(t.o_report);
+    if (n <= TREE_SMALL)
+    {
+        bvh.nodes.reserve(sizeof(BvhNode) * (size_t)count);
+        hipLaunchKernelGGL(k_tree_small, dim3(1), dim3(TREE_BLOCK), 0, s, d_nodes, count, n, bvh.nodes.as<BvhNode>(),
+                           t.report);
+        build_wide(ctx, count, false, t);
+        bvh.valid = true;
+        return;
+    }
     const unsigned check_blocks = blocks(count, CHECK_BLOCK);
-    BuildScratch sc;
-    const size_t o_tri = sc.add(4 * (size_t)n), o_starts = sc.add(4 * (size_t)n), o_before = sc.add(4 * (size_t)n),
-                 o_top = sc.add(4 * (size_t)n), o_node = sc.add(4 * (size_t)count),
-                 o_stats = sc.add(sizeof(TreeStats) * (check_blocks + 1));
-    size_t scan_bytes = 0;
-    HIP_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr, 0u, (size_t)n,
-                                      rocprim::plus<uint32_t>(), s));
-    const size_t o_scan = sc.add(scan_bytes > 0 ? scan_bytes : 1);
-    sc.allocate();
-    uint32_t *tri_seen = sc.get<uint32_t>(o_tri), *starts = sc.get<uint32_t>(o_starts),
-             *before = sc.get<uint32_t>(o_before), *node_seen = sc.get<uint32_t>(o_node);
-    int32_t* top_depth = sc.get<int32_t>(o_top);
-    TreeStats* stats = sc.get<TreeStats>(o_stats);
+    uint32_t *tri_seen = sc.get<uint32_t>(t.o_tri), *starts = sc.get<uint32_t>(t.o_starts),
+             *before = sc.get<uint32_t>(t.o_before), *node_seen = sc.get<uint32_t>(t.o_node);
+    int32_t* top_depth = sc.get<int32_t>(t.o_top);
+    TreeStats* stats = sc.get<TreeStats>(t.o_stats);
     const unsigned wide_grid = blocks(std::max(n, count), 256);
     hipLaunchKernelGGL(k_check_init, dim3(wide_grid), dim3(256), 0, s, tri_seen, starts, top_depth, n, node_seen, count);
     hipLaunchKernelGGL(k_tree_check, dim3(check_blocks), dim3(CHECK_BLOCK), 0, s, d_nodes, count, n, tri_seen,
                        node_seen, starts, top_depth, stats);
     hipLaunchKernelGGL(k_tree_complete, dim3(wide_grid), dim3(256), 0, s, d_nodes, count, n, tri_seen, node_seen,
                        stats);
-    HIP_CHECK(rocprim::exclusive_scan(sc.get<void>(o_scan), scan_bytes, (const uint32_t*)starts, before, 0u, (size_t)n,
-                                      rocprim::plus<uint32_t>(), s));
+    size_t scan_bytes = t.scan_bytes;
+    HIP_CHECK(rocprim::exclusive_scan(sc.get<void>(t.o_scan), scan_bytes, (const uint32_t*)starts, before, 0u,
+                                      (size_t)n, rocprim::plus<uint32_t>(), s));
     HIP_CHECK(hipGetLastError());
     std::vector<TreeStats> hs(check_blocks + 1);
     HIP_CHECK(hipMemcpy(hs.data(), stats, sizeof(TreeStats) * hs.size(), hipMemcpyDeviceToHost));
     const double root_area = hs.back().sah;
     hs.pop_back();
-    TreeStats t{};
+    TreeStats sum{};
     for (const TreeStats& b : hs)
     {
-        t.sah += b.sah;
-        t.inner += b.inner;
-        t.leaves += b.leaves;
-        t.errors += b.errors;
-        t.max_depth = std::max(t.max_depth, b.max_depth);
-        t.max_leaf = std::max(t.max_leaf, b.max_leaf);
+        sum.sah += b.sah;
+        sum.inner += b.inner;
+        sum.leaves += b.leaves;
+        sum.errors += b.errors;
+        sum.max_depth = std::max(sum.max_depth, b.max_depth);
+        sum.max_leaf = std::max(sum.max_leaf, b.max_leaf);
     }
-    if (t.errors != 0u)
-        fail(MIPT_ERR_HIP, "BVH validation failed: " + std::to_string(t.errors) +
-                               " nodes or triangles missing, out of range or in two places");
-    bvh.nodes.reserve(sizeof(BvhNode) * (size_t)t.inner);
+    set_statistics(ctx, sum, root_area);
+    bvh.nodes.reserve(sizeof(BvhNode) * (size_t)bvh.node_count);
     hipLaunchKernelGGL(k_tree_layout, dim3(blocks(count, 256)), dim3(256), 0, s, d_nodes, count, n, before, top_depth,
                        bvh.nodes.as<BvhNode>());
     HIP_CHECK(hipGetLastError());
-    bvh.node_count = (int32_t)t.inner;
-    bvh.leaf_count = (int32_t)t.leaves;
-    bvh.max_depth = (int32_t)t.max_depth;
-    bvh.max_leaf_size = (int32_t)t.max_leaf;
-    bvh.sah_cost = root_area > 0 ? (t.sah + SAH_C_NODE * root_area) / root_area : 0.0;
-    build_wide(ctx);
+    build_wide(ctx, bvh.node_count, true, t);
     bvh.valid = true;
 }
 
@@ -505,6 +665,7 @@ void build_lbvh(Ctx& ctx)
                  o_leaf_parent = sc.add(4 * N), o_range_lo = sc.add(4 * I), o_range_hi = sc.add(4 * I),
                  o_visits = sc.add(4 * I), o_nlo = sc.add(sizeof(float4) * I), o_nhi = sc.add(sizeof(float4) * I),
                  o_cost = sc.add(4 * I), o_collapse = sc.add(I), o_nodes = sc.add(sizeof(BvhNode) * I);
+    TreeScratch tree = tree_scratch(sc, n, ninner);
     sc.allocate();
     float4 *plo = sc.get<float4>(o_plo), *phi = sc.get<float4>(o_phi), *nlo = sc.get<float4>(o_nlo),
            *nhi = sc.get<float4>(o_nhi);
@@ -524,14 +685,11 @@ void build_lbvh(Ctx& ctx)
     hipLaunchKernelGGL(bvhc::k_tri_boxes, dim3(bgrid), dim3(bvhc::BOUNDS_BLOCK), 0, s, verts, idx, n, plo, phi,
                        partial);
     hipLaunchKernelGGL(bvhc::k_bounds_final, dim3(1), dim3(bvhc::BOUNDS_FINAL_BLOCK), 0, s, partial, (int32_t)bgrid, bounds, pad);
-    hipLaunchKernelGGL(k_morton, dim3(blocks(n, B)), dim3(B), 0, s, plo, phi, n, bounds, keys, vals);
+    hipLaunchKernelGGL(k_morton, dim3(blocks(n, B)), dim3(B), 0, s, plo, phi, n, bounds, keys, vals,
+                       ninner, visits, node_parent, leaf_parent, collapse);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(rocprim::radix_sort_pairs(sc.get<void>(o_sort), tmp_bytes, keys, keys_sorted, vals, vals_sorted, (size_t)n,
                                         0u, 63u, s));
-    HIP_CHECK(hipMemsetAsync(visits, 0, sizeof(uint32_t) * ninner, s));
-    HIP_CHECK(hipMemsetAsync(node_parent, 0xff, sizeof(int32_t) * ninner, s));
-    HIP_CHECK(hipMemsetAsync(leaf_parent, 0xff, sizeof(int32_t) * n, s));
-    HIP_CHECK(hipMemsetAsync(collapse, 0, sizeof(uint8_t) * ninner, s));
 
     if (n == 1)
         write_single_triangle_root(nodes, plo, phi);
@@ -547,8 +705,8 @@ void build_lbvh(Ctx& ctx)
     hipLaunchKernelGGL(bvhc::k_emit_tris, dim3(blocks(n, B)), dim3(B), 0, s, verts, idx, n, vals_sorted,
                        bvh.tris.as<TriRecord>());
     HIP_CHECK(hipGetLastError());
-    finalize_bvh(ctx, nodes, ninner);
-    HIP_CHECK(hipEventRecord(ev1, s));
+    tree.done = ev1;
+    finalize_bvh(ctx, sc, tree, nodes, ninner);
     HIP_CHECK(hipEventSynchronize(ev1));
     float ms = 0.0f;
     HIP_CHECK(hipEventElapsedTime(&ms, ev0, ev1));

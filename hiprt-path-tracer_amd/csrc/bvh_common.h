@@ -208,12 +208,58 @@ struct BuildScratch {
 // them.
 constexpr int32_t NODE_UNUSED = -1;
 
+// What nodes add up to.
+struct TreeStats {
+    double sah; // sum of C_node area over interior children and C_tri count area over leaves
+    uint32_t inner, leaves, max_depth, max_leaf, errors, pad;
+};
+
+// Levels of the wide tree past those that one block makes. A binary tree is at
+// most 96 levels deep (LBVH), and a wide level takes one of them at least.
+constexpr int WIDE_LEVELS = 128;
+
+struct WideCounters {
+    uint32_t tris, max_stack;
+    struct {
+        uint32_t begin, count;
+    } level[WIDE_LEVELS + 1]; // [0]: the first that k_wide_small left to do
+};
+
+// What the host reads of a finished tree.
+struct TreeReport {
+    TreeStats sums;
+    double root_area;
+    WideCounters wide;
+};
+
+// Temporaries of finalize_bvh, in the builder's scratch.
+struct TreeScratch {
+    size_t o_tri, o_starts, o_before, o_top, o_node, o_stats, o_scan, scan_bytes; // trees of more than one block
+    size_t o_item_ref, o_item_stack, o_tri_src, o_report;
+    int32_t* item_ref;
+    uint32_t* item_stack;
+    uint32_t* tri_src;
+    TreeReport* report;
+    hipEvent_t done; // recorded after the last kernel
+};
+
+// Adds the temporaries for a tree of n triangles and `count` nodes. Defined in bvh_build.hip.
+TreeScratch tree_scratch(BuildScratch& sc, int32_t n, int32_t count);
+
 // After a builder wrote `count` such nodes (root = node 0) and the
 // TriRecords: validates the tree (each interior node referenced once, by a
 // parent one level up, each triangle in exactly one leaf), computes its
 // statistics and SAH cost, and lays it out depth first into ctx.bvh.nodes, then
 // makes the wide tree. Defined in bvh_build.hip.
-void finalize_bvh(Ctx& ctx, const BvhNode* d_nodes, int32_t count);
+void finalize_bvh(Ctx& ctx, const BuildScratch& sc, TreeScratch& t, const BvhNode* d_nodes, int32_t count);
+
+// Statistics of the binary tree into ctx.bvh; fails if it is not valid.
+// Defined in bvh_build.hip.
+void set_statistics(Ctx& ctx, const TreeStats& t, double root_area);
+
+// The 6-wide tree from the binary one in ctx.bvh. Without `checked` the
+// binary tree's statistics are still on the device, in the report. Defined in bvh_wide.hip.
+void build_wide(Ctx& ctx, int32_t capacity, bool checked, const TreeScratch& t);
 
 // The one-triangle tree: a root whose first child is the leaf and whose
 // second child has an empty box. Defined in bvh_build.hip.

@@ -998,6 +998,7 @@ void build_sah_binned(Ctx& ctx)
                  // tasks, [3] whole subtrees, [8 + i] node of large task i
                  o_counters = sc.add(4 * (8 + max_large)), o_chunk = sc.add(sizeof(Chunk) * max_chunks),
                  o_chunk_left = sc.add(4 * max_chunks), o_nodes = sc.add(sizeof(BvhNode) * (size_t)ninner);
+    TreeScratch tree = tree_scratch(sc, n, ninner);
     sc.allocate();
     float4 *lo = sc.get<float4>(o_lo), *hi = sc.get<float4>(o_hi), *plo = sc.get<float4>(o_plo),
            *phi = sc.get<float4>(o_phi);
@@ -1136,8 +1137,8 @@ void build_sah_binned(Ctx& ctx)
                        ref, bvh.tris.as<TriRecord>());
     HIP_CHECK(hipGetLastError());
     // every split makes a node, and a whole subtree takes its count - 1 ids: n - 1 in all
-    finalize_bvh(ctx, nodes, ninner);
-    HIP_CHECK(hipEventRecord(ev1, s));
+    tree.done = ev1;
+    finalize_bvh(ctx, sc, tree, nodes, ninner);
     HIP_CHECK(hipEventSynchronize(ev1));
     float ms = 0.0f;
     HIP_CHECK(hipEventElapsedTime(&ms, ev0, ev1));

@@ -95,9 +95,8 @@ struct Bvh {
     DeviceBuffer nodes;           // BvhNode[node_count]
     DeviceBuffer tris;            // TriRecord[triangle_count] in leaf order
     // the 6-wide tree the traversal walks, made from the binary one
-    int32_t wide_count = 0;       // nodes, root = node 0
     int32_t wide_stack = 0;       // entries a traversal's stack can hold at most
-    DeviceBuffer wide;            // WideNode[wide_count]
+    DeviceBuffer wide;            // WideNode, root = node 0
     DeviceBuffer wide_tris;       // TriRecord[triangle_count] in the wide leaves' order
 };
 
@@ -290,9 +289,6 @@ void restir_spatiotemporal_pass(Ctx& ctx, uint32_t sample_number, uint32_t rando
 // bvh_build.hip
 void build_lbvh(Ctx& ctx);
 void build_sah_binned(Ctx& ctx);
-
-// bvh_wide.hip: the 6-wide tree from the finished binary one.
-void build_wide(Ctx& ctx);
 
 // pathtrace.hip: fills tri_info and light_info from the scene's geometry.
 void build_light_records(Ctx& ctx);

@@ -41,6 +41,7 @@
 #include <utility>
 
 #include "internal.h"
+#include "lane_groups.h"
 #include "pt_math.h"
 #include "seglist.h"
 
@@ -139,37 +140,7 @@ __host__ __device__ __forceinline__ uint32_t wave_batch(uint32_t total, uint32_t
 // 41 us, 120,000 (which end one lane to a ray until eight are left in a wave)
 // 142 us and 116 us; 2,073,600 516 us and 506 us. Eight rays is what the lanes
 // hold; a wave with more has enough to issue.
-constexpr int GROUP = 8;
 constexpr int GROUPS = 64 / GROUP;
-
-// Value of the lane whose index in the group of eight is lane ^ X.
-template <int X> __device__ __forceinline__ uint32_t group_xor(uint32_t v)
-{
-    constexpr int QUAD = X & 4 ? 3 - (X & 3) : X; // half-row mirror is ^ 7
-    int r = (int)v;
-    if (X & 4)
-        r = __builtin_amdgcn_mov_dpp(r, 0x141, 0xf, 0xf, true); // row_half_mirror
-    if (QUAD == 1)
-        r = __builtin_amdgcn_mov_dpp(r, 0xb1, 0xf, 0xf, true); // quad_perm 1 0 3 2
-    else if (QUAD == 2)
-        r = __builtin_amdgcn_mov_dpp(r, 0x4e, 0xf, 0xf, true); // quad_perm 2 3 0 1
-    else if (QUAD == 3)
-        r = __builtin_amdgcn_mov_dpp(r, 0x1b, 0xf, 0xf, true); // quad_perm 3 2 1 0
-    return (uint32_t)r;
-}
-
-__device__ __forceinline__ uint32_t group_min(uint32_t v)
-{
-    v = min(v, group_xor<1>(v));
-    v = min(v, group_xor<2>(v));
-    return min(v, group_xor<7>(v));
-}
-
-// Lanes of the group (bit c for lane c) that vote yes.
-__device__ __forceinline__ uint32_t group_ballot(bool yes, uint32_t group_shift)
-{
-    return (uint32_t)(__ballot(yes) >> group_shift) & 0xffu;
-}
 
 template <int I> __device__ __forceinline__ float byte_of(uint32_t w) { return (float)((w >> (8 * I)) & 0xffu); }
 
