@@ -9,9 +9,11 @@
 //   * small tasks (<= SMALL_MAX primitives): one 256-thread block per task
 //     loads the range into registers, reduces its box and centroid bounds,
 //     bins the centroids into NB bins per axis in LDS, sweeps the 3 x (NB-1)
-//     split planes (one wave per axis, scans by lane shuffles), decides leaf
-//     or split by the SAH, partitions the range in place and appends the
-//     two children to the next round's list;
+//     split planes (one wave per axis, scans by lane shuffles), partitions the
+//     range in place and appends the two children to the next round's list;
+//   * whole subtrees (<= WAVE_MAX primitives): listed as the rounds meet them and
+//     built after the last round, one wave each, to their leaves (k_sah_wave);
+//     only here is a task weighed against a leaf;
 //   * large tasks: the same steps spread over chunks of SMALL_MAX primitives
 //     (one block per chunk; bins merged with global atomics, the partition
 //     through per-chunk offsets computed on the host, so the result does
@@ -290,7 +292,9 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wsum, 
     return base + inc - v;
 }
 
-// One round of every small task: one block each.
+// One round of every small task: one block each. A task of more than WAVE_MAX
+// triangles is never a leaf.
+static_assert(WAVE_MAX >= MAX_LEAF_SIZE, "leaves of several triangles are k_sah_wave's alone");
 __global__ __launch_bounds__(SB) void k_sah_small(const SahTask* __restrict__ tasks, uint32_t* __restrict__ ref,
                                                   const float4* __restrict__ blo, const float4* __restrict__ bhi,
                                                   BvhNode* __restrict__ nodes, uint32_t* __restrict__ counters,
@@ -325,7 +329,6 @@ __global__ __launch_bounds__(SB) void k_sah_small(const SahTask* __restrict__ ta
         }
     }
     block_bounds(v, red, tb);
-    const float4 tlo = make_float4(tb[0], tb[1], tb[2], 0.0f), thi = make_float4(tb[3], tb[4], tb[5], 0.0f);
     float cmin[3], scale[3];
     for (int a = 0; a < 3; a++)
     {
@@ -361,16 +364,6 @@ __global__ __launch_bounds__(SB) void k_sah_small(const SahTask* __restrict__ ta
         if (best[a].cost < best[axis].cost)
             axis = a;
     const AxisBest b = best[axis];
-    const float area = half_area(tlo, thi);
-    const float split_cost = bvhc::SAH_C_NODE + bvhc::SAH_C_TRI * b.cost / area;
-    const float leaf_cost = bvhc::SAH_C_TRI * (float)task.count;
-    const bool can_leaf = task.count <= MAX_LEAF_SIZE && task.slot >= 0;
-    if (can_leaf && (leaf_cost <= split_cost || task.depth >= DEPTH_LIMIT || !(b.cost < INFINITY)))
-    {
-        if (t == 0)
-            set_slot(nodes, task.slot, make_leaf(task.begin, task.count));
-        return;
-    }
     const bool median = !(b.cost < INFINITY) || task.depth >= DEPTH_LIMIT;
     int32_t nl;
     float4 llo, lhi, rlo, rhi;
