@@ -89,7 +89,6 @@ struct Bvh {
     int32_t leaf_count = 0;
     int32_t max_depth = 0;
     int32_t max_leaf_size = 0;
-    int32_t root = 0;             // node index of the root
     double build_ms = 0.0;
     double sah_cost = 0.0;
     DeviceBuffer nodes;           // BvhNode[node_count]

@@ -1551,11 +1551,6 @@ PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfC
     return compensated(final_color, t.coat_compensation);
 }
 
-PT_HD Color principled_eval(const BsdfGlobals& g, const Material& m, const BsdfCtx& c, float& pdf)
-{
-    return principled_eval(g, m, c, view_terms(g, m, c), pdf);
-}
-
 // Principled.h:1802-1939. Returns the BSDF value of the sampled direction;
 // pdf = 0 when the sample is invalid. `c.info` receives the sampled lobe
 // (the sheen lobe leaves it as it was). With c.update, a reflection pops the
@@ -1627,12 +1622,6 @@ PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& 
         return col(0.0f);
     c.to_light = out_dir;
     return principled_eval(g, m, c, t, pdf);
-}
-
-PT_HD Color principled_sample(const BsdfGlobals& g, const Material& m, BsdfCtx& c, f3& out_dir, float& pdf,
-                              Xorshift32& rng)
-{
-    return principled_sample(g, m, c, view_terms(g, m, c), out_dir, pdf, rng);
 }
 
 // ---------------------------------------------------------------------------
