@@ -4,10 +4,12 @@
 // MFMA units (FP32 accumulation), a relative-L2 loss and Adam, all trained on
 // the GPU from the tracer's own paths.
 //
-// MFMA: v_mfma_f32_16x16x32_bf16, one wave per 16-row tile. Operand layout
-// of lane l (0..63): A[m = l%16][k = 8*(l/16) + j], B[k = 8*(l/16) + j][n = l%16]
-// for j < 8; D[m = 4*(l/16) + i][n = l%16] for i < 4. Activations move between
-// layers through a padded LDS tile (D layout -> row-major -> A layout).
+// MFMA: v_mfma_f32_16x16x32_bf16. Operand layout of lane l (0..63):
+// A[m = l%16][k = 8*(l/16) + j], B[k = 8*(l/16) + j][n = l%16] for j < 8;
+// D[m = 4*(l/16) + i][n = l%16] for i < 4. Inference has a wave for 64 rows, whose
+// activations stay in registers (k_nrc_forward); training one for a 16-row tile,
+// whose activations move between layers through a padded LDS tile
+// (D layout -> row-major -> A layout).
 #include <hip/hip_runtime.h>
 
 #include <cstring>

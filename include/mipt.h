@@ -318,7 +318,7 @@ typedef struct mipt_trace_tuning {
     int32_t block_size, lds_stack, queue_tile;
     int32_t configurations; /* timed */
     double best_ms;         /* mean launch time of the chosen configuration */
-    double default_ms;      /* of 128 threads, 16 LDS entries, tile 1 */
+    double default_ms;      /* of 128 threads, 8 LDS entries, tile 1 */
 } mipt_trace_tuning;
 int mipt_autotune_trace(mipt_ctx* ctx, const mipt_ray* d_rays, uint32_t n, int32_t repeats, void* stream,
                         mipt_trace_tuning* out, double* table_ms);
