@@ -28,6 +28,7 @@ namespace {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4))); // in a caller's array of floats
 
 // Rows from which the grid gradient is binned instead of added by global
 // atomics: the bins' five launches cost the same with few levels as with many,
@@ -415,7 +416,7 @@ constexpr int FWD_FRAGS = (NRC_LAYERS - 1) * 8 + 2; // 64-lane weight fragments:
 // columns blocks) of a wave: through LDS tiles of 16 rows, with the fragments
 // read for each, 1,000,003 rows took 132 us.
 __global__ __launch_bounds__(256, 3) void k_nrc_forward(const uint16_t* __restrict__ wt_global, EncDev E, int levels,
-                                                     const uint32_t* count, uint32_t n, float4* __restrict__ out)
+                                                     const uint32_t* count, uint32_t n, v4f_any* __restrict__ out)
 {
     __shared__ uint4 frag[FWD_FRAGS * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(256, 3) void k_nrc_forward(const uint16_t* __restri
             acc = mfma(a0, operand(x[q][0]), acc);
             acc = mfma(a1, operand(x[q][1]), acc);
             if (g == 0 && r + q < rows)
-                out[r + q] = make_float4(acc[0], acc[1], acc[2], 0.0f);
+                out[r + q] = v4f_any{acc[0], acc[1], acc[2], 0.0f};
         }
     }
 }
@@ -1254,7 +1255,7 @@ void nrc_infer(Ctx& ctx, const float* d_queries, const uint32_t* d_count, uint32
     encode_launch(P, d_queries, RowSel{d_count, 1u, 0u, n}, n, 1u, E, s);
     const unsigned grid = (unsigned)std::min<size_t>(blocks_for((n + 63) / 64, 4), (size_t)ctx.cu_count * 3);
     hipLaunchKernelGGL(k_nrc_forward, dim3(grid), dim3(256), 0, s, C.wt.as<uint16_t>(), E, P.levels, d_count, n,
-                       reinterpret_cast<float4*>(d_out));
+                       reinterpret_cast<v4f_any*>(d_out));
     HIP_CHECK(hipGetLastError());
 }
 

@@ -40,6 +40,23 @@ def test_rows_are_independent(mipt_mod, torch_mod, scene1, levels):
     ctx.close()
 
 
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_output_rows_at_any_float(mipt_mod, torch_mod, scene1, offset):
+    """Rows of an array of floats that does not begin at a multiple of 16 bytes."""
+    rng = np.random.default_rng(offset)
+    ctx, cs = _make(mipt_mod, scene1, grid_levels=16, grid_log2_table=13)
+    _randomize_grid(ctx, cs, rng)
+    n = 1003
+    d_q = mipt_mod.to_device(_queries(rng, scene1, n))
+    want = torch_mod.empty(4 * n, device="cuda")
+    ctx.cache_infer(d_q, n, want)
+    buf = torch_mod.full((4 * n + 8,), -7.0, device="cuda")
+    ctx.cache_infer(d_q, n, buf[offset:])
+    assert torch_mod.equal(buf[offset:offset + 4 * n], want)
+    assert (buf[:offset] == -7.0).all() and (buf[offset + 4 * n:] == -7.0).all()
+    ctx.close()
+
+
 @pytest.mark.parametrize("levels", [1, 7, 8, 9, 16])
 def test_encoded_rows_are_independent(mipt_mod, torch_mod, scene1, levels):
     rng = np.random.default_rng(levels)
