@@ -4,7 +4,8 @@ through the C ABI: hit records bit-identical on two calls in a row, the
 second over fewer rays, on the 1,040,384-triangle scene's 1920x1080
 incoherent bounce rays; the same on a context whose first traversal is the
 no-allocation one; a BVH deep enough that the grid's spill columns exceed
-the scratch (LDS stack of 8 entries) still gives the same hits."""
+the scratch still gives the same hits (the call then keeps more of the stack in
+LDS, or runs on fewer blocks: test_gpu_launches.py)."""
 import numpy as np
 import pytest
 
@@ -56,7 +57,7 @@ def test_noalloc_equals_trace_closest(mipt_mod, torch_mod, scene2, builder):
         got = _hits(mipt_mod, torch_mod, ctx.trace_closest_noalloc, d_rays, count)
         assert _same(got, want), f"{count} rays: hit records differ"
         assert (got["prim"] >= 0).mean() > 0.3
-    # a deep-spill configuration: 8 LDS entries, the rest in the scratch
+    # from 8 LDS entries on, the call takes the depth that leaves the most blocks
     ctx.set_trace_config(128, 8)
     for count in (n, 1000):
         print(f"noalloc {builder}, LDS stack 8: {count} rays", flush=True)
