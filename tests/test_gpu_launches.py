@@ -226,4 +226,4 @@ def test_build_time_is_whole(mipt_mod, torch_mod, scene1, builder):
         share.append(ctx.bvh_info().build_ms * 1e-3 / (time.perf_counter() - t))
     ctx.close()
     print(f"builder {builder}: {sorted(share)[4]:.2f} of the wall time")
-    assert 0.75 <= sorted(share)[4] <= 1.0
+    assert 0.75 <= sorted(share)[4] <= 1.05
