@@ -185,13 +185,16 @@ def _empty_ctx(mipt_mod, first=None, builder=1):
 def test_empty_scene_holds_no_stacks(mipt_mod, torch_mod, scene2, builder):
     """The traversal's buffers are those of the tree at hand: a scene without triangles after one of
     1,040,384 takes no stacks (its first sample allocated those of the tree that was gone)."""
+    first = _empty_ctx(mipt_mod)
+    first.render_sample(0)  # what a process's first sample loads
     ctx = _empty_ctx(mipt_mod, scene2, builder)
     torch_mod.cuda.synchronize()
     before = torch_mod.cuda.mem_get_info()[0]
     ctx.render_sample(0)
     torch_mod.cuda.synchronize()
-    assert before - torch_mod.cuda.mem_get_info()[0] <= 32 << 20  # tables and a 64 x 32 envmap
+    assert before - torch_mod.cuda.mem_get_info()[0] <= 48 << 20  # tables and a 64 x 32 envmap; the stacks are 103 MB
     ctx.close()
+    first.close()
 
 
 def test_empty_scene_graph(mipt_mod, torch_mod):
